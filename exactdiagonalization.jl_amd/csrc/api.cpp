@@ -898,8 +898,13 @@ struct edhip_op {
   bool keeps_popcount = true;  // every off-diagonal term's image has its row's popcount
   // device terms
   DevBuf off_row, off_col, diag, all_row, all_col;
-  DevBuf mv_row, mv_col;  // paired copies of off_row / off_col for the matvec
-  int n_mv = 0;
+  // the products' entries, row form [0] and column form [1] (OpDev)
+  struct MvHost {
+    DevBuf ent, tab, rest;
+    std::vector<MvEntry> entries;
+    int n_lin = 0, n_rest = 0;
+  };
+  MvHost mv[2], mv_plain[2];  // mv_plain: off term by term, for operators without LDS room for the tables
   int n_off = 0, n_diag = 0;
   std::vector<int64_t> diag_ids, off_ids;  // original term index of each device term
   OpDev dev_row{}, dev_col{};
@@ -992,37 +997,45 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   }
   d.off = transpose ? op->off_col.as<OffTerm>() : op->off_row.as<OffTerm>();
   d.diag = op->diag.as<DiagTerm>();
-  // the matvec stages 36 bytes per padded term, the other kernels 40 per term
   const uint32_t w_bytes = d.ix.rank_mode ? (uint32_t)((sp->n_bits + 1) * (sp->n_bits + 1) * 8) : 0u;
   const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
-  const uint32_t paired_bytes = std::max(plain_bytes, align_up((uint32_t)(op->n_mv * 36), 16));
   const uint32_t group_bytes = align_up(d.lay.total, 16);
-  d.mv_off = transpose ? op->mv_col.as<OffTerm>() : op->mv_row.as<OffTerm>();
-  d.n_mv = op->n_mv;
-  if (group_bytes + paired_bytes + w_bytes > 64 * 1024 && group_bytes + plain_bytes + w_bytes <= 64 * 1024)
-    d.n_mv = 0;  // no room for the paired copy: match term by term
-  const uint32_t op_bytes = (d.n_mv ? paired_bytes : plain_bytes) + w_bytes;
-  if (d.g.pair_table && group_bytes + op_bytes > 64 * 1024) {
+  const int form = transpose ? 1 : 0;
+  d.n_chunk = mv_chunks(sp->n_bits);
+  const MvLayout full = mv_layout(op->mv[form].n_lin, d.n_chunk, op->mv[form].n_rest, 1);
+  const bool no_room = group_bytes + std::max(full.total, plain_bytes) + w_bytes > 64 * 1024 &&
+                       group_bytes + plain_bytes + w_bytes <= 64 * 1024;
+  const auto& mv = no_room ? op->mv_plain[form] : op->mv[form];
+  d.ent = mv.ent.as<MvEntry>();
+  d.lin_tab = mv.tab.as<uint64_t>();
+  d.rest = no_room ? d.off : mv.rest.as<OffTerm>();
+  d.n_lin = mv.n_lin;
+  d.n_rest = mv.n_rest;
+  d.rest_paired = no_room ? 0 : 1;
+  d.stripe = ~0ull;
+  const uint32_t mv_bytes = align_up(mv_layout(d.n_lin, d.n_chunk, d.n_rest, d.rest_paired).total, 16);
+  if (d.g.pair_table && group_bytes + std::max(plain_bytes, mv_bytes) + w_bytes > 64 * 1024) {
     // not enough LDS next to this operator's terms: use the per-row table path
     d.g.pair_table = 0;
     d.lay.bytes_pair = 0;
     d.lay.total = d.lay.off_pair;
   }
-  uint32_t off = align_up(d.lay.total, 16);
-  d.off_lds = off;
-  off += d.n_mv ? paired_bytes : plain_bytes;
-  off = align_up(off, 16);
-  d.w_lds = off;
-  d.w_bytes = d.ix.rank_mode ? (uint32_t)((sp->n_bits + 1) * (sp->n_bits + 1) * 8) : 0u;
-  off += d.w_bytes;
-  d.lds_total = align_up(off, 16);
-  // the matvec alone stages the code table of the spread x after the rest
+  // (room for the largest code table of the spread x and the colex rank table)
+  const uint32_t codes_bytes = (2u << kXTopBits) + 2u * 4096u;
+  d.off_lds = d.mv_lds = align_up(d.lay.total, 16);
+  d.w_bytes = w_bytes;
+  d.w_lds = d.off_lds + plain_bytes;
+  d.lds_total = align_up(d.w_lds + w_bytes, 16);
+  d.mv_w_lds = d.mv_lds + mv_bytes;
+  d.mv_lds_total = align_up(d.mv_w_lds + w_bytes, 16);
+  // the products and the term pass stage the code table of the spread x after the rest
   d.xm = XMapDev{};
-  // (room for the largest code table and the colex rank table)
-  d.codes_lds = d.lds_total + (2u << kXTopBits) + 2u * 4096u <= 64 * 1024 ? d.lds_total : 0;
-  if (d.lds_total > 64 * 1024)
+  d.codes_lds = d.lds_total + codes_bytes <= 64 * 1024 ? d.lds_total : 0;
+  d.mv_codes_lds = d.mv_lds_total + codes_bytes <= 64 * 1024 ? d.mv_lds_total : 0;
+  const uint32_t most = std::max(d.lds_total, d.mv_lds_total);
+  if (most > 64 * 1024)
     fail(EDHIP_ERR_ARGUMENT, "operator and symmetry tables exceed the 64 KiB LDS budget of the matvec kernels (" +
-                                 std::to_string(d.lds_total) + " bytes)");
+                                 std::to_string(most) + " bytes)");
   return d;
 }
 
@@ -1179,7 +1192,8 @@ bool ensure_diag(edhip_op* op) {
 // x / sqrt(N) on reduced spaces (the products then weigh an image without
 // its orbit size, and their canonicalisers skip counting the stabiliser).
 // Returns whether it did.
-bool attach_spread(edhip_op* op, int prec, OpDev& d, const void* x, hipStream_t st, bool scaled = false) {
+bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const void* x, hipStream_t st,
+                   bool scaled = false) {
   const edhip_space* sp = op->space;
   const bool rank_mode = sp->is_sector && !sp->group;
   const int idx_lookup = (op->strat_lookup == 2) ? 0 : op->strat_lookup;
@@ -1192,7 +1206,7 @@ bool attach_spread(edhip_op* op, int prec, OpDev& d, const void* x, hipStream_t 
   const bool dense = sp->ensure_xtop() <= ratio * (uint64_t)sp->dim && (uint64_t)sp->dim * es > kXMapCachedBytes;
   const bool want = idx_lookup == 4 ||
                     (idx_lookup == 0 && (rank_mode || sp->ensure_xtop() * es <= kXMapCachedBytes || dense));
-  if (!want || !d.codes_lds) return false;
+  if (!want || !codes_lds) return false;
   const edhip_space::XMapHost* X = sp->ensure_xmap(es);
   if (!X) return false;
   const uint16_t* orbit = (scaled && sp->group) ? sp->orbit.as<uint16_t>() : nullptr;
@@ -1245,14 +1259,12 @@ bool ensure_assembled(edhip_op* op, uint64_t max_bytes = ~0ull) {
   if (col_bits > 31) fail(EDHIP_ERR_ARGUMENT, "assembled rows hold at most 2^31 basis states");
   OpDev d = op->dev_row;
   d.ix = sp->index_dev(0);
-  const int nt = d.n_mv ? d.n_mv : d.n_off;
-  std::vector<OffTerm> terms((size_t)nt);
-  if (nt)
-    HIP_OR_THROW(hipMemcpy(terms.data(), d.n_mv ? d.mv_off : d.off, (size_t)nt * sizeof(OffTerm), hipMemcpyDeviceToHost));
+  const std::vector<MvEntry>& terms = (d.ent == op->mv[0].ent.as<MvEntry>() ? op->mv[0] : op->mv_plain[0]).entries;
+  const int nt = (int)terms.size();
   std::vector<std::complex<double>> amps, phs;
   std::vector<uint32_t> acls((size_t)std::max(nt, 1), 1u);
   for (int t = 0; t < nt; ++t) {
-    if (terms[(size_t)t].match == terms[(size_t)t].image) continue;  // padding: never matches
+    if (terms[(size_t)t].flip == 0) continue;  // padding: never matches
     const std::complex<double> a(terms[(size_t)t].are, terms[(size_t)t].aim);
     const size_t k = (size_t)(std::find(amps.begin(), amps.end(), a) - amps.begin());
     if (k == amps.size()) amps.push_back(a);
@@ -1356,6 +1368,21 @@ void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) 
   }
 }
 
+// log2 of the lanes that share a row in the term-list products: one lane per
+// row where the rows alone give the chip half of the 2^19 lanes it holds;
+// smaller spaces take more (at most 16, and at most one per 4 entries), whose
+// shorter chains of images end sooner: 4x6 J1-J2 (pi, 0), 112,792 rows and 96
+// entries, FP32: 109.4 us a call with 1 lane, 89.5 with 2, 83.5 with 4, 90.4
+// with 8; 5x6, 5.2M rows: 2072 us with 1, 2360 with 2.  The rule looks at the
+// whole space, not at the rows computed, so that a share of the rows is bitwise
+// the same as in the whole product.
+constexpr int64_t kMvLanes = 1 << 18;
+int mv_row_lanes(int64_t dim, int entries) {
+  int lg = 0;
+  while (lg < 4 && (dim << lg) < kMvLanes && (4 << lg) <= entries) ++lg;
+  return lg;
+}
+
 // Term-list kernel over the output rows [row_begin, row_end) (y holds them
 // from y[0]); x is the whole input vector.
 void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, const void* x, void* y,
@@ -1369,13 +1396,15 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   d.xcd_chunk = g_xcd_chunk.load();
   d.row_begin = row_begin;
   d.dim = row_end;
+  d.row_lanes = mv_row_lanes(sp->dim, d.n_lin + d.n_rest);
+  d.stripe = d.row_lanes == 0 ? ~0ull : ~0ull / ((1ull << (1 << d.row_lanes)) - 1ull);
   if (ensure_diag(op)) {
     d.diag_re = op->diag_re.as<double>();
     d.diag_im = op->diag_im.as<double>();
   }
   op->used_kernel = 1;
   op->used_lookup = rank_mode ? 1 : (d.ix.bm_bits ? 3 : 1);
-  if (attach_spread(op, prec, d, x, st, true)) op->used_lookup = 4;
+  if (attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
   if (idx_lookup == 4 && !d.xm.values) fail(EDHIP_ERR_ARGUMENT, "x cannot be spread over the words of this space");
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
   HIP_OR_THROW(launch_matvec(d, prec, transpose ? 1 : 0, accumulate ? 1 : 0, x, y, st));
@@ -2381,24 +2410,22 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
     op->n_diag = (int)dg.size();
     upload(op->off_row, offr, ctx->stream);
     upload(op->off_col, offc, ctx->stream);
-    // runs of equal masks padded to even lengths (both forms share the masks,
-    // so they pad alike); the padding term keeps the mask, matches nothing
-    // (a match outside the mask) and flips nothing
-    auto pad_runs = [](const std::vector<OffTerm>& v) {
-      std::vector<OffTerm> out;
-      for (size_t i = 0; i < v.size();) {
-        size_t j = i;
-        while (j < v.size() && v[j].mask == v[i].mask) ++j;
-        out.insert(out.end(), v.begin() + i, v.begin() + j);
-        if ((j - i) & 1) out.push_back(OffTerm{v[i].mask, ~v[i].mask, ~v[i].mask, 0.0, 0.0});
-        i = j;
-      }
-      return out;
-    };
-    const std::vector<OffTerm> mvr = pad_runs(offr), mvc = pad_runs(offc);
-    op->n_mv = (int)mvr.size();
-    upload(op->mv_row, mvr, ctx->stream);
-    upload(op->mv_col, mvc, ctx->stream);
+    for (int form = 0; form < 2; ++form) {
+      const std::vector<OffTerm>& v = form ? offc : offr;
+      const MvSplit S = mv_split(v);
+      edhip_op::MvHost& M = op->mv[form];
+      M.n_lin = (int)S.lin.size();
+      M.n_rest = (int)S.rest.size();
+      M.entries = S.lin;
+      for (const OffTerm& o : S.rest) M.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});
+      upload(M.tab, mv_tables(S, space->n_bits), ctx->stream);
+      upload(M.rest, S.rest, ctx->stream);
+      upload(M.ent, M.entries, ctx->stream);
+      edhip_op::MvHost& P = op->mv_plain[form];
+      P.n_rest = (int)v.size();
+      for (const OffTerm& o : v) P.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});
+      upload(P.ent, P.entries, ctx->stream);
+    }
     upload(op->diag, dg, ctx->stream);
     upload(op->all_row, allr, ctx->stream);
     upload(op->all_col, allc, ctx->stream);
@@ -2827,7 +2854,7 @@ int edhip_term_expect(edhip_op* op, int prec, const void* phi, const void* psi, 
     // psi of the images from its spread, as the products read x, where its
     // code table leaves LDS room for the bins
     OpDev d = op->dev_row;
-    if (attach_spread(op, prec, d, psi, op->ctx->stream) && term_expect_window(d, nc) < 1) d.xm = XMapDev{};
+    if (attach_spread(op, prec, d, d.codes_lds, psi, op->ctx->stream) && term_expect_window(d, nc) < 1) d.xm = XMapDev{};
     edhip_ctx* ctx = op->ctx;
     if (ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(ctx->ev[14], ctx->stream));
     HIP_OR_THROW(launch_term_expect(d, prec, phi, psi, op->ex_partial.as<double>(), nb, op->ex_out.as<double>(),

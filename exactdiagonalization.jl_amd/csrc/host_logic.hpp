@@ -1,7 +1,8 @@
 // Host-side logic with no device code, so that a host-only build (with
 // sanitizers) can test it: the linear algebra of the eigensolver's small
 // projected (tridiagonal or arrowhead) matrices, and the closure and
-// inverses of a symmetry group given as bit permutations with XOR words.
+// inverses of a symmetry group given as bit permutations with XOR words, and
+// the split of an operator's terms into the products' entries.
 #pragma once
 
 #include <stdint.h>
@@ -14,6 +15,84 @@
 #include <vector>
 
 namespace edhip {
+
+// Off-diagonal term as the products see it: the row b matches iff
+// (b & mask) == match; its image is (b & ~mask) | image.
+struct OffTerm {
+  uint64_t mask, match, image;
+  double are, aim;
+};
+
+// One entry of the products: a matching row b has the image b ^ flip.
+struct MvEntry {
+  uint64_t flip;
+  double are, aim;
+};
+
+// Parity entries of a list of terms (mv_split): entry e matches b iff
+// parity(b & q[e]) ^ c[e] is 1.
+struct MvSplit {
+  std::vector<uint64_t> q;
+  std::vector<int> c;
+  std::vector<MvEntry> lin;   // the parity entries
+  std::vector<OffTerm> rest;  // the other terms, runs of equal masks padded to even lengths
+};
+
+// Two terms on one mask of one or two bits with the same flip and amplitude
+// whose matches are each other's complement match together wherever the parity
+// of the masked bits has one value (two bits: 01 and 10, or 00 and 11), or
+// everywhere (one bit: 0 and 1): S+S- + S-S+ bonds, transverse fields.  The
+// padding terms of rest keep the mask, match nothing (a match outside the
+// mask) and flip nothing.
+inline MvSplit mv_split(const std::vector<OffTerm>& v) {
+  MvSplit S;
+  std::vector<char> used(v.size(), 0);
+  for (size_t i = 0; i < v.size();) {
+    size_t j = i;
+    while (j < v.size() && v[j].mask == v[i].mask) ++j;
+    const uint64_t m = v[i].mask;
+    const int bits = __builtin_popcountll(m);
+    for (size_t a = i; a < j && (bits == 1 || bits == 2); ++a)
+      for (size_t b = a + 1; b < j && !used[a]; ++b) {
+        if (used[b] || (v[a].match ^ v[b].match) != m || (v[a].match ^ v[a].image) != (v[b].match ^ v[b].image) ||
+            v[a].are != v[b].are || v[a].aim != v[b].aim)
+          continue;
+        used[a] = used[b] = 1;
+        S.q.push_back(bits == 2 ? m : 0);
+        S.c.push_back(bits == 2 ? 1 ^ (__builtin_popcountll(v[a].match) & 1) : 1);
+        S.lin.push_back(MvEntry{v[a].match ^ v[a].image, v[a].are, v[a].aim});
+      }
+    size_t kept = 0;
+    for (size_t a = i; a < j; ++a)
+      if (!used[a]) {
+        S.rest.push_back(v[a]);
+        ++kept;
+      }
+    if (kept & 1) S.rest.push_back(OffTerm{m, ~m, ~m, 0.0, 0.0});
+    i = j;
+  }
+  return S;
+}
+
+// 4-bit chunks of nb-bit words, rounded up to a multiple of 3 (the unroll of
+// the kernels' loop over them).
+inline int mv_chunks(int nb) { return ((nb + 3) / 4 + 2) / 3 * 3; }
+
+// The parity tables: bit e of the XOR over the chunks k of entry
+// [segment][k][k-th chunk of b] tells whether entry 64 segment + e matches b.
+inline std::vector<uint64_t> mv_tables(const MvSplit& S, int nb) {
+  const int nc = mv_chunks(nb);
+  const size_t n_seg = (S.lin.size() + 63) / 64;
+  std::vector<uint64_t> tab(n_seg * (size_t)nc * 16, 0);
+  for (size_t e = 0; e < S.lin.size(); ++e)
+    for (int k = 0; k < nc; ++k)
+      for (int x = 0; x < 16; ++x) {
+        const uint64_t part = 4 * k < 64 ? (uint64_t)x << (4 * k) : 0;
+        const int bit = (__builtin_popcountll(part & S.q[e]) & 1) ^ (k == 0 ? S.c[e] : 0);
+        if (bit) tab[((e / 64) * nc + (size_t)k) * 16 + (size_t)x] |= 1ull << (e % 64);
+      }
+  return tab;
+}
 
 // Householder reduction of a dense symmetric matrix (row-major, n x n) to
 // tridiagonal form A = Q T Q^T; returns d (diagonal), e (e[i] = T[i][i+1]).

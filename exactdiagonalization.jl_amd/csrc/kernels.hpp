@@ -78,18 +78,24 @@ hipError_t exclusive_scan_u32_to_u64(const uint32_t* d_in, uint64_t* d_out, uint
 hipError_t exclusive_scan_i64(const int64_t* d_in, int64_t* d_out, uint64_t n, void* d_tmp, size_t& tmp_bytes,
                               hipStream_t st);
 
-// ---- matvec.hip ------------------------------------------------------------
-// Off-diagonal term as the matvec sees it: the row matches iff
-// (b & mask) == match; its image is (b & ~mask) | image.
-struct OffTerm {
-  uint64_t mask, match, image;
-  double are, aim;
-};
-
+// ---- matvec.hip, product_*.hip ---------------------------------------------
 struct DiagTerm {
   uint64_t mask, match;
   double are, aim;
 };
+
+// LDS offsets of the products' entries, from mv_lds.
+struct MvLayout {
+  uint32_t off_mm, off_fa, off_ai, total;
+};
+__host__ __device__ __forceinline__ MvLayout mv_layout(int n_lin, int n_chunk, int n_rest, int paired) {
+  MvLayout Y;
+  Y.off_mm = (uint32_t)(((n_lin + 63) / 64) * n_chunk) * 128u;
+  Y.off_fa = (Y.off_mm + (uint32_t)(paired ? n_rest / 2 * 24 : n_rest * 16) + 15u) & ~15u;
+  Y.off_ai = Y.off_fa + (uint32_t)(n_lin + n_rest) * 16u;
+  Y.total = Y.off_ai + (uint32_t)(n_lin + n_rest) * 8u;
+  return Y;
+}
 
 struct OpDev {
   IndexDev ix;           // lookup of canonical images
@@ -104,12 +110,20 @@ struct OpDev {
   int word_bits;         // bits of the words and of every diagonal term's mask and match
   int xcd_chunk;         // products: consecutive blocks each XCD takes per window of 8 xcd_chunk (<= 1: plain order)
   const OffTerm* off;    // row form: match = R, image = C ; column form: match = C, image = R
-  // The matvec's copy of off: every run of equal masks padded to an even
-  // length (padding terms carry the run's mask, a match outside it and no
-  // flip), so terms 2q and 2q + 1 share a mask and are matched together.
-  const OffTerm* mv_off;
-  int n_mv;              // padded length (0: the matvec matches off term by term)
-  int pad_mv_;
+  // The entries of the products (each an off-diagonal term, or two with one
+  // flip and amplitude): n_lin parity entries, matched 64 at a time through
+  // the tables lin_tab, then n_rest others matched by mask (rest).  Operators
+  // without LDS room for them match off term by term (n_lin = 0, rest = off).
+  const MvEntry* ent;       // n_lin + n_rest
+  const uint64_t* lin_tab;  // [segment of 64 entries][chunk of 4 word bits][16]
+  const OffTerm* rest;
+  int n_lin;
+  int n_chunk;              // chunks per segment (a multiple of 3; those past the word are zero)
+  int n_rest;
+  int rest_paired;          // rest comes in pairs that share a mask (runs of equal masks padded to even lengths
+                            // with terms that match nothing and flip nothing)
+  int row_lanes;            // products: log2 of the lanes that share a row
+  uint64_t stripe;          // products: bits of a segment that the first of them takes
   const DiagTerm* diag;
   const double* diag_re; // per-row diagonal element (summed diagonal terms), or nullptr
   const double* diag_im; // its imaginary part, or nullptr when every diagonal amplitude is real
@@ -118,7 +132,11 @@ struct OpDev {
   uint32_t w_bytes;
   XMapDev xm;            // matvec: x read from its spread over word positions (xm.values != null)
   uint32_t codes_lds;    // LDS offset of xm's code table, after lds_total (0: no room)
-  uint32_t lds_total;    // LDS of the kernels (the matvec adds xm's code table)
+  uint32_t lds_total;    // LDS of the kernels (the term pass adds xm's code table)
+  uint32_t mv_lds;       // the products' LDS: entries (mv_layout), rank table, xm's code table
+  uint32_t mv_w_lds;
+  uint32_t mv_codes_lds; // (0: no room for xm's code table)
+  uint32_t mv_lds_total; // without xm's code table
 };
 
 enum Prec : int { kF64 = 0, kC128 = 1, kF32 = 2, kC64 = 3 };
@@ -127,12 +145,18 @@ enum Prec : int { kF64 = 0, kC128 = 1, kF32 = 2, kC64 = 3 };
 hipError_t launch_matvec(const OpDev& op, int prec, int transpose, int accumulate, const void* x, void* y,
                          hipStream_t st);
 
+// the same for one vector type (product_*.hip)
+hipError_t launch_product_f32(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
+hipError_t launch_product_f64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
+hipError_t launch_product_c64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
+hipError_t launch_product_c128(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
+
 // ---- assembled rows (row form): entries col | cls << col_bits per image ----
 constexpr int kAsmMaxClasses = 256;
 struct AsmFillDev {
   const uint64_t* rowptr;  // dim + 1 offsets of the rows' entries
   uint32_t* ent;
-  const uint32_t* acls;    // per matvec term: amplitude class, 1-based
+  const uint32_t* acls;    // per product entry: amplitude class, 1-based
   const uint32_t* pcls;    // per group element: phase class (nullptr: every phase 1)
   int n_ph;
   int col_bits;

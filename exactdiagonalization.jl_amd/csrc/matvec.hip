@@ -1,164 +1,11 @@
-// Matrix-free application of an operator on a (possibly symmetry-reduced)
-// basis, in gather form with no atomics: one lane owns one output entry.
-//
-// Row form (apply!(out, opr, state), abstract_operator_representation.jl:296-316):
-//   y[r] += sum_t [ (b_r & m_t) == R_t ] w * x[s],  image b' = (b_r & ~m_t) | C_t
-// Column form (apply!(out, state, opr), :327-347) swaps R_t and C_t and uses
-// the column element of reduced_operator_representation.jl:88-116.
-//
-// For a reduced basis, b' is canonicalised to its representative s = h(b'),
-// and the element is a * phase[h] * sqrt(N_r / N_s) (row form) with
-// phase[h] = conj(chi(h^-1)); this equals a * U[b'] / U[b_r] of
-// reduced_operator_representation.jl:57-85 with U[g(s)] = conj(chi(g))/sqrt(N_s).
-#include <type_traits>
-
-#include "kernels.hpp"
+// The other kernels that walk an operator: diagonal elements, raw iterators,
+// sparse and dense export, term expectations, assembled rows, pair groups.
+#include "opterms.hpp"
 
 namespace edhip {
 
 namespace {
 
-constexpr int kBlock = 256;
-
-template <int MODE>
-struct Canon {
-  // NEED_H = false: h is left 0 where the canonicaliser can skip tracking it
-  template <bool NEED_H = true>
-  __device__ __forceinline__ static void run(const GroupDev& g, const GroupLds& L, uint64_t b, uint64_t& s, int& h,
-                                             int& cnt) {
-    if constexpr (MODE == kGroupNone) {
-      s = b;
-      h = 0;
-      cnt = 1;
-    } else if constexpr (MODE == kGroupTorusPairs) {
-      canonicalize_torus_pairs<0, 0, NEED_H>(g, L, b, s, h, cnt);
-    } else if constexpr (MODE == kTorusPairs6x6) {
-      canonicalize_torus_pairs<6, 6, NEED_H>(g, L, b, s, h, cnt);
-    } else if constexpr (MODE == kTorusPairs4x6) {
-      canonicalize_torus_pairs<4, 6, NEED_H>(g, L, b, s, h, cnt);
-    } else if constexpr (MODE == kTorusPairs6x4) {
-      canonicalize_torus_pairs<6, 4, NEED_H>(g, L, b, s, h, cnt);
-    } else if constexpr (MODE == kTorusPairs4x4) {
-      canonicalize_torus_pairs<4, 4, NEED_H>(g, L, b, s, h, cnt);
-    } else if constexpr (MODE >= kTransPairs6x6 && MODE <= kTransPairs4x4) {
-      // translations only: the identity coset, whose element table maps the
-      // translation found to the group element
-      constexpr int LX = (MODE == kTransPairs6x6 || MODE == kTransPairs6x4) ? 6 : 4;
-      constexpr int LY = (MODE == kTransPairs6x6 || MODE == kTransPairs4x6) ? 6 : 4;
-      int pos;
-      canonicalize_torus_pairs_t<LX, LY, NEED_H>(g, L, L.coset_inv, b, s, pos, cnt);
-      h = NEED_H ? L.coset_elem[pos] : 0;
-    } else {
-      canonicalize(g, L, b, s, h, cnt);
-    }
-  }
-};
-
-struct Staged {
-  GroupLds L;
-  const OffTerm* off;
-  const uint64_t* W;
-};
-
-template <int MODE>
-__device__ __forceinline__ Staged stage_op(const OpDev& op, unsigned char* lds) {
-  Staged S;
-  if constexpr (MODE != kGroupNone) {
-    S.L = stage_group(op.g, op.lay, lds);
-  }
-  lds_copy(lds + op.off_lds, op.off, (uint32_t)(op.n_off * sizeof(OffTerm)));
-  S.off = (const OffTerm*)(lds + op.off_lds);
-  lds_copy(lds + op.w_lds, op.ix.W, op.w_bytes);
-  S.W = (const uint64_t*)(lds + op.w_lds);
-  return S;
-}
-
-// The matvec's copy of the off-diagonal terms in LDS, split by use: (mask,
-// match) pairs read by every lane alike while matching a row, and (flip,
-// amplitude) pairs read per matched term, where flip = match ^ image gives the
-// image of a matching row b as b ^ flip; imaginary parts apart.
-struct MvTerms {
-  const uint64_t* mm;  // term by term: mask, match; paired (n_mv): mask, match 2q, match 2q+1
-  const uint64_t* fa;  // 2 per term: flip, bits of Re(amplitude)
-  const double* ai;    // Im(amplitude)
-};
-
-// paired: the padded copy (op.n_mv > 0) with one mask per pair of terms;
-// else the terms of op.off one by one, indexed as in op.off.  amp32: the real
-// amplitude is kept as an FP32 value in the low half of its slot.
-__device__ __forceinline__ MvTerms stage_mv_terms(const OpDev& op, unsigned char* lds, bool paired,
-                                                  bool amp32 = false) {
-  const int n = paired ? op.n_mv : op.n_off;
-  const OffTerm* src = paired ? op.mv_off : op.off;
-  uint64_t* mm = (uint64_t*)(lds + op.off_lds);  // at most 40 bytes per term, as reserved
-  uint64_t* fa = mm + (paired ? 3 * (n / 2) : 2 * n);
-  double* ai = (double*)(fa + 2 * n);
-  for (int t = threadIdx.x; t < n; t += blockDim.x) {
-    const OffTerm o = src[t];
-    if (paired) {
-      if ((t & 1) == 0) {
-        mm[3 * (t >> 1)] = o.mask;
-        mm[3 * (t >> 1) + 1] = o.match;
-      } else {
-        mm[3 * (t >> 1) + 2] = o.match;
-      }
-    } else {
-      mm[2 * t] = o.mask;
-      mm[2 * t + 1] = o.match;
-    }
-    fa[2 * t] = o.match ^ o.image;
-    fa[2 * t + 1] = amp32 ? (uint64_t)__float_as_uint((float)o.are) : (uint64_t)__double_as_longlong(o.are);
-    ai[t] = o.aim;
-  }
-  return MvTerms{mm, fa, ai};
-}
-
-// Weight of an off-diagonal element: a * phase^(conj if TRANS) * sqrt(N_own) / sqrt(N_img)
-// (SCALED: without 1 / sqrt(N_img), which the spread x / sqrt(N) carries)
-template <int MODE, bool TRANS, bool UNIT = false, bool SCALED = false>
-__device__ __forceinline__ void element_weight_a(const OpDev& op, const GroupLds& L, double are, double aim, int h,
-                                                 int cnt, double sqrt_own, double& wr, double& wi) {
-  if constexpr (MODE == kGroupNone) {
-    wr = are;
-    wi = aim;
-  } else {
-    const double sc = SCALED ? sqrt_own : sqrt_own * L.sqcnt[cnt];
-    if (UNIT || op.g.unit_phases) {
-      wr = are * sc;
-      wi = aim * sc;
-    } else {
-      const double pr = L.ph_re[h];
-      const double pi = TRANS ? -L.ph_im[h] : L.ph_im[h];
-      wr = (are * pr - aim * pi) * sc;
-      wi = (are * pi + aim * pr) * sc;
-    }
-  }
-}
-
-template <int MODE, bool TRANS>
-__device__ __forceinline__ void element_weight(const OpDev& op, const Staged& S, const OffTerm& t, int h, int cnt,
-                                               double sqrt_own, double& wr, double& wi) {
-  if constexpr (MODE == kGroupNone) {
-    wr = t.are;
-    wi = t.aim;
-  } else {
-    double pr = S.L.ph_re[h];
-    double pi = TRANS ? -S.L.ph_im[h] : S.L.ph_im[h];
-    double sc = sqrt_own * S.L.sqcnt[cnt];
-    wr = (t.are * pr - t.aim * pi) * sc;
-    wi = (t.are * pi + t.aim * pr) * sc;
-  }
-}
-
-__device__ __forceinline__ void diag_sum(const OpDev& op, uint64_t b, double& dre, double& dim_) {
-  for (int t = 0; t < op.n_diag; ++t) {
-    const DiagTerm d = op.diag[t];
-    if ((b & d.mask) == d.match) {
-      dre += d.are;
-      dim_ += d.aim;
-    }
-  }
-}
 
 __global__ __launch_bounds__(kBlock) void k_diag_values(OpDev op, double* __restrict__ re, double* __restrict__ im) {
   const int64_t row = (int64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -169,178 +16,6 @@ __global__ __launch_bounds__(kBlock) void k_diag_values(OpDev op, double* __rest
   if (im) im[row] = dim_;
 }
 
-// The matvec runs 512-lane blocks, one row per lane, over a grid that covers
-// the rows in order (blocks that run together work on neighbouring rows, whose
-// images share cache lines of the index and of x).
-constexpr int kMvBlock = 512;
-
-// UNIT: every character is 1 (op.g.unit_phases): the weight needs no phase,
-// so the canonicaliser does not track the element reaching the image.
-// SCALED: x is read from its spread holding x / sqrt(N) (op.xm.scaled), so the
-// weight needs no orbit size of the image and the stabiliser goes uncounted.
-template <typename V, int MODE, bool TRANS, bool UNIT, bool SCALED>
-__global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restrict__ x, V* __restrict__ y, int accumulate) {
-  extern __shared__ unsigned char lds[];
-  GroupLds L{};
-  if constexpr (MODE != kGroupNone) L = stage_group(op.g, op.lay, lds);
-  // FP32 weights: a real FP32 product whose images need no phase and no orbit
-  // size (unit characters, scaled spread) weighs each image a * sqrt(N_r) in
-  // FP32, from FP32 amplitudes (no FP64 multiply and conversion per image)
-  constexpr bool kW32 = UNIT && SCALED && std::is_same<V, float>::value;
-  const MvTerms T = stage_mv_terms(op, lds, op.n_mv != 0, kW32);
-  lds_copy(lds + op.w_lds, op.ix.W, op.w_bytes);
-  const uint64_t* W = (const uint64_t*)(lds + op.w_lds);
-  // code table of the spread x (the host sets xm only with room for it)
-  uint16_t* codes = (uint16_t*)(lds + op.codes_lds);
-  if (op.xm.values) xmap_stage(op.xm, codes);
-  __syncthreads();
-  const int64_t row = op.row_begin + xcd_chunked_block(blockIdx.x, gridDim.x, op.xcd_chunk) * kMvBlock + threadIdx.x;
-  if (row >= op.dim) return;
-  using R = typename VT<V>::R;
-  const uint64_t b = op.rows[row];
-
-  // diagonal terms (C == R): the element is the summed amplitude (U[b]/U[b] = 1)
-  double dre = 0.0, dim_ = 0.0;
-  if (op.diag_re) {
-    dre = op.diag_re[row];
-    if (op.diag_im) dim_ = op.diag_im[row];
-  } else {
-    diag_sum(op, b, dre, dim_);
-  }
-  V acc = vzero<V>();
-  vfma(acc, (R)dre, (R)dim_, x[row]);
-
-  double sqrt_own = 1.0;
-  if constexpr (MODE != kGroupNone) sqrt_own = sqrt((double)op.orbit[row]);
-  const float so32 = (float)sqrt_own;
-
-  const int n_terms = op.n_mv ? op.n_mv : op.n_off;
-  for (int seg = 0; seg < n_terms; seg += 64) {
-    const int nseg = (n_terms - seg) < 64 ? (n_terms - seg) : 64;
-    uint64_t bits = 0;
-    if (op.n_mv) {  // two terms with one mask per test (nseg is even)
-      for (int j = 0; j < nseg; j += 2) {
-        const uint64_t* m = T.mm + 3 * ((seg + j) >> 1);
-        const uint64_t xm = b & m[0];
-        bits |= (uint64_t)((uint32_t)(xm == m[1]) | ((uint32_t)(xm == m[2]) << 1)) << j;
-      }
-    } else {
-      for (int j = 0; j < nseg; ++j) {
-        const uint64_t* m = T.mm + 2 * (seg + j);
-        bits |= (uint64_t)((b & m[0]) == m[1]) << j;
-      }
-    }
-    // two images per step: both canonical forms first, then both lookups and
-    // both x gathers issued before either is used (twice the loads in flight;
-    // measured 5% faster at 6x6 than one image per step, three or four per
-    // step are slower: more steps end with an empty slot)
-    constexpr int NW = 2;
-    while (bits) {
-      int t[NW];
-      bool ok[NW];
-      t[0] = seg + __builtin_ctzll(bits);  // bits != 0 here
-      ok[0] = true;
-      bits &= bits - 1;
-#pragma unroll
-      for (int k = 1; k < NW; ++k) {  // an empty slot repeats the first image and is dropped
-        ok[k] = bits != 0;
-        t[k] = ok[k] ? seg + __builtin_ctzll(bits) : t[0];
-        bits &= ok[k] ? bits - 1 : bits;
-      }
-      ulonglong2 fa[NW];  // flip = match ^ image: a matching row b has the image b ^ flip
-      uint64_t sk[NW];
-      int hk[NW], ck[NW];
-#pragma unroll
-      for (int k = 0; k < NW; ++k) {
-        fa[k] = *(const ulonglong2*)(T.fa + 2 * t[k]);
-        Canon<MODE>::template run<!UNIT>(op.g, L, b ^ fa[k].x, sk[k], hk[k], ck[k]);
-      }
-      int64_t ik[NW];
-      V xv[NW];
-      if (op.xm.values) {  // x of each image with one load at its word position
-        bool f0, f1;
-        xmap_fetch2(op.xm, codes, sk[0], sk[1], xv[0], xv[1], f0, f1);
-        ik[0] = f0 ? 0 : -1;
-        ik[1] = (ok[1] && f1) ? 0 : -1;
-      } else {
-        index_of2(op.ix, W, sk[0], sk[1], ik[0], ik[1]);
-#pragma unroll
-        for (int k = 0; k < NW; ++k) {
-          ik[k] = ok[k] ? ik[k] : -1;
-          xv[k] = x[ik[k] >= 0 ? ik[k] : 0];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < NW; ++k) {
-        if (ik[k] >= 0) {
-          if constexpr (kW32) {
-            vfma(acc, __uint_as_float((uint32_t)fa[k].y) * so32, 0.f, xv[k]);
-          } else {
-            double wr, wi;
-            element_weight_a<MODE, TRANS, UNIT, SCALED>(op, L, __longlong_as_double((long long)fa[k].y),
-                                                  VT<V>::cx ? T.ai[t[k]] : 0.0, hk[k], ck[k], sqrt_own, wr, wi);
-            vfma(acc, (R)wr, (R)wi, xv[k]);
-          }
-        }
-      }
-    }
-  }
-  V* yr = y + (row - op.row_begin);
-  *yr = accumulate ? vadd(*yr, acc) : acc;
-}
-
-template <typename V, int MODE>
-hipError_t launch_mv_t(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st) {
-  dim3 grid((unsigned)((op.dim - op.row_begin + kMvBlock - 1) / kMvBlock));
-  // unit-phase kernels only where the canonicaliser can drop the element (row-pair tori)
-  const bool unit = MODE >= kGroupTorusPairs && op.g.unit_phases;
-  const uint32_t lds = op.xm.values ? op.codes_lds + xmap_lds_bytes(op.xm) : op.lds_total;
-#define EDHIP_MV(T, U, S)                                                                                              \
-  hipLaunchKernelGGL((k_matvec<V, MODE, T, U, S>), grid, dim3(kMvBlock), lds, st, op, (const V*)x, (V*)y, accumulate)
-  if constexpr (MODE != kGroupNone) {
-    if (op.xm.values && op.xm.scaled) {
-      if (transpose) {
-        if (unit) EDHIP_MV(true, MODE >= kGroupTorusPairs, true); else EDHIP_MV(true, false, true);
-      } else {
-        if (unit) EDHIP_MV(false, MODE >= kGroupTorusPairs, true); else EDHIP_MV(false, false, true);
-      }
-      return hipGetLastError();
-    }
-  }
-  if (transpose) {
-    if (unit) EDHIP_MV(true, MODE >= kGroupTorusPairs, false); else EDHIP_MV(true, false, false);
-  } else {
-    if (unit) EDHIP_MV(false, MODE >= kGroupTorusPairs, false); else EDHIP_MV(false, false, false);
-  }
-#undef EDHIP_MV
-  return hipGetLastError();
-}
-
-template <typename V>
-hipError_t launch_mv_v(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st) {
-  switch (op.g.mode) {
-    case kGroupNone:
-      return launch_mv_t<V, kGroupNone>(op, transpose, accumulate, x, y, st);
-    case kGroupGeneric:
-      return launch_mv_t<V, kGroupGeneric>(op, transpose, accumulate, x, y, st);
-    default:
-      if (op.g.pair_table) {
-        const int Lx = op.g.Lx, Ly = op.g.Ly;
-        if (op.g.n_cosets == 1) {
-          if (Lx == 6 && Ly == 6) return launch_mv_t<V, kTransPairs6x6>(op, transpose, accumulate, x, y, st);
-          if (Lx == 4 && Ly == 6) return launch_mv_t<V, kTransPairs4x6>(op, transpose, accumulate, x, y, st);
-          if (Lx == 6 && Ly == 4) return launch_mv_t<V, kTransPairs6x4>(op, transpose, accumulate, x, y, st);
-          if (Lx == 4 && Ly == 4) return launch_mv_t<V, kTransPairs4x4>(op, transpose, accumulate, x, y, st);
-        }
-        if (Lx == 6 && Ly == 6) return launch_mv_t<V, kTorusPairs6x6>(op, transpose, accumulate, x, y, st);
-        if (Lx == 4 && Ly == 6) return launch_mv_t<V, kTorusPairs4x6>(op, transpose, accumulate, x, y, st);
-        if (Lx == 6 && Ly == 4) return launch_mv_t<V, kTorusPairs6x4>(op, transpose, accumulate, x, y, st);
-        if (Lx == 4 && Ly == 4) return launch_mv_t<V, kTorusPairs4x4>(op, transpose, accumulate, x, y, st);
-        return launch_mv_t<V, kGroupTorusPairs>(op, transpose, accumulate, x, y, st);
-      }
-      return launch_mv_t<V, kGroupTorus>(op, transpose, accumulate, x, y, st);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // Raw iterators (index or -1, value) in term order, for a list of rows.
@@ -578,7 +253,7 @@ __global__ __launch_bounds__(kBlock) void k_term_expect(OpDev op, const V* __res
   extern __shared__ unsigned char lds[];
   GroupLds L{};
   if constexpr (MODE != kGroupNone) L = stage_group(op.g, op.lay, lds);
-  const MvTerms T = stage_mv_terms(op, lds, false);
+  const PlainTerms T = stage_plain_terms(op, lds);
   lds_copy(lds + op.w_lds, op.ix.W, op.w_bytes);
   const uint64_t* W = (const uint64_t*)(lds + op.w_lds);
   // psi of the images from its spread over the word positions (op.xm set):
@@ -895,60 +570,44 @@ hipError_t launch_expect_v(const OpDev& op, const void* phi, const void* psi, do
 // (prepared once per product) and scales each row's sum by sqrt(N_r).
 // ---------------------------------------------------------------------------
 
-// Bits of the terms seg .. seg + nseg - 1 (nseg <= 64) that match the word b,
-// as the matvec tests them (two terms per mask test on the paired copy).
-__device__ __forceinline__ uint64_t match_bits(const OpDev& op, const MvTerms& T, uint64_t b, int seg, int nseg) {
-  uint64_t bits = 0;
-  if (op.n_mv) {
-    for (int j = 0; j < nseg; j += 2) {
-      const uint64_t* m = T.mm + 3 * ((seg + j) >> 1);
-      const uint64_t xm = b & m[0];
-      bits |= (uint64_t)((uint32_t)(xm == m[1]) | ((uint32_t)(xm == m[2]) << 1)) << j;
-    }
-  } else {
-    for (int j = 0; j < nseg; ++j) {
-      const uint64_t* m = T.mm + 2 * (seg + j);
-      bits |= (uint64_t)((b & m[0]) == m[1]) << j;
-    }
-  }
-  return bits;
-}
-
 // counts[r] = number of terms matching row r (the entries it will hold)
 __global__ __launch_bounds__(kMvBlock) void k_asm_count(OpDev op, uint32_t* __restrict__ counts) {
   extern __shared__ unsigned char lds[];
-  const MvTerms T = stage_mv_terms(op, lds, op.n_mv != 0);
+  const MvTerms T = stage_mv_terms(op, lds, false, false);
   __syncthreads();
   const int64_t row = (int64_t)blockIdx.x * kMvBlock + threadIdx.x;
   if (row >= op.dim) return;
   const uint64_t b = op.rows[row];
-  const int n_terms = op.n_mv ? op.n_mv : op.n_off;
+  const int n_seg = mv_segments(op);
   uint32_t n = 0;
-  for (int seg = 0; seg < n_terms; seg += 64)
-    n += (uint32_t)__builtin_popcountll(match_bits(op, T, b, seg, (n_terms - seg) < 64 ? (n_terms - seg) : 64));
+  for (int seg = 0; seg < n_seg; ++seg) {
+    int base;
+    n += (uint32_t)__builtin_popcountll(mv_match(op, T, b, seg, base));
+  }
   counts[row] = n;
 }
 
-// Entries of every row: acls[t] is the amplitude class (1-based) of matvec
-// term t; with phases, cls = 1 + (acls - 1) * n_ph + pcls[h].
+// Entries of every row: acls[t] is the amplitude class (1-based) of product
+// entry t; with phases, cls = 1 + (acls - 1) * n_ph + pcls[h].
 template <int MODE, bool UNIT>
 __global__ __launch_bounds__(kMvBlock) void k_asm_fill(OpDev op, AsmFillDev a) {
   extern __shared__ unsigned char lds[];
   GroupLds L{};
   if constexpr (MODE != kGroupNone) L = stage_group(op.g, op.lay, lds);
-  const MvTerms T = stage_mv_terms(op, lds, op.n_mv != 0);
-  lds_copy(lds + op.w_lds, op.ix.W, op.w_bytes);
-  const uint64_t* W = (const uint64_t*)(lds + op.w_lds);
+  const MvTerms T = stage_mv_terms(op, lds, false, false);
+  lds_copy(lds + op.mv_w_lds, op.ix.W, op.w_bytes);
+  const uint64_t* W = (const uint64_t*)(lds + op.mv_w_lds);
   __syncthreads();
   const int64_t row = (int64_t)blockIdx.x * kMvBlock + threadIdx.x;
   if (row >= op.dim) return;
   const uint64_t b = op.rows[row];
   uint32_t* out = a.ent + a.rowptr[row];
-  const int n_terms = op.n_mv ? op.n_mv : op.n_off;
-  for (int seg = 0; seg < n_terms; seg += 64) {
-    uint64_t bits = match_bits(op, T, b, seg, (n_terms - seg) < 64 ? (n_terms - seg) : 64);
+  const int n_seg = mv_segments(op);
+  for (int seg = 0; seg < n_seg; ++seg) {
+    int base;
+    uint64_t bits = mv_match(op, T, b, seg, base);
     while (bits) {
-      const int t = seg + __builtin_ctzll(bits);
+      const int t = base + __builtin_ctzll(bits);
       bits &= bits - 1;
       uint64_t s;
       int h, cnt;
@@ -1068,9 +727,9 @@ template <int MODE>
 hipError_t launch_asm_fill_t(const OpDev& op, const AsmFillDev& a, hipStream_t st) {
   dim3 grid((unsigned)((op.dim + kMvBlock - 1) / kMvBlock));
   if (MODE == kGroupNone || op.g.unit_phases)
-    hipLaunchKernelGGL((k_asm_fill<MODE, true>), grid, dim3(kMvBlock), op.lds_total, st, op, a);
+    hipLaunchKernelGGL((k_asm_fill<MODE, true>), grid, dim3(kMvBlock), op.mv_lds_total, st, op, a);
   else
-    hipLaunchKernelGGL((k_asm_fill<MODE, false>), grid, dim3(kMvBlock), op.lds_total, st, op, a);
+    hipLaunchKernelGGL((k_asm_fill<MODE, false>), grid, dim3(kMvBlock), op.mv_lds_total, st, op, a);
   return hipGetLastError();
 }
 
@@ -1106,7 +765,7 @@ hipError_t launch_asm_spmv_v(const OpDev& op, const AsmDev& a, int lanes, int ba
 
 hipError_t launch_asm_count(const OpDev& op, uint32_t* d_counts, hipStream_t st) {
   if (op.dim == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_asm_count, dim3((unsigned)((op.dim + kMvBlock - 1) / kMvBlock)), dim3(kMvBlock), op.lds_total,
+  hipLaunchKernelGGL(k_asm_count, dim3((unsigned)((op.dim + kMvBlock - 1) / kMvBlock)), dim3(kMvBlock), op.mv_lds_total,
                      st, op, d_counts);
   return hipGetLastError();
 }
@@ -1198,13 +857,13 @@ hipError_t launch_matvec(const OpDev& op, int prec, int transpose, int accumulat
   if (op.dim <= op.row_begin) return hipSuccess;
   switch (prec) {
     case kF64:
-      return launch_mv_v<double>(op, transpose, accumulate, x, y, st);
+      return launch_product_f64(op, transpose, accumulate, x, y, st);
     case kC128:
-      return launch_mv_v<Cx<double>>(op, transpose, accumulate, x, y, st);
+      return launch_product_c128(op, transpose, accumulate, x, y, st);
     case kF32:
-      return launch_mv_v<float>(op, transpose, accumulate, x, y, st);
+      return launch_product_f32(op, transpose, accumulate, x, y, st);
     case kC64:
-      return launch_mv_v<Cx<float>>(op, transpose, accumulate, x, y, st);
+      return launch_product_c64(op, transpose, accumulate, x, y, st);
     default:
       return hipErrorInvalidValue;
   }

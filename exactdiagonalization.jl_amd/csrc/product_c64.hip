@@ -1,0 +1,11 @@
+// The product kernels for one vector type (one translation unit per type: they
+// compile side by side).
+#include "product.hpp"
+
+namespace edhip {
+
+hipError_t launch_product_c64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st) {
+  return launch_mv_v<Cx<float>>(op, transpose, accumulate, x, y, st);
+}
+
+}  // namespace edhip
