@@ -202,7 +202,7 @@ struct GroupHost {
   int n_cosets = 1;  // torus: cosets T p of the translations
   // device tables
   DevBuf nib, minrot, pair, rot_hi, rot_lo, g_of_ab, inv_d, trivial, ph_re, ph_im, invsqrt, sqcnt, xr_d, coset_nib_d,
-      coset_pidx_d, coset_xr_d, coset_kind_d, coset_elem_d, coset_inv_d;
+      coset_pidx_d, coset_xr_d, coset_kind_d, coset_elem_d, coset_inv_d, win_tab, win_elem;
   GroupDev dev{};
   GroupLdsLayout lay{};
 };
@@ -379,10 +379,12 @@ struct edhip_space {
         std::vector<uint32_t> fl((size_t)1 << t);
         HIP_OR_THROW(hipMemcpyAsync(fl.data(), flags.p, fl.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
         ctx->sync();
-        codes.assign(fl.size(), 0xffff);
         nc = 0;
-        for (size_t v = 0; v < fl.size(); ++v)
-          if (fl[v]) codes[v] = (uint16_t)nc++;
+        for (size_t v = 0; v < fl.size(); ++v) nc += fl[v] ? 1 : 0;
+        codes.assign(fl.size() + 8, (uint16_t)nc);  // (one for words past the table, the others to pad to 16 bytes)
+        for (size_t v = 0, q = 0; v < fl.size(); ++v)
+          if (fl[v]) codes[v] = (uint16_t)q++;
+        ++nc;  // the code of no basis word has positions too, which stay 0
         if (!xcolex_on || ((nc << (sh - 12)) * (uint64_t)kColexStride >> 32) == 0) break;
       }
       upload(xtop, codes, ctx->stream);
@@ -411,7 +413,8 @@ struct edhip_space {
       HIP_OR_THROW(hipMemsetAsync(X.values.p, 0, n_pos * es, ctx->stream));
       ctx->sync();
       X.dev = XMapDev{X.values.p, xtop.as<uint16_t>(), xcolex_on ? xcolex.as<uint16_t>() : nullptr, xtop_K,
-                      xtop_bits, xtop_shift, xcolex_on ? xtop_shift - 12 : 0, single_popcount(), 0};
+                      xtop_bits, xtop_shift, xcolex_on ? xtop_shift - 12 : 0, single_popcount(), 0,
+                      n_bits - xtop_shift <= 32 ? 1 : 0};
       X.ok = true;
       return &X;
     } catch (const Error& e) {
@@ -783,6 +786,15 @@ void build_group(GroupHost& gh, int nb, double tol, hipStream_t st) {
         if (cxr[c]) d.cx_bits |= 1u << c;
       }
     }
+    if (nc == 1 && win_kind(bestLx, bestLy) != kWinNone) {
+      upload(gh.win_tab, win_table(bestLx, bestLy), st);
+      std::vector<int32_t> elem(64, 0);
+      const std::vector<int> pos = win_positions(bestLx, bestLy);
+      for (int bit = 0; bit < 64; ++bit) elem[(size_t)bit] = coset_elem[(size_t)pos[(size_t)bit]];
+      upload(gh.win_elem, elem, st);
+      d.win_tab = gh.win_tab.as<uint16_t>();
+      d.win_elem = gh.win_elem.as<int32_t>();
+    }
     L.bytes_cnib = (uint32_t)(cnib.size() * 8);
     L.bytes_cxr = (uint32_t)(nc * 8);
     L.bytes_ckind = (uint32_t)(nc * 4);
@@ -1021,7 +1033,8 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
     d.lay.total = d.lay.off_pair;
   }
   // (room for the largest code table of the spread x and the colex rank table)
-  const uint32_t codes_bytes = (2u << kXTopBits) + 2u * 4096u;
+  const uint32_t codes_bytes = kXCodesBytesMax + 2u * 4096u;
+  static_assert(kXTopBits == 12, "kXCodesBytesMax");
   d.off_lds = d.mv_lds = align_up(d.lay.total, 16);
   d.w_bytes = w_bytes;
   d.w_lds = d.off_lds + plain_bytes;
@@ -1147,14 +1160,14 @@ FastOpDev make_fast(edhip_op* op, int transpose, const HashDev* hash) {
 
 // y = (accumulate ? y : 0) + A x (or x A), choosing the kernel and lookup.
 // Per-row diagonal elements, computed once per operator when the operator
-// has more than one diagonal term and the array (8 or 16 bytes per row) stays
+// has diagonal terms and the array (8 or 16 bytes per row) stays
 // under 16 GiB; the matvec then reads one number per row instead of looping
 // over the diagonal terms.  Returns false when not cached.
 bool ensure_diag(edhip_op* op) {
   if (op->diag_tried) return op->diag_re.p != nullptr;
   op->diag_tried = true;
   const int64_t D = op->space->dim;
-  if (op->n_diag < 2 || D == 0) return false;
+  if (op->n_diag < 1 || D == 0) return false;
   bool cx = false;
   for (int64_t t : op->diag_ids) cx = cx || op->aim[t] != 0.0;
   const uint64_t bytes = (uint64_t)D * 8ull * (cx ? 2ull : 1ull);
@@ -1204,8 +1217,14 @@ bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const v
   // x: 57.8 ms against 67.0 ms through its spread)
   const uint64_t ratio = es == 4 ? kXMapDenseRatio32 : kXMapDenseRatio;
   const bool dense = sp->ensure_xtop() <= ratio * (uint64_t)sp->dim && (uint64_t)sp->dim * es > kXMapCachedBytes;
+  // the products on the shapes of window.hpp read x only through the spread and
+  // take it wherever it is dense: 4x8 J1-J2, FP64 (x 150 MB, spread 0.6 GB) 4.14
+  // ms against 8.16 ms through the rank index and the general kernel; 5x6, C128,
+  // 1.31 against 2.26 ms
+  const bool shape = scaled && d.g.win_tab && op->keeps_popcount && sp->ensure_xtop() <= ratio * (uint64_t)sp->dim &&
+                     sp->xcolex_on;
   const bool want = idx_lookup == 4 ||
-                    (idx_lookup == 0 && (rank_mode || sp->ensure_xtop() * es <= kXMapCachedBytes || dense));
+                    (idx_lookup == 0 && (rank_mode || shape || sp->ensure_xtop() * es <= kXMapCachedBytes || dense));
   if (!want || !codes_lds) return false;
   const edhip_space::XMapHost* X = sp->ensure_xmap(es);
   if (!X) return false;
@@ -1383,6 +1402,16 @@ int mv_row_lanes(int64_t dim, int entries) {
   return lg;
 }
 
+// Whether the product runs the kernel of its shape (window.hpp): translations
+// alone, x in its scaled colex spread, images that keep the popcount, the
+// diagonal at hand, and LDS room.
+bool window_product(const edhip_op* op, const OpDev& d) {
+  return d.g.win_tab && d.xm.values && d.xm.scaled && d.xm.colex && d.xm.pop < 0 && d.xm.narrow &&
+         (d.diag_re || op->n_diag == 0) &&
+         win_fixed_bytes(win_kind(d.g.Lx, d.g.Ly), d.g.Lx) + win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <=
+             64 * 1024;
+}
+
 // Term-list kernel over the output rows [row_begin, row_end) (y holds them
 // from y[0]); x is the whole input vector.
 void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, const void* x, void* y,
@@ -1407,7 +1436,17 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   if (attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
   if (idx_lookup == 4 && !d.xm.values) fail(EDHIP_ERR_ARGUMENT, "x cannot be spread over the words of this space");
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
-  HIP_OR_THROW(launch_matvec(d, prec, transpose ? 1 : 0, accumulate ? 1 : 0, x, y, st));
+  if (window_product(op, d)) {
+    const GroupDev& g = d.g;
+    const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.win_tab, g.win_elem, g.ph_re,
+                  g.ph_im,     d.xm.topcode, d.xm.colex, d.xm.values, d.lin_tab, d.ent,      d.rest,
+                  d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
+                  op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, d.xm.top_bits, d.xm.top_shift,
+                  d.xm.hbits};
+    HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
+  } else {
+    HIP_OR_THROW(launch_matvec(d, prec, transpose ? 1 : 0, accumulate ? 1 : 0, x, y, st));
+  }
   if (op->ctx->kernel_timing) {
     HIP_OR_THROW(hipEventRecord(op->ctx->ev[15], st));
     HIP_OR_THROW(hipEventSynchronize(op->ctx->ev[15]));

@@ -293,6 +293,10 @@ struct GroupDev {
   const double* ph_im;
   const double* invsqrt;   // G+1: 1/sqrt(N)
   const double* sqcnt;     // G+1: sqrt(cnt/G) = 1/sqrt(G/cnt) for a stabiliser of cnt elements
+  // translations alone on a shape of window.hpp (win_tab null: not one): its
+  // table, and per candidate bit the element index of the translation
+  const uint16_t* win_tab;
+  const int32_t* win_elem;
 };
 
 // Pointers to the LDS copies of the group tables (same meaning as GroupDev).
@@ -799,6 +803,16 @@ __device__ __forceinline__ void lds_copy(unsigned char* dst, const void* src, ui
   for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x) d[i] = s[i];
 }
 
+// The same for tables of whole 16-byte units on 16-byte boundaries, one unit
+// per lane and step (not unrolled: the staging must not set the register count
+// of the kernel).
+__device__ __forceinline__ void lds_copy16(unsigned char* dst, const void* src, uint32_t bytes) {
+  const uint4* s = (const uint4*)src;
+  uint4* d = (uint4*)dst;
+#pragma unroll 1
+  for (uint32_t i = threadIdx.x; i < bytes >> 4; i += blockDim.x) d[i] = s[i];
+}
+
 __device__ __forceinline__ GroupLds stage_group(const GroupDev& g, const GroupLdsLayout& lay, unsigned char* lds) {
   GroupLds L;
   lds_copy(lds + lay.off_nib, g.nib, lay.bytes_nib);
@@ -905,33 +919,40 @@ __device__ __forceinline__ uint32_t hash_word(uint64_t s) {
 
 // The input vector spread over word positions (the matvec's lookup): a
 // word's position is its bits below top_shift under the code of its top bits
-// (topcode: the rank of the top value among those of the basis words, 0xffff
-// for none; the codes keep the order).  values[position] holds the element
-// of x of the basis word there, 0 at every other position, so that a
-// canonical image finds its x element with one load and no rank; an image
-// outside the basis adds w * 0.  Refreshed before every product.
-// The spread of x over the word positions.  Plain: position = (code of the
-// word's top bits) << top_shift | (the bits below).  Colex (every word of the
-// space has one popcount, colex != null): the low 12 bits are replaced by
-// their colex rank among the 12-bit words of their popcount (which the
-// higher bits fix), position = ((code << hbits | bits 12..top_shift-1) *
-// 924 + rank: 4.4 times fewer positions, so that more of the lines the
-// images touch are shared (6x6 J1-J2: 4.1 GB instead of 18.3 GB in FP32).
+// (topcode: the rank of the top value among those of the basis words; the
+// codes keep the order; top values of no basis word, and any past the table,
+// have the code after the last, whose positions hold 0).  values[position]
+// holds the element of x of the basis word there, 0 at every other position,
+// so that a canonical image finds its x element with one load and no rank; an
+// image outside the basis adds w * 0.  Refreshed before every product.
+// Plain: position = (code of the word's top bits) << top_shift | (the bits
+// below).  Colex (every word of the space has one popcount, colex != null):
+// the low 12 bits are replaced by their colex rank among the 12-bit words of
+// their popcount (which the higher bits fix), position = ((code << hbits |
+// bits 12..top_shift-1) * 924 + rank: 4.4 times fewer positions, so that more
+// of the lines the images touch are shared (6x6 J1-J2: 4.1 GB instead of 18.3
+// GB in FP32).
 struct XMapDev {
   void* values;             // null: not used
-  const uint16_t* topcode;  // 2^top_bits codes (global memory; the kernels copy it to LDS)
+  const uint16_t* topcode;  // 2^top_bits + 1 codes (global memory; the kernels copy them to LDS)
   const uint16_t* colex;    // colex rank of every 12-bit word, u16[4096] (global; copied to LDS after the codes), or null
-  int bm_bits;              // words must be below 2^bm_bits
+  int bm_bits;              // basis words lie below 2^bm_bits
   int top_bits, top_shift;
   int hbits;                // colex: top_shift - 12
   int pop;                  // colex: the popcount of every word (a word of another popcount has no position);
                             // -1 where every image keeps the popcount (no test needed)
   int scaled;               // 1: the spread holds x / sqrt(N) of each representative (orbit size N)
+  int narrow;               // 1: the bits of every word of the space above top_shift fit in 32 bits
 };
 
-// LDS bytes of the code table and, when used, the colex tables after it.
+// LDS bytes of the code table (padded to 16) and, when used, the colex table after it.
+constexpr uint32_t kXCodesBytesMax = (2u << 12) + 16u;
+__host__ __device__ __forceinline__ uint32_t xmap_codes_bytes(int top_bits) { return (2u << top_bits) + 16u; }
 __host__ __device__ __forceinline__ uint32_t xmap_lds_bytes(const XMapDev& X) {
-  return (2u << X.top_bits) + (X.colex ? 2u * 4096u : 0u);
+  return xmap_codes_bytes(X.top_bits) + (X.colex ? 2u * 4096u : 0u);
+}
+__device__ __forceinline__ const uint16_t* xmap_colex_lds(const XMapDev& X, const uint16_t* codes) {
+  return codes + xmap_codes_bytes(X.top_bits) / 2;
 }
 
 // Position of word k whose top bits have code c; cx: the colex rank table
@@ -948,44 +969,35 @@ __device__ __forceinline__ uint64_t xmap_pos(const XMapDev& X, const uint16_t* c
   return ((uint64_t)c << X.top_shift) | (k & ((1ull << X.top_shift) - 1ull));
 }
 
-// x element of one canonical image k (false: the word has no position).
-// codes: the code table in LDS, followed by the colex rank table when used.
-template <typename V>
-__device__ __forceinline__ bool xmap_fetch1(const XMapDev& X, const uint16_t* codes, uint64_t k, V& x) {
+// The table index of the top bits of k (2^top_bits: no position).
+__device__ __forceinline__ uint32_t xmap_top(const XMapDev& X, uint64_t k) {
+  // (colex positions are unique within one popcount only)
   const bool in = (k >> X.bm_bits) == 0 && (!X.colex || X.pop < 0 || __builtin_popcountll(k) == X.pop);
-  const uint32_t c = codes[in ? (uint32_t)(k >> X.top_shift) : 0u];
-  const bool f = in && c != 0xffffu;
-  x = ((const V*)X.values)[f ? xmap_pos(X, codes + (1u << X.top_bits), c, k) : 0ull];
-  return f;
+  return in ? (uint32_t)(k >> X.top_shift) : 1u << X.top_bits;
 }
 
-// x elements of two canonical images k0, k1 (f0, f1: the word has a
-// position), without branches: both code reads are issued, then both loads;
-// an image without a position loads position 0 and is dropped by the caller.
+// x element of one canonical image k, 0 if the word has no position.
+// codes: the code table in LDS, followed by the colex rank table when used.
+template <typename V>
+__device__ __forceinline__ V xmap_fetch1(const XMapDev& X, const uint16_t* codes, uint64_t k) {
+  return ((const V*)X.values)[xmap_pos(X, xmap_colex_lds(X, codes), codes[xmap_top(X, k)], k)];
+}
+
+// x elements of two canonical images: both code reads are issued, then both loads.
 template <typename V>
 __device__ __forceinline__ void xmap_fetch2(const XMapDev& X, const uint16_t* codes, uint64_t k0, uint64_t k1, V& x0,
-                                            V& x1, bool& f0, bool& f1) {
-  // (colex positions are unique within one popcount only)
-  bool in0 = (k0 >> X.bm_bits) == 0, in1 = (k1 >> X.bm_bits) == 0;
-  if (X.colex && X.pop >= 0) {  // the same branch in every lane
-    in0 = in0 && __builtin_popcountll(k0) == X.pop;
-    in1 = in1 && __builtin_popcountll(k1) == X.pop;
-  }
-  const uint32_t c0 = codes[in0 ? (uint32_t)(k0 >> X.top_shift) : 0u];
-  const uint32_t c1 = codes[in1 ? (uint32_t)(k1 >> X.top_shift) : 0u];
-  f0 = in0 && c0 != 0xffffu;
-  f1 = in1 && c1 != 0xffffu;
-  const uint16_t* cx = codes + (1u << X.top_bits);
-  const uint64_t p0 = f0 ? xmap_pos(X, cx, c0, k0) : 0ull;
-  const uint64_t p1 = f1 ? xmap_pos(X, cx, c1, k1) : 0ull;
+                                            V& x1) {
+  const uint32_t c0 = codes[xmap_top(X, k0)], c1 = codes[xmap_top(X, k1)];
+  const uint16_t* cx = xmap_colex_lds(X, codes);
+  const uint64_t p0 = xmap_pos(X, cx, c0, k0), p1 = xmap_pos(X, cx, c1, k1);
   x0 = ((const V*)X.values)[p0];
   x1 = ((const V*)X.values)[p1];
 }
 
-// Stages the code table and the colex tables of X into LDS at codes.
+// Stages the code table and the colex table of X into LDS at codes.
 __device__ __forceinline__ void xmap_stage(const XMapDev& X, uint16_t* codes) {
-  lds_copy((unsigned char*)codes, X.topcode, 2u << X.top_bits);
-  if (X.colex) lds_copy((unsigned char*)(codes + (1u << X.top_bits)), X.colex, 2u * 4096u);
+  lds_copy((unsigned char*)codes, X.topcode, (2u << X.top_bits) + 4u);
+  if (X.colex) lds_copy((unsigned char*)xmap_colex_lds(X, codes), X.colex, 2u * 4096u);
 }
 
 struct HashDev {

@@ -14,7 +14,51 @@
 #include <utility>
 #include <vector>
 
+#include "window.hpp"
+
 namespace edhip {
+
+// Window table of an Lx x Ly torus (window.hpp): entry = rank << mask bits | mask.
+inline std::vector<uint16_t> win_table(int Lx, int Ly) {
+  const int kind = win_kind(Lx, Ly);
+  if (kind == kWinNone) return {};
+  const int nv = 1 << win_index_bits(kind, Lx), mb = win_mask_bits(kind);
+  const int na = kind == kWinChain ? 6 : Lx;
+  const uint32_t rm = (1u << std::min(Lx, 12)) - 1u;
+  auto rot = [&](uint32_t v, int a) { return ((v << a) | (v >> (Lx - a))) & rm; };
+  auto beginning = [&](uint32_t v, int a) -> uint32_t {
+    if (kind == kWinChain) return (v >> (5 - a)) & 127u;
+    if (kind == kWinRows) return rot(v, a);
+    return (rot(v >> Lx, a) << Lx) | rot(v & rm, a);
+  };
+  std::vector<uint32_t> least(nv, ~0u), mask(nv, 0);
+  for (int v = 0; v < nv; ++v)
+    for (int a = 0; a < na; ++a) {
+      const uint32_t x = beginning((uint32_t)v, a);
+      if (x < least[v]) least[v] = x, mask[v] = 0;
+      if (x == least[v]) mask[v] |= 1u << a;
+    }
+  std::vector<uint32_t> order(least);
+  std::sort(order.begin(), order.end());
+  order.erase(std::unique(order.begin(), order.end()), order.end());
+  std::vector<uint16_t> tab(nv);
+  for (int v = 0; v < nv; ++v) {
+    const size_t rank = (size_t)(std::lower_bound(order.begin(), order.end(), least[v]) - order.begin());
+    tab[v] = (uint16_t)(rank << mb | mask[v]);
+  }
+  return tab;
+}
+
+// a + Lx b of the translation of every candidate bit 8 y + a (0 past the last).
+inline std::vector<int> win_positions(int Lx, int Ly) {
+  std::vector<int> pos(64, 0);
+  const bool chain = win_kind(Lx, Ly) == kWinChain;
+  for (int bit = 0; bit < 64; ++bit) {
+    const int y = bit >> 3, a = bit & 7;
+    if (chain ? (a < 6 && 6 * y + a < Lx) : (a < Lx && y < Ly)) pos[bit] = chain ? 6 * y + a : a + Lx * (Ly - 1 - y);
+  }
+  return pos;
+}
 
 // Off-diagonal term as the products see it: the row b matches iff
 // (b & mask) == match; its image is (b & ~mask) | image.

@@ -139,6 +139,39 @@ struct OpDev {
   uint32_t mv_lds_total; // without xm's code table
 };
 
+// The products on the shapes of window.hpp (translations alone): what their
+// kernels read.
+struct WinOp {
+  const uint64_t* rows;
+  const uint16_t* orbit;
+  const double* diag_re;  // null: no diagonal terms
+  const double* diag_im;
+  const uint16_t* win_tab;
+  const int32_t* win_elem;
+  const double* ph_re;
+  const double* ph_im;
+  const uint16_t* topcode;
+  const uint16_t* colex;
+  const void* values;     // the spread x / sqrt(N)
+  const uint64_t* lin_tab;
+  const MvEntry* ent;
+  const OffTerm* rest;
+  uint64_t stripe;
+  int64_t dim, row_begin;
+  int n_bits, n_lin, n_chunk, n_rest, real_amp;
+  int row_lanes, xcd_chunk, accumulate;
+  int top_bits, top_shift, hbits;
+};
+// LDS bytes of the entries (at most: 16 per entry, 8 for Im(amplitude), 16 for mask and match)
+inline uint32_t win_entries_bytes(int n_lin, int n_chunk, int n_rest) {
+  return (uint32_t)(((n_lin + 63) / 64) * n_chunk) * 128u + (uint32_t)(n_lin + n_rest + 1) * 24u +
+         (uint32_t)n_rest * 16u;
+}
+// LDS bytes below the entries (WinLds, at most)
+inline uint32_t win_fixed_bytes(int kind, int Lx) {
+  return (2u << win_index_bits(kind, Lx)) + 64u * 16u + kXCodesBytesMax + 2u * 4096u;
+}
+
 enum Prec : int { kF64 = 0, kC128 = 1, kF32 = 2, kC64 = 3 };
 
 // y = (accumulate ? y : 0) + A x   (transpose=0: row form; 1: column form, y = x A)
@@ -150,6 +183,18 @@ hipError_t launch_product_f32(const OpDev& op, int transpose, int accumulate, co
 hipError_t launch_product_f64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
 hipError_t launch_product_c64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
 hipError_t launch_product_c128(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
+
+// The same on a shape of window.hpp, x spread (P.values).
+hipError_t launch_window_product(const WinOp& P, int Lx, int Ly, int unit, int prec, int transpose, const void* x,
+                                 void* y, hipStream_t st);
+hipError_t launch_window_product_f32(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                                    hipStream_t st);
+hipError_t launch_window_product_f64(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                                    hipStream_t st);
+hipError_t launch_window_product_c64(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                                    hipStream_t st);
+hipError_t launch_window_product_c128(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                                    hipStream_t st);
 
 // ---- assembled rows (row form): entries col | cls << col_bits per image ----
 constexpr int kAsmMaxClasses = 256;

@@ -290,8 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_term_expect(OpDev op, const V* __res
           Canon<MODE>::run(op.g, L, img, s, h, cnt);
           double sr, si;
           if (op.xm.values) {
-            V xv;
-            if (!xmap_fetch1(op.xm, codes, s, xv)) continue;
+            const V xv = xmap_fetch1<V>(op.xm, codes, s);
             load_c(&xv, 0, sr, si);
           } else {
             const int64_t idx = index_of(op.ix, W, s);
@@ -368,8 +367,8 @@ __global__ __launch_bounds__(kBlock) void k_term_expect_lock(OpDev op, const V* 
         if ((b & mask) == match) {
           const uint64_t s = (b & ~mask) | op.off[j].image;
           if (op.xm.values) {
-            V xv;
-            if (xmap_fetch1(op.xm, codes, s, xv)) load_c(&xv, 0, sr[q], si[q]);
+            const V xv = xmap_fetch1<V>(op.xm, codes, s);
+            load_c(&xv, 0, sr[q], si[q]);
           } else {
             const int64_t idx = index_of(op.ix, W, s);
             if (idx >= 0) load_c(psi, idx, sr[q], si[q]);
@@ -864,6 +863,23 @@ hipError_t launch_matvec(const OpDev& op, int prec, int transpose, int accumulat
       return launch_product_f32(op, transpose, accumulate, x, y, st);
     case kC64:
       return launch_product_c64(op, transpose, accumulate, x, y, st);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_window_product(const WinOp& P, int Lx, int Ly, int unit, int prec, int transpose, const void* x,
+                                 void* y, hipStream_t st) {
+  if (P.dim <= P.row_begin) return hipSuccess;
+  switch (prec) {
+    case kF64:
+      return launch_window_product_f64(P, Lx, Ly, unit, transpose, x, y, st);
+    case kC128:
+      return launch_window_product_c128(P, Lx, Ly, unit, transpose, x, y, st);
+    case kF32:
+      return launch_window_product_f32(P, Lx, Ly, unit, transpose, x, y, st);
+    case kC64:
+      return launch_window_product_c64(P, Lx, Ly, unit, transpose, x, y, st);
     default:
       return hipErrorInvalidValue;
   }

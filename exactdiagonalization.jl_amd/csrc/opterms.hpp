@@ -162,12 +162,14 @@ __device__ __forceinline__ uint64_t mv_match(const OpDev& op, const MvTerms& T, 
   base = op.n_lin + s0;
   const int n = op.n_rest - s0 < 64 ? op.n_rest - s0 : 64;
   if (op.rest_paired) {  // two terms with one mask per test (n is even)
+#pragma unroll 2
     for (int j = 0; j < n; j += 2) {
       const uint64_t* m = T.mm + 3 * ((s0 + j) >> 1);
       const uint64_t xm = b & m[0];
       bits |= (uint64_t)((uint32_t)(xm == m[1]) | ((uint32_t)(xm == m[2]) << 1)) << j;
     }
   } else {
+#pragma unroll 2
     for (int j = 0; j < n; ++j) {
       const uint64_t* m = T.mm + 2 * (s0 + j);
       bits |= (uint64_t)((b & m[0]) == m[1]) << j;

@@ -95,10 +95,9 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
       int64_t ik[NW];
       V xv[NW];
       if (op.xm.values) {  // x of each image with one load at its word position
-        bool f0, f1;
-        xmap_fetch2(op.xm, codes, sk[0], sk[1], xv[0], xv[1], f0, f1);
-        ik[0] = f0 ? 0 : -1;
-        ik[1] = (ok[1] && f1) ? 0 : -1;
+        xmap_fetch2(op.xm, codes, sk[0], sk[1], xv[0], xv[1]);
+        ik[0] = 0;
+        ik[1] = ok[1] ? 0 : -1;
       } else {
         index_of2(op.ix, W, sk[0], sk[1], ik[0], ik[1]);
 #pragma unroll
@@ -144,6 +143,210 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
   *yr = accumulate ? vadd(*yr, out) : out;
 }
 
+// ---- translations alone on a shape of window.hpp ------------------------------
+// Everything the kernel reads per image lies at LDS offsets known at compile
+// time: the window table, the phases by candidate bit, the code table of the
+// spread, the colex ranks, then the entries.
+template <int KIND, int LX, int LY, bool UNIT>
+struct WinLds {
+  using S = Win<KIND, LX, LY>;
+  static constexpr uint32_t tab = 0;
+  static constexpr uint32_t phase = tab + S::kTab * 2;
+  static constexpr uint32_t codes = phase + (UNIT ? 0 : 64 * 16);
+  static constexpr uint32_t colex = codes + kXCodesBytesMax;
+  static constexpr uint32_t entries = colex + 2 * 4096;
+};
+
+// One product entry in LDS, in 8 bytes where flip and amplitude fit (32-bit
+// words, FP32 weights), else in 16.
+template <typename W, typename A>
+struct WinEntry {
+  W flip;
+  A amp;
+};
+
+// The product for translation groups on the shapes of window.hpp, x read from
+// its colex spread x / sqrt(N) (XMapDev: every image keeps the popcount, narrow).
+// It is bound by instruction issue and by the line fills of the x gathers
+// together, so what counts is the number of instructions per image: the shape,
+// the word width (32 bits up to 32 sites) and the LDS offsets are fixed at
+// compile time, the canonical form comes from 16-bit window entries (two per
+// register), a position needs no test (XMapDev), and the phase is read by
+// candidate bit.
+template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS>
+__global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __restrict__ x, V* __restrict__ y) {
+  using S = Win<KIND, LX, LY>;
+  using W = typename S::W;
+  using R = typename VT<V>::R;
+  using Lay = WinLds<KIND, LX, LY, UNIT>;
+  constexpr bool CX = VT<V>::cx;
+  // FP32 vectors without a complex phase weigh in FP32, from FP32 amplitudes and phases of +-1
+  constexpr bool kW32 = std::is_same<R, float>::value && (!CX || UNIT);
+  using A = typename std::conditional<kW32, float, double>::type;
+  using E = WinEntry<W, A>;
+  extern __shared__ unsigned char lds[];
+  lds_copy16(lds + Lay::tab, P.win_tab, S::kTab * 2);
+  if constexpr (!UNIT) {
+    double* ph = (double*)(lds + Lay::phase);
+    if (threadIdx.x < 64) {
+      const int h = P.win_elem[threadIdx.x];
+      ph[2 * threadIdx.x] = P.ph_re[h];
+      ph[2 * threadIdx.x + 1] = TRANS ? -P.ph_im[h] : P.ph_im[h];
+    }
+  }
+  lds_copy16(lds + Lay::codes, P.topcode, xmap_codes_bytes(P.top_bits));
+  lds_copy16(lds + Lay::colex, P.colex, 2u * 4096u);
+  constexpr int n_chunk = S::kChain ? 0 : (((S::NB + 3) / 4 + 2) / 3) * 3;
+  const int nch = n_chunk ? n_chunk : P.n_chunk;
+  const uint32_t tab_bytes = (uint32_t)(((P.n_lin + 63) / 64) * nch) * 128u;
+  unsigned char* ptab = lds + Lay::entries;
+  lds_copy16(ptab, P.lin_tab, tab_bytes);
+  E* ent = (E*)(ptab + tab_bytes);
+  const int n_ent = P.n_lin + P.n_rest;
+  double* aim = (double*)(ent + ((n_ent + 1) & ~1));
+  uint64_t* mm = (uint64_t*)(aim + (CX ? n_ent : 0));
+#pragma unroll 1
+  for (int t = threadIdx.x; t < n_ent; t += kMvBlock) {
+    const MvEntry e = P.ent[t];
+    ent[t] = E{(W)e.flip, (A)e.are};
+    if (CX) aim[t] = e.aim;
+  }
+#pragma unroll 1
+  for (int t = threadIdx.x; t < P.n_rest; t += kMvBlock) {
+    mm[2 * t] = P.rest[t].mask;
+    mm[2 * t + 1] = P.rest[t].match;
+  }
+  __syncthreads();
+  const int64_t lane = xcd_chunked_block(blockIdx.x, gridDim.x, P.xcd_chunk) * kMvBlock + threadIdx.x;
+  const int64_t row = P.row_begin + (lane >> P.row_lanes);
+  if (row >= P.dim) return;
+  const int sub = (int)threadIdx.x & ((1 << P.row_lanes) - 1);
+  const W b = (W)P.rows[row];
+
+  const uint16_t* tab = (const uint16_t*)(lds + Lay::tab);
+  const uint16_t* codes = (const uint16_t*)(lds + Lay::codes);
+  const uint16_t* colex = (const uint16_t*)(lds + Lay::colex);
+  const double2* phase = (const double2*)(lds + Lay::phase);
+  const uint32_t top_max = 1u << P.top_bits;
+  auto fetch = [&](W s) {  // x / sqrt(N) of the canonical word s
+    const uint32_t top = (uint32_t)(s >> P.top_shift);
+    const uint32_t c = codes[top < top_max ? top : top_max];
+    const uint32_t lo = (uint32_t)s;
+    const uint32_t hc = (c << P.hbits) | __builtin_amdgcn_ubfe(lo, 12u, (uint32_t)P.hbits);
+    return ((const V*)P.values)[(uint64_t)(__umul24(hc, 924u) + (uint32_t)colex[lo & 0xfffu])];
+  };
+  V acc = vzero<V>();
+  auto add = [&](const V& xv, int t, const E& e, int bit) {
+    if constexpr (UNIT) {
+      if (!CX || P.real_amp) {
+        if constexpr (CX) {
+          acc.re += (R)e.amp * xv.re;
+          acc.im += (R)e.amp * xv.im;
+        } else {
+          acc += (R)e.amp * xv;
+        }
+      } else {
+        vfma(acc, (R)e.amp, (R)aim[t], xv);
+      }
+    } else if constexpr (!CX) {
+      if constexpr (kW32)
+        acc += e.amp * (float)phase[bit].x * xv;
+      else
+        acc += (R)(e.amp * phase[bit].x) * xv;
+    } else {
+      const double2 p = phase[bit];
+      if (P.real_amp) {
+        vfma(acc, (R)(e.amp * p.x), (R)(e.amp * p.y), xv);
+      } else {
+        const double ai = aim[t];
+        vfma(acc, (R)(e.amp * p.x - ai * p.y), (R)(e.amp * p.y + ai * p.x), xv);
+      }
+    }
+  };
+  const int n_ls = (P.n_lin + 63) / 64, n_seg = n_ls + (P.n_rest + 63) / 64;
+  for (int seg = 0; seg < n_seg; ++seg) {
+    uint64_t bits = 0;
+    int base;
+    if (seg < n_ls) {  // parity entries (mv_match)
+      base = 64 * seg;
+      const uint64_t* pt = (const uint64_t*)ptab + seg * (nch << 4);
+      if constexpr (n_chunk > 0) {
+#pragma unroll
+        for (int k = 0; k < n_chunk; ++k)
+          if (4 * k < S::NB) bits ^= pt[(k << 4) + (int)((b >> (4 * k)) & 15)];
+      } else {
+        for (int k = 0; k < nch; k += 3) {
+          uint64_t v[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) v[q] = pt[((k + q) << 4) + (int)(((uint64_t)b >> (4 * (k + q))) & 15)];
+          bits ^= v[0] ^ v[1] ^ v[2];
+        }
+      }
+    } else {
+      const int s0 = (seg - n_ls) * 64;
+      base = P.n_lin + s0;
+      const int n = P.n_rest - s0 < 64 ? P.n_rest - s0 : 64;
+#pragma unroll 2
+      for (int j = 0; j < n; ++j) bits |= (uint64_t)(((uint64_t)b & mm[2 * (s0 + j)]) == mm[2 * (s0 + j) + 1]) << j;
+    }
+    bits &= P.stripe << sub;
+    // two images per step, as in k_matvec
+    while (bits) {
+      const int t0 = base + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      const bool two = bits != 0;
+      const int t1 = two ? base + __builtin_ctzll(bits) : t0;
+      bits &= two ? bits - 1 : bits;
+      const E e0 = ent[t0], e1 = ent[t1];
+      W s0, s1;
+      int w0, w1;
+      S::canonical(tab, b ^ e0.flip, P.n_bits, s0, w0);
+      S::canonical(tab, b ^ e1.flip, P.n_bits, s1, w1);
+      const V x0 = fetch(s0), x1 = fetch(s1);
+      add(x0, t0, e0, w0);
+      if (two) add(x1, t1, e1, w1);
+    }
+  }
+  acc = row_lanes_sum(acc, P.row_lanes);
+  if (sub != 0) return;
+  V out = vzero<V>();
+  if (P.diag_re) vfma(out, (R)P.diag_re[row], (R)(P.diag_im ? P.diag_im[row] : 0.0), x[row]);
+  vfma(out, (R)sqrt((double)P.orbit[row]), (R)0, acc);
+  V* yr = y + (row - P.row_begin);
+  *yr = P.accumulate ? vadd(*yr, out) : out;
+}
+
+template <typename V, int KIND, int LX, int LY>
+hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, void* y, hipStream_t st) {
+  const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
+  const dim3 grid((unsigned)((lanes + kMvBlock - 1) / kMvBlock));
+  const uint32_t dyn = win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest);
+  // the column form only conjugates the phase
+  constexpr bool kT = VT<V>::cx;
+  if (unit)
+    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, true, false>), grid, dim3(kMvBlock),
+                       (WinLds<KIND, LX, LY, true>::entries + dyn), st, P, (const V*)x, (V*)y);
+  else if (transpose)
+    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, false, kT>), grid, dim3(kMvBlock),
+                       (WinLds<KIND, LX, LY, false>::entries + dyn), st, P, (const V*)x, (V*)y);
+  else
+    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, false, false>), grid, dim3(kMvBlock),
+                       (WinLds<KIND, LX, LY, false>::entries + dyn), st, P, (const V*)x, (V*)y);
+  return hipGetLastError();
+}
+
+template <typename V>
+hipError_t launch_win_v(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                        hipStream_t st) {
+#define EDHIP_X(K, X, Y) \
+  if (Lx == X && Ly == Y) return launch_win_t<V, K, X, Y>(P, unit, transpose, x, y, st);
+  EDHIP_WIN_SHAPES(EDHIP_X)
+#undef EDHIP_X
+  if (Ly == 1 && Lx <= 32) return launch_win_t<V, kWinChain, 32, 1>(P, unit, transpose, x, y, st);
+  if (Ly == 1 && Lx <= 48) return launch_win_t<V, kWinChain, 48, 1>(P, unit, transpose, x, y, st);
+  return hipErrorInvalidValue;
+}
+
 template <typename V, int MODE>
 hipError_t launch_mv_t(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st) {
   const uint64_t lanes = (uint64_t)(op.dim - op.row_begin) << op.row_lanes;
@@ -184,12 +387,6 @@ hipError_t launch_mv_v(const OpDev& op, int transpose, int accumulate, const voi
     default:
       if (op.g.pair_table) {
         const int Lx = op.g.Lx, Ly = op.g.Ly;
-        if (op.g.n_cosets == 1) {
-          if (Lx == 6 && Ly == 6) return launch_mv_t<V, kTransPairs6x6>(op, transpose, accumulate, x, y, st);
-          if (Lx == 4 && Ly == 6) return launch_mv_t<V, kTransPairs4x6>(op, transpose, accumulate, x, y, st);
-          if (Lx == 6 && Ly == 4) return launch_mv_t<V, kTransPairs6x4>(op, transpose, accumulate, x, y, st);
-          if (Lx == 4 && Ly == 4) return launch_mv_t<V, kTransPairs4x4>(op, transpose, accumulate, x, y, st);
-        }
         if (Lx == 6 && Ly == 6) return launch_mv_t<V, kTorusPairs6x6>(op, transpose, accumulate, x, y, st);
         if (Lx == 4 && Ly == 6) return launch_mv_t<V, kTorusPairs4x6>(op, transpose, accumulate, x, y, st);
         if (Lx == 6 && Ly == 4) return launch_mv_t<V, kTorusPairs6x4>(op, transpose, accumulate, x, y, st);
