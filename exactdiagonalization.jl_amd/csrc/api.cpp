@@ -335,6 +335,21 @@ struct edhip_space {
   mutable DevBuf xcolex;  // colex rank of every 12-bit word (single-popcount spaces)
   mutable bool xcolex_on = false;
 
+  // Rank tables of a sector of one popcount and at most kRankBits bits (RankTables)
+  mutable DevBuf rank_low, rank_base;
+  mutable int rank_low_bits = 0;
+  bool ensure_rank_tables() const {
+    if (group || !is_sector || popcounts.size() != 1 || n_bits > kRankBits) return false;
+    if (!rank_low_bits) {
+      const RankTables T = rank_tables(n_bits, popcounts[0]);
+      upload(rank_low, T.low, ctx->stream);
+      upload(rank_base, T.base, ctx->stream);
+      ctx->sync();
+      rank_low_bits = T.low_bits;
+    }
+    return true;
+  }
+
   // The popcount every word of the space has, or -1: a popcount sector with
   // one allowed popcount, or a reduction of one.
   int single_popcount() const {
@@ -1402,14 +1417,25 @@ int mv_row_lanes(int64_t dim, int entries) {
   return lg;
 }
 
-// Whether the product runs the kernel of its shape (window.hpp): translations
-// alone, x in its scaled colex spread, images that keep the popcount, the
-// diagonal at hand, and LDS room.
+// Whether the product runs the kernel of its shape (window.hpp; translations
+// alone, or no group): x in its colex spread, images that keep the popcount,
+// the diagonal at hand, and LDS room.
 bool window_product(const edhip_op* op, const OpDev& d) {
-  return d.g.win_tab && d.xm.values && d.xm.scaled && d.xm.colex && d.xm.pop < 0 && d.xm.narrow &&
+  const bool none = d.g.mode == kGroupNone;
+  return (none || (d.g.win_tab && d.xm.scaled)) && d.xm.values && d.xm.colex && d.xm.pop < 0 && d.xm.narrow &&
          (d.diag_re || op->n_diag == 0) &&
-         win_fixed_bytes(win_kind(d.g.Lx, d.g.Ly), d.g.Lx) + win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <=
-             64 * 1024;
+         (none ? win_fixed_bytes(kWinRows, 1) : win_fixed_bytes(win_kind(d.g.Lx, d.g.Ly), d.g.Lx)) +
+                 win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <= 64 * 1024;
+}
+
+// Whether it runs by rank: a sector of one popcount without a group, up to
+// kRankBits bits (the figures stand at k_product_win).
+bool rank_product(const edhip_op* op, const OpDev& d) {
+  const edhip_space* sp = op->space;
+  return d.g.mode == kGroupNone && op->keeps_popcount && (d.diag_re || op->n_diag == 0) && d.n_lin + d.n_rest > 0 &&
+         sp->ensure_rank_tables() &&
+         (2u << sp->rank_low_bits) + (uint32_t)sp->rank_base.bytes +
+                 win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <= 64 * 1024;
 }
 
 // Term-list kernel over the output rows [row_begin, row_end) (y holds them
@@ -1433,17 +1459,21 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   }
   op->used_kernel = 1;
   op->used_lookup = rank_mode ? 1 : (d.ix.bm_bits ? 3 : 1);
-  if (attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
+  const bool ranked = idx_lookup <= 1 && rank_product(op, d);
+  if (!ranked && attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
   if (idx_lookup == 4 && !d.xm.values) fail(EDHIP_ERR_ARGUMENT, "x cannot be spread over the words of this space");
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
-  if (window_product(op, d)) {
+  if (ranked || window_product(op, d)) {
     const GroupDev& g = d.g;
     const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.win_tab, g.win_elem, g.ph_re,
                   g.ph_im,     d.xm.topcode, d.xm.colex, d.xm.values, d.lin_tab, d.ent,      d.rest,
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, d.xm.top_bits, d.xm.top_shift,
-                  d.xm.hbits};
-    HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
+                  d.xm.hbits,  ranked ? sp->rank_low.as<uint16_t>() : nullptr, sp->rank_base.as<uint32_t>(),
+                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes};
+    const bool none = g.mode == kGroupNone;
+    HIP_OR_THROW(launch_window_product(P, none ? 0 : g.Lx, none ? 0 : g.Ly, none ? 1 : g.unit_phases, prec,
+                                       transpose ? 1 : 0, x, y, st));
   } else {
     HIP_OR_THROW(launch_matvec(d, prec, transpose ? 1 : 0, accumulate ? 1 : 0, x, y, st));
   }

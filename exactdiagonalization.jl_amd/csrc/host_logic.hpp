@@ -18,6 +18,33 @@
 
 namespace edhip {
 
+// Rank tables of the n-bit words of popcount pop: rank(w) = base[w >> low_bits]
+// + low[w & mask], low the rank of a low_bits-bit word among those of its
+// popcount, base the number of words whose upper part is smaller.  base is
+// padded to whole 16 bytes.
+struct RankTables {
+  int low_bits = 0;
+  std::vector<uint16_t> low;
+  std::vector<uint32_t> base;
+};
+inline RankTables rank_tables(int n, int pop) {
+  RankTables T;
+  T.low_bits = n <= 24 ? 12 : 13;
+  T.low.resize((size_t)1 << T.low_bits);
+  std::vector<uint32_t> of_pop((size_t)T.low_bits + 1, 0);
+  for (size_t w = 0; w < T.low.size(); ++w) T.low[w] = (uint16_t)of_pop[(size_t)__builtin_popcountll(w)]++;
+  const int hi = std::max(0, n - T.low_bits);
+  uint32_t sum = 0;
+  for (size_t w = 0; w < ((size_t)1 << hi); ++w) {
+    T.base.push_back(sum);
+    const int need = pop - __builtin_popcountll(w);
+    // (a lower part wider than the word has its upper bits clear)
+    if (need >= 0 && need <= T.low_bits && n >= T.low_bits) sum += of_pop[(size_t)need];
+  }
+  while (T.base.size() % 4) T.base.push_back(sum);
+  return T;
+}
+
 // Window table of an Lx x Ly torus (window.hpp): entry = rank << mask bits | mask.
 inline std::vector<uint16_t> win_table(int Lx, int Ly) {
   const int kind = win_kind(Lx, Ly);

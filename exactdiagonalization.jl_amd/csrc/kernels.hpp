@@ -161,7 +161,14 @@ struct WinOp {
   int n_bits, n_lin, n_chunk, n_rest, real_amp;
   int row_lanes, xcd_chunk, accumulate;
   int top_bits, top_shift, hbits;
+  // sectors without a group, by rank (rank_low null: through the spread)
+  const uint16_t* rank_low;   // colex rank of every low_bits-bit word among those of its popcount
+  const uint32_t* rank_base;  // number of sector words with a smaller upper part
+  int low_bits;
+  uint32_t base_bytes;        // of rank_base, a multiple of 16
 };
+// Sectors of up to this many bits are ranked by two LDS tables (13 + 13 bits: 48 KiB)
+constexpr int kRankBits = 26;
 // LDS bytes of the entries (at most: 16 per entry, 8 for Im(amplitude), 16 for mask and match)
 inline uint32_t win_entries_bytes(int n_lin, int n_chunk, int n_rest) {
   return (uint32_t)(((n_lin + 63) / 64) * n_chunk) * 128u + (uint32_t)(n_lin + n_rest + 1) * 24u +
@@ -184,7 +191,8 @@ hipError_t launch_product_f64(const OpDev& op, int transpose, int accumulate, co
 hipError_t launch_product_c64(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
 hipError_t launch_product_c128(const OpDev& op, int transpose, int accumulate, const void* x, void* y, hipStream_t st);
 
-// The same on a shape of window.hpp, x spread (P.values).
+// The same on a shape of window.hpp, x spread (P.values); Ly = 0: no group, x
+// spread or ranked.
 hipError_t launch_window_product(const WinOp& P, int Lx, int Ly, int unit, int prec, int transpose, const void* x,
                                  void* y, hipStream_t st);
 hipError_t launch_window_product_f32(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,

@@ -143,10 +143,11 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
   *yr = accumulate ? vadd(*yr, out) : out;
 }
 
-// ---- translations alone on a shape of window.hpp ------------------------------
+// ---- translations alone on a shape of window.hpp, and sectors without a group ----
 // Everything the kernel reads per image lies at LDS offsets known at compile
 // time: the window table, the phases by candidate bit, the code table of the
-// spread, the colex ranks, then the entries.
+// spread, the colex ranks, then the entries (by rank: the two rank tables, then
+// the entries).
 template <int KIND, int LX, int LY, bool UNIT>
 struct WinLds {
   using S = Win<KIND, LX, LY>;
@@ -173,7 +174,14 @@ struct WinEntry {
 // compile time, the canonical form comes from 16-bit window entries (two per
 // register), a position needs no test (XMapDev), and the phase is read by
 // candidate bit.
-template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS>
+//
+// KIND = kWinNone: sectors of one popcount without a group.  RANK: of at most
+// kRankBits bits, x is read itself, at the word's rank: the number of sector
+// words with a smaller upper part plus the colex rank of the lower part, one
+// read of each of two LDS tables (no spread to fill, and x is denser: 4x6 XXZ,
+// 2.7e6 states, FP64: 174 us a call through the spread by the general kernel,
+// 118 us by rank).
+template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS, bool RANK = false>
 __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __restrict__ x, V* __restrict__ y) {
   using S = Win<KIND, LX, LY>;
   using W = typename S::W;
@@ -194,12 +202,18 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
       ph[2 * threadIdx.x + 1] = TRANS ? -P.ph_im[h] : P.ph_im[h];
     }
   }
-  lds_copy16(lds + Lay::codes, P.topcode, xmap_codes_bytes(P.top_bits));
-  lds_copy16(lds + Lay::colex, P.colex, 2u * 4096u);
+  const uint32_t rank_low = 2u << P.low_bits;  // RANK: bytes of the lower table
+  if constexpr (RANK) {
+    lds_copy16(lds, P.rank_low, rank_low);
+    lds_copy16(lds + rank_low, P.rank_base, P.base_bytes);
+  } else {
+    lds_copy16(lds + Lay::codes, P.topcode, xmap_codes_bytes(P.top_bits));
+    lds_copy16(lds + Lay::colex, P.colex, 2u * 4096u);
+  }
   constexpr int n_chunk = S::kChain ? 0 : (((S::NB + 3) / 4 + 2) / 3) * 3;
   const int nch = n_chunk ? n_chunk : P.n_chunk;
   const uint32_t tab_bytes = (uint32_t)(((P.n_lin + 63) / 64) * nch) * 128u;
-  unsigned char* ptab = lds + Lay::entries;
+  unsigned char* ptab = lds + (RANK ? rank_low + P.base_bytes : Lay::entries);
   lds_copy16(ptab, P.lin_tab, tab_bytes);
   E* ent = (E*)(ptab + tab_bytes);
   const int n_ent = P.n_lin + P.n_rest;
@@ -228,7 +242,11 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   const uint16_t* colex = (const uint16_t*)(lds + Lay::colex);
   const double2* phase = (const double2*)(lds + Lay::phase);
   const uint32_t top_max = 1u << P.top_bits;
-  auto fetch = [&](W s) {  // x / sqrt(N) of the canonical word s
+  auto fetch = [&](W s) {  // x (/ sqrt(N)) of the canonical word s
+    if constexpr (RANK) {
+      const uint32_t lo = (uint32_t)s & ((1u << P.low_bits) - 1u);
+      return x[((const uint32_t*)(lds + rank_low))[s >> P.low_bits] + (uint32_t)((const uint16_t*)lds)[lo]];
+    }
     const uint32_t top = (uint32_t)(s >> P.top_shift);
     const uint32_t c = codes[top < top_max ? top : top_max];
     const uint32_t lo = (uint32_t)s;
@@ -290,28 +308,45 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
       for (int j = 0; j < n; ++j) bits |= (uint64_t)(((uint64_t)b & mm[2 * (s0 + j)]) == mm[2 * (s0 + j) + 1]) << j;
     }
     bits &= P.stripe << sub;
-    // two images per step, as in k_matvec
+    // two images per step, as in k_matvec (three: 6x6 61.2 against 59.8 ms;
+    // sectors without a group, six: 108 against 114 us on the 4x6 XXZ case)
+    constexpr int NW = 2;
     while (bits) {
-      const int t0 = base + __builtin_ctzll(bits);
+      int t[NW];
+      bool ok[NW];
+      t[0] = base + __builtin_ctzll(bits);
       bits &= bits - 1;
-      const bool two = bits != 0;
-      const int t1 = two ? base + __builtin_ctzll(bits) : t0;
-      bits &= two ? bits - 1 : bits;
-      const E e0 = ent[t0], e1 = ent[t1];
-      W s0, s1;
-      int w0, w1;
-      S::canonical(tab, b ^ e0.flip, P.n_bits, s0, w0);
-      S::canonical(tab, b ^ e1.flip, P.n_bits, s1, w1);
-      const V x0 = fetch(s0), x1 = fetch(s1);
-      add(x0, t0, e0, w0);
-      if (two) add(x1, t1, e1, w1);
+#pragma unroll
+      for (int k = 1; k < NW; ++k) {
+        ok[k] = bits != 0;
+        t[k] = ok[k] ? base + __builtin_ctzll(bits) : t[0];
+        bits &= ok[k] ? bits - 1 : bits;
+      }
+      E e[NW];
+      W s[NW];
+      int w[NW];
+      V xv[NW];
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+        e[k] = ent[t[k]];
+        S::canonical(tab, b ^ e[k].flip, P.n_bits, s[k], w[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < NW; ++k) xv[k] = fetch(s[k]);
+      add(xv[0], t[0], e[0], w[0]);
+#pragma unroll
+      for (int k = 1; k < NW; ++k)
+        if (ok[k]) add(xv[k], t[k], e[k], w[k]);
     }
   }
   acc = row_lanes_sum(acc, P.row_lanes);
   if (sub != 0) return;
   V out = vzero<V>();
   if (P.diag_re) vfma(out, (R)P.diag_re[row], (R)(P.diag_im ? P.diag_im[row] : 0.0), x[row]);
-  vfma(out, (R)sqrt((double)P.orbit[row]), (R)0, acc);
+  if constexpr (KIND != kWinNone)
+    vfma(out, (R)sqrt((double)P.orbit[row]), (R)0, acc);
+  else
+    out = vadd(out, acc);
   V* yr = y + (row - P.row_begin);
   *yr = P.accumulate ? vadd(*yr, out) : out;
 }
@@ -342,6 +377,22 @@ hipError_t launch_win_v(const WinOp& P, int Lx, int Ly, int unit, int transpose,
   if (Lx == X && Ly == Y) return launch_win_t<V, K, X, Y>(P, unit, transpose, x, y, st);
   EDHIP_WIN_SHAPES(EDHIP_X)
 #undef EDHIP_X
+  if (Ly == 0) {  // no group
+    const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
+    const dim3 grid((unsigned)((lanes + kMvBlock - 1) / kMvBlock));
+    const uint32_t dyn = win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest);
+    constexpr uint32_t fixed = WinLds<kWinNone, 32, 1, true>::entries;
+    if (P.rank_low)
+      hipLaunchKernelGGL((k_product_win<V, kWinNone, 32, 1, true, false, true>), grid, dim3(kMvBlock),
+                         ((2u << P.low_bits) + P.base_bytes + dyn), st, P, (const V*)x, (V*)y);
+    else if (P.n_bits <= 32)
+      hipLaunchKernelGGL((k_product_win<V, kWinNone, 32, 1, true, false>), grid, dim3(kMvBlock), (fixed + dyn), st, P,
+                         (const V*)x, (V*)y);
+    else
+      hipLaunchKernelGGL((k_product_win<V, kWinNone, 64, 1, true, false>), grid, dim3(kMvBlock), (fixed + dyn), st, P,
+                         (const V*)x, (V*)y);
+    return hipGetLastError();
+  }
   if (Ly == 1 && Lx <= 32) return launch_win_t<V, kWinChain, 32, 1>(P, unit, transpose, x, y, st);
   if (Ly == 1 && Lx <= 48) return launch_win_t<V, kWinChain, 48, 1>(P, unit, transpose, x, y, st);
   return hipErrorInvalidValue;

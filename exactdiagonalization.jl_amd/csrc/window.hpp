@@ -200,4 +200,17 @@ struct Win {
   }
 };
 
+// No group: every word is its own image (LX: bits of the widest word).
+template <int LX, int LY>
+struct Win<kWinNone, LX, LY> {
+  static constexpr bool kChain = true;  // (the number of word bits is a run-time value)
+  static constexpr int NB = LX;
+  static constexpr int kTab = 0;
+  using W = typename WinWord<(LX > 32)>::T;
+  EDHIP_HD static void canonical(const uint16_t*, W b, int, W& s, int& bit) {
+    s = b;
+    bit = 0;
+  }
+};
+
 }  // namespace edhip

@@ -1,4 +1,4 @@
-// The products' entries (mv_split, mv_tables of host_logic.hpp) against the
+// The rank tables of a sector against counting, and the products' entries (mv_split, mv_tables of host_logic.hpp) against the
 // terms they stand for: every word matches the same flips with the same
 // amplitudes, counted with multiplicity, as when each term is tested by itself.
 #include <algorithm>
@@ -62,7 +62,24 @@ static int run(std::mt19937_64& rng, int nb, int n_masks) {
   return 0;
 }
 
+// The rank tables against counting, word by word.
+static int ranks(int n, int pop) {
+  const edhip::RankTables T = edhip::rank_tables(n, pop);
+  uint32_t rank = 0;
+  for (uint64_t w = 0; w < (1ull << n); ++w)
+    if (__builtin_popcountll(w) == pop) {
+      const uint32_t got = T.base[w >> T.low_bits] + T.low[w & ((1ull << T.low_bits) - 1)];
+      if (got != rank++) return std::printf("rank of %llx in (%d, %d): %u\n", (unsigned long long)w, n, pop, got), 1;
+    }
+  return T.base.size() % 4 ? 1 : 0;
+}
+
 int main() {
+  for (int n : {1, 3, 11, 12, 13, 14, 20})
+    for (int pop : {0, 1, 2, n / 2, n})
+      if (pop <= n && ranks(n, pop)) return 1;
+  for (int pop : {0, 2, 12, 13, 26})
+    if (ranks(pop == 12 ? 24 : 26, pop == 12 ? 12 : std::min(pop, 26))) return 1;
   std::mt19937_64 rng(7);
   for (int nb : {1, 2, 5, 12, 13, 36, 37, 63, 64})
     for (int n_masks : {0, 1, 3, 63, 64, 65, 130, 300})
