@@ -2481,7 +2481,12 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
     upload(op->off_col, offc, ctx->stream);
     for (int form = 0; form < 2; ++form) {
       const std::vector<OffTerm>& v = form ? offc : offr;
-      const MvSplit S = mv_split(v);
+      // without a group the images are near their rows where the flips are the
+      // same: the lanes of a wave share their upper bits, so the entries that
+      // flip upper bits only go first and are taken by all lanes in the same step
+      // (4x6 XXZ product 114 -> 90 us; on reduced spaces, whose images scatter
+      // anyway, the order of the terms is better: 5x6 1.00 against 1.06 ms)
+      const MvSplit S = mv_split(v, !space->group);
       edhip_op::MvHost& M = op->mv[form];
       M.n_lin = (int)S.lin.size();
       M.n_rest = (int)S.rest.size();

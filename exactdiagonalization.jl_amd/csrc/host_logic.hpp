@@ -115,7 +115,9 @@ struct MvSplit {
 // everywhere (one bit: 0 and 1): S+S- + S-S+ bonds, transverse fields.  The
 // padding terms of rest keep the mask, match nothing (a match outside the
 // mask) and flip nothing.
-inline MvSplit mv_split(const std::vector<OffTerm>& v) {
+// by_low_bit: the parity entries in descending order of the lowest bit they
+// flip, else in the order of the terms.
+inline MvSplit mv_split(const std::vector<OffTerm>& v, bool by_low_bit = false) {
   MvSplit S;
   std::vector<char> used(v.size(), 0);
   for (size_t i = 0; i < v.size();) {
@@ -141,6 +143,19 @@ inline MvSplit mv_split(const std::vector<OffTerm>& v) {
       }
     if (kept & 1) S.rest.push_back(OffTerm{m, ~m, ~m, 0.0, 0.0});
     i = j;
+  }
+  if (by_low_bit) {
+    std::vector<size_t> at(S.lin.size());
+    for (size_t e = 0; e < at.size(); ++e) at[e] = e;
+    std::stable_sort(at.begin(), at.end(), [&](size_t a, size_t b) {
+      return __builtin_ctzll(S.lin[a].flip) > __builtin_ctzll(S.lin[b].flip);
+    });
+    const MvSplit T = S;
+    for (size_t e = 0; e < at.size(); ++e) {
+      S.q[e] = T.q[at[e]];
+      S.c[e] = T.c[at[e]];
+      S.lin[e] = T.lin[at[e]];
+    }
   }
   return S;
 }

@@ -31,7 +31,9 @@ static int run(std::mt19937_64& rng, int nb, int n_masks) {
       v.push_back({m, o.match ^ m, o.image ^ m, o.are, o.aim});
     }
   }
-  const edhip::MvSplit S = edhip::mv_split(v);
+  const edhip::MvSplit S = edhip::mv_split(v, n_masks % 2 == 1);
+  for (size_t e = 1; n_masks % 2 == 1 && e < S.lin.size(); ++e)
+    if (__builtin_ctzll(S.lin[e].flip) > __builtin_ctzll(S.lin[e - 1].flip)) return std::printf("order\n"), 1;
   const std::vector<uint64_t> tab = edhip::mv_tables(S, nb);
   const int nc = edhip::mv_chunks(nb);
   if (nc % 3 || 4 * nc < nb) return std::printf("chunks\n"), 1;
