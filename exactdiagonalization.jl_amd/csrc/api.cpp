@@ -202,7 +202,7 @@ struct GroupHost {
   int n_cosets = 1;  // torus: cosets T p of the translations
   // device tables
   DevBuf nib, minrot, pair, rot_hi, rot_lo, g_of_ab, inv_d, trivial, ph_re, ph_im, invsqrt, sqcnt, xr_d, coset_nib_d,
-      coset_pidx_d, coset_xr_d, coset_kind_d, coset_elem_d, coset_inv_d, win_tab, win_elem;
+      coset_pidx_d, coset_xr_d, coset_kind_d, coset_elem_d, coset_inv_d, win_tab, win_elem, point_tab, point_elem;
   GroupDev dev{};
   GroupLdsLayout lay{};
 };
@@ -437,6 +437,46 @@ struct edhip_space {
       (void)hipGetLastError();  // no room: the products use the rank index
       X.values.release();
       return nullptr;
+    }
+  }
+
+  // Rank blocks over the colex positions of the words (layout as the blocked
+  // rank index, 6 positions per byte): 6x6 A1, 172 MB against 5.7 GB over the
+  // words themselves.
+  mutable DevBuf pos_blocks;
+  mutable bool pos_tried = false;
+  mutable XMapDev pos_dev{};
+  bool ensure_positions() const {
+    if (pos_tried) return pos_blocks.p != nullptr;
+    pos_tried = true;
+    if (dim == 0) return false;
+    const uint64_t n_pos = ensure_xtop();
+    if (!xcolex_on || n_bits - xtop_shift > 32) return false;
+    const uint64_t n_blocks = (n_pos + kRankBlockWords - 1) / kRankBlockWords;
+    if (n_blocks * 64 > std::max<uint64_t>(kBitmapMaxRatio * (uint64_t)dim * 8ull, 1ull << 20)) return false;
+    pos_dev = XMapDev{nullptr, xtop.as<uint16_t>(), xcolex.as<uint16_t>(), xtop_K, xtop_bits, xtop_shift,
+                      xtop_shift - 12, -1, 0, 1};
+    try {
+      DevBuf pos, totals, base, tmp;
+      pos.alloc((size_t)dim * 8);
+      totals.alloc(n_blocks * 4);
+      base.alloc(n_blocks * 8);
+      pos_blocks.alloc(n_blocks * 64);
+      HIP_OR_THROW(hipMemsetAsync(pos_blocks.p, 0, n_blocks * 64, ctx->stream));
+      HIP_OR_THROW(launch_xmap_positions(pos_dev, keys.as<uint64_t>(), dim, pos.as<uint64_t>(), ctx->stream));
+      size_t tb = 0;
+      HIP_OR_THROW(launch_bitmap_build(pos.as<uint64_t>(), dim, pos_blocks.as<uint64_t>(), n_blocks,
+                                       totals.as<uint32_t>(), base.as<uint64_t>(), nullptr, tb, ctx->stream));
+      tmp.alloc(tb);
+      HIP_OR_THROW(launch_bitmap_build(pos.as<uint64_t>(), dim, pos_blocks.as<uint64_t>(), n_blocks,
+                                       totals.as<uint32_t>(), base.as<uint64_t>(), tmp.p, tb, ctx->stream));
+      ctx->sync();
+      return true;
+    } catch (const Error& e) {
+      pos_blocks.release();
+      if (e.code != EDHIP_ERR_MEMORY) throw;
+      (void)hipGetLastError();  // no room: the general kernels
+      return false;
     }
   }
 
@@ -809,6 +849,28 @@ void build_group(GroupHost& gh, int nb, double tol, hipStream_t st) {
       upload(gh.win_elem, elem, st);
       d.win_tab = gh.win_tab.as<uint16_t>();
       d.win_elem = gh.win_elem.as<int32_t>();
+    }
+    if (nc > 1 && bestLx == bestLy && win_point_side(bestLx) && !gh.has_xor) {
+      // the elements among the candidates of Win<kWinPoint>: a set of variants,
+      // alone or with the same set after the transposition
+      std::vector<int32_t> elem(512, -1);
+      int variants[2] = {0, 0}, found = 0;
+      for (int code = 0; code < 512; ++code) {
+        if ((code & 7) >= bestLx || ((code >> 3) & 7) >= bestLx) continue;
+        auto it = index.find(std::make_pair(win_point_perm(bestLx, code), (uint64_t)0));
+        if (it == index.end()) continue;
+        elem[(size_t)code] = it->second;
+        variants[code >> 8] |= 1 << ((code >> 6) & 3);
+        ++found;
+      }
+      if (found == G && (variants[1] == 0 || variants[1] == variants[0])) {
+        for (int32_t& e : elem) e = std::max(e, 0);
+        upload(gh.point_tab, win_point_table(bestLx, variants[0]), st);
+        upload(gh.point_elem, elem, st);
+        d.point_tab = gh.point_tab.as<uint16_t>();
+        d.point_elem = gh.point_elem.as<int32_t>();
+        d.point_swap = variants[1] ? 1 : 0;
+      }
     }
     L.bytes_cnib = (uint32_t)(cnib.size() * 8);
     L.bytes_cxr = (uint32_t)(nc * 8);
@@ -1438,6 +1500,24 @@ bool rank_product(const edhip_op* op, const OpDev& d) {
                  win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <= 64 * 1024;
 }
 
+// Whether it runs the kernel of the torus's point operations, and x / sqrt(N) in
+// the operator's buffer.
+bool point_product(edhip_op* op, const OpDev& d, int prec, const void* x) {
+  const edhip_space* sp = op->space;
+  if (!d.g.point_tab || !d.orbit || !op->keeps_popcount || !(d.diag_re || op->n_diag == 0) ||
+      win_point_bytes(d.g.Lx, d.n_lin, d.n_chunk, d.n_rest) > 64 * 1024 || !sp->ensure_positions())
+    return false;
+  try {
+    op->asm_xt.ensure((size_t)sp->dim * elem_size(prec));
+  } catch (const Error& e) {
+    if (e.code != EDHIP_ERR_MEMORY) throw;
+    (void)hipGetLastError();
+    return false;
+  }
+  HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, x, op->asm_xt.p, op->ctx->stream));
+  return true;
+}
+
 // Term-list kernel over the output rows [row_begin, row_end) (y holds them
 // from y[0]); x is the whole input vector.
 void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, const void* x, void* y,
@@ -1447,7 +1527,6 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   const bool rank_mode = sp->is_sector && !sp->group;
   const int idx_lookup = (op->strat_lookup == 2) ? 0 : op->strat_lookup;  // the hash applies to the pair kernel only
   OpDev d = transpose ? op->dev_col : op->dev_row;
-  d.ix = sp->index_dev(idx_lookup == 4 ? 0 : idx_lookup);
   d.xcd_chunk = g_xcd_chunk.load();
   d.row_begin = row_begin;
   d.dim = row_end;
@@ -1458,19 +1537,31 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
     d.diag_im = op->diag_im.as<double>();
   }
   op->used_kernel = 1;
-  op->used_lookup = rank_mode ? 1 : (d.ix.bm_bits ? 3 : 1);
+  const bool point = idx_lookup == 0 && point_product(op, d, prec, x);
+  if (!point) d.ix = sp->index_dev(idx_lookup == 4 ? 0 : idx_lookup);
+  op->used_lookup = rank_mode ? 1 : (point || d.ix.bm_bits ? 3 : 1);
   const bool ranked = idx_lookup <= 1 && rank_product(op, d);
-  if (!ranked && attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
+  if (!point && !ranked && attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
   if (idx_lookup == 4 && !d.xm.values) fail(EDHIP_ERR_ARGUMENT, "x cannot be spread over the words of this space");
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
-  if (ranked || window_product(op, d)) {
+  if (point) {
+    const GroupDev& g = d.g;
+    const XMapDev& X = sp->pos_dev;
+    const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.point_tab, g.point_elem, g.ph_re,
+                  g.ph_im,     X.topcode, X.colex,     op->asm_xt.p, d.lin_tab, d.ent,      d.rest,
+                  d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
+                  op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, X.top_bits, X.top_shift,
+                  X.hbits,     nullptr,   nullptr,     0,          0,         sp->pos_blocks.as<uint64_t>(),
+                  g.point_swap};
+    HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
+  } else if (ranked || window_product(op, d)) {
     const GroupDev& g = d.g;
     const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.win_tab, g.win_elem, g.ph_re,
                   g.ph_im,     d.xm.topcode, d.xm.colex, d.xm.values, d.lin_tab, d.ent,      d.rest,
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, d.xm.top_bits, d.xm.top_shift,
                   d.xm.hbits,  ranked ? sp->rank_low.as<uint16_t>() : nullptr, sp->rank_base.as<uint32_t>(),
-                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes};
+                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes, nullptr, 0};
     const bool none = g.mode == kGroupNone;
     HIP_OR_THROW(launch_window_product(P, none ? 0 : g.Lx, none ? 0 : g.Ly, none ? 1 : g.unit_phases, prec,
                                        transpose ? 1 : 0, x, y, st));

@@ -174,6 +174,27 @@ __device__ __forceinline__ int64_t bitmap_index(const IndexDev& ix, uint64_t key
   return ((word >> bit) & 1ull) ? r : -1;
 }
 
+// The same for a position below 2^32 in blocks of their own, the loads apart
+// from their use.
+struct RankBlock {
+  uint64_t word;
+  ulonglong2 tail;
+};
+__device__ __forceinline__ RankBlock rank_block(const uint64_t* blocks, uint32_t pos) {
+  const uint32_t j = __umulhi(pos >> 7, 0xAAAAAAABu) >> 1;
+  const uint64_t* blk = blocks + (uint64_t)j * 8u;
+  return RankBlock{blk[(pos - j * kRankBlockWords) >> 6], *(const ulonglong2*)(blk + 6)};
+}
+// Whether pos is a member; i: its rank, 0 if not.
+__device__ __forceinline__ bool rank_in(const RankBlock& r, uint32_t pos, uint64_t& i) {
+  const uint32_t j = __umulhi(pos >> 7, 0xAAAAAAABu) >> 1;
+  const uint32_t w = (pos - j * kRankBlockWords) >> 6, bit = pos & 63u;
+  const uint32_t sub = w ? (uint32_t)(r.tail.y >> (9u * (w - 1u))) & 511u : 0u;
+  const bool in = (r.word >> bit) & 1ull;
+  i = in ? r.tail.x + sub + (uint64_t)__builtin_popcountll(r.word & ((1ull << bit) - 1ull)) : 0ull;
+  return in;
+}
+
 __device__ __forceinline__ int64_t search_sorted(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ prefix,
                                                  uint64_t n_buckets, int shift, uint64_t key) {
   uint64_t bucket = key >> shift;
@@ -297,6 +318,13 @@ struct GroupDev {
   // table, and per candidate bit the element index of the translation
   const uint16_t* win_tab;
   const int32_t* win_elem;
+  // translations and point operations of a square torus (Win<kWinPoint>; null:
+  // not one): tables, the element of every candidate code, and whether the
+  // group transposes
+  const uint16_t* point_tab;
+  const int32_t* point_elem;
+  int point_swap;
+  int pad_pt_;
 };
 
 // Pointers to the LDS copies of the group tables (same meaning as GroupDev).

@@ -87,6 +87,52 @@ inline std::vector<int> win_positions(int Lx, int Ly) {
   return pos;
 }
 
+// Tables of Win<kWinPoint, L, L> for the variants in the mask (bit v), as bytes:
+// ranks, then masks.
+inline std::vector<unsigned char> win_point_table(int L, int variants) {
+  const int nv = 1 << (2 * L);
+  const uint32_t rm = (1u << L) - 1u;
+  auto rot = [&](uint32_t v, int a) { return ((v << a) | (v >> (L - a))) & rm; };
+  auto rev = [&](uint32_t v) {
+    uint32_t o = 0;
+    for (int i = 0; i < L; ++i) o |= ((v >> i) & 1u) << (L - 1 - i);
+    return o;
+  };
+  std::vector<uint32_t> least((size_t)nv, ~0u), mask((size_t)nv, 0);
+  for (int w = 0; w < nv; ++w)
+    for (int v = 0; v < 4; ++v) {
+      if (!((variants >> v) & 1)) continue;
+      uint32_t hi = (uint32_t)w >> L, lo = (uint32_t)w & rm;
+      if (v & 2) std::swap(hi, lo);
+      if (v & 1) hi = rev(hi), lo = rev(lo);
+      for (int a = 0; a < L; ++a) {
+        const uint32_t x = (rot(hi, a) << L) | rot(lo, a);
+        if (x < least[(size_t)w]) least[(size_t)w] = x, mask[(size_t)w] = 0;
+        if (x == least[(size_t)w]) mask[(size_t)w] |= 1u << (8 * v + a);
+      }
+    }
+  std::vector<unsigned char> out((size_t)nv * 6);
+  uint16_t* rank = (uint16_t*)out.data();  // (the values themselves are below 2^12)
+  for (int w = 0; w < nv; ++w) rank[w] = (uint16_t)least[(size_t)w];
+  std::copy(mask.begin(), mask.end(), (uint32_t*)(out.data() + 2 * (size_t)nv));
+  return out;
+}
+
+// The bit permutation of a candidate code of Win<kWinPoint, L, L>.
+inline std::vector<int32_t> win_point_perm(int L, int code) {
+  const int v = (code >> 6) & 3, top = (code >> 3) & 7, a = code & 7;
+  std::vector<int32_t> perm((size_t)(L * L));
+  for (int y = 0; y < L; ++y)
+    for (int x = 0; x < L; ++x) {
+      int i = x, j = y;
+      if (code >> 8) std::swap(i, j);
+      if (v & 1) i = L - 1 - i;
+      if (v & 2) j = L - 1 - j;
+      perm[(size_t)(x + L * y)] = (i + a) % L + L * ((j + L - 1 - top) % L);
+    }
+  return perm;
+}
+
 // Off-diagonal term as the products see it: the row b matches iff
 // (b & mask) == match; its image is (b & ~mask) | image.
 struct OffTerm {

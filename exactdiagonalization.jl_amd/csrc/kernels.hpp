@@ -29,6 +29,8 @@ hipError_t launch_mark_tops(const uint64_t* d_keys, int64_t dim, int shift, uint
 // x / sqrt(orbit) (the orbit factor of the images, X.scaled).
 hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, int64_t dim, const void* x,
                             const uint16_t* d_orbit, hipStream_t st);
+// positions of the keys in the spread X
+hipError_t launch_xmap_positions(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t* d_pos, hipStream_t st);
 // prefix[j] = lower_bound(keys, j << shift), j <= n_buckets
 hipError_t launch_build_prefix(const uint64_t* d_keys, int64_t dim, int shift, uint64_t n_buckets, uint32_t* d_prefix,
                                hipStream_t st);
@@ -166,6 +168,9 @@ struct WinOp {
   const uint32_t* rank_base;  // number of sector words with a smaller upper part
   int low_bits;
   uint32_t base_bytes;        // of rank_base, a multiple of 16
+  // point operations (values: x / sqrt(N) itself): rank blocks over the positions
+  const uint64_t* pos_blocks;
+  int point_swap;
 };
 // Sectors of up to this many bits are ranked by two LDS tables (13 + 13 bits: 48 KiB)
 constexpr int kRankBits = 26;
@@ -177,6 +182,13 @@ inline uint32_t win_entries_bytes(int n_lin, int n_chunk, int n_rest) {
 // LDS bytes below the entries (WinLds, at most)
 inline uint32_t win_fixed_bytes(int kind, int Lx) {
   return (2u << win_index_bits(kind, Lx)) + 64u * 16u + kXCodesBytesMax + 2u * 4096u;
+}
+
+// The same with point operations of an L x L torus, phases by candidate code
+// and the flip's four words included
+inline uint32_t win_point_bytes(int L, int n_lin, int n_chunk, int n_rest) {
+  return (6u << (2 * L)) + 512u * 16u + kXCodesBytesMax + 2u * 4096u + win_entries_bytes(n_lin, n_chunk, n_rest) +
+         24u * (uint32_t)(n_lin + n_rest + 1);
 }
 
 enum Prec : int { kF64 = 0, kC128 = 1, kF32 = 2, kC64 = 3 };

@@ -151,9 +151,10 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
 template <int KIND, int LX, int LY, bool UNIT>
 struct WinLds {
   using S = Win<KIND, LX, LY>;
+  static constexpr uint32_t n_codes = S::kPoint ? 512 : 64;  // candidates
   static constexpr uint32_t tab = 0;
-  static constexpr uint32_t phase = tab + S::kTab * 2;
-  static constexpr uint32_t codes = phase + (UNIT ? 0 : 64 * 16);
+  static constexpr uint32_t phase = tab + S::kTabBytes;
+  static constexpr uint32_t codes = phase + (UNIT ? 0 : n_codes * 16);
   static constexpr uint32_t colex = codes + kXCodesBytesMax;
   static constexpr uint32_t entries = colex + 2 * 4096;
 };
@@ -163,6 +164,12 @@ struct WinLds {
 template <typename W, typename A>
 struct WinEntry {
   W flip;
+  A amp;
+};
+// with point operations: the flip's words (Win<kWinPoint>)
+template <typename W, typename A>
+struct PointEntry {
+  W flip[4];
   A amp;
 };
 
@@ -181,6 +188,12 @@ struct WinEntry {
 // read of each of two LDS tables (no spread to fill, and x is denser: 4x6 XXZ,
 // 2.7e6 states, FP64: 174 us a call through the spread by the general kernel,
 // 118 us by rank).
+//
+// KIND = kWinPoint: translations and point operations.  These spaces are 8
+// times sparser in their words, so a spread would take a line per state (6x6
+// A1, FP64: 8.2 GB for 31.6M states): the position of the spread is ranked
+// through bits instead (blocks of 384 positions, 172 MB, which stay in the
+// last-level cache with x / sqrt(N) itself).
 template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS, bool RANK = false>
 __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __restrict__ x, V* __restrict__ y) {
   using S = Win<KIND, LX, LY>;
@@ -191,12 +204,12 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   // FP32 vectors without a complex phase weigh in FP32, from FP32 amplitudes and phases of +-1
   constexpr bool kW32 = std::is_same<R, float>::value && (!CX || UNIT);
   using A = typename std::conditional<kW32, float, double>::type;
-  using E = WinEntry<W, A>;
+  using E = typename std::conditional<S::kPoint, PointEntry<W, A>, WinEntry<W, A>>::type;
   extern __shared__ unsigned char lds[];
-  lds_copy16(lds + Lay::tab, P.win_tab, S::kTab * 2);
+  lds_copy16(lds + Lay::tab, P.win_tab, S::kTabBytes);
   if constexpr (!UNIT) {
     double* ph = (double*)(lds + Lay::phase);
-    if (threadIdx.x < 64) {
+    if (threadIdx.x < Lay::n_codes) {
       const int h = P.win_elem[threadIdx.x];
       ph[2 * threadIdx.x] = P.ph_re[h];
       ph[2 * threadIdx.x + 1] = TRANS ? -P.ph_im[h] : P.ph_im[h];
@@ -222,7 +235,12 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
 #pragma unroll 1
   for (int t = threadIdx.x; t < n_ent; t += kMvBlock) {
     const MvEntry e = P.ent[t];
-    ent[t] = E{(W)e.flip, (A)e.are};
+    if constexpr (S::kPoint) {
+      S::words((W)e.flip, ent[t].flip);
+      ent[t].amp = (A)e.are;
+    } else {
+      ent[t] = E{(W)e.flip, (A)e.are};
+    }
     if (CX) aim[t] = e.aim;
   }
 #pragma unroll 1
@@ -242,16 +260,21 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   const uint16_t* colex = (const uint16_t*)(lds + Lay::colex);
   const double2* phase = (const double2*)(lds + Lay::phase);
   const uint32_t top_max = 1u << P.top_bits;
+  W bw[4];  // (point operations: the row's words)
+  if constexpr (S::kPoint) S::words(b, bw);
+  auto position = [&](W s) {  // of the canonical word s in the spread
+    const uint32_t top = (uint32_t)(s >> P.top_shift);
+    const uint32_t c = codes[top < top_max ? top : top_max];
+    const uint32_t lo = (uint32_t)s;
+    const uint32_t hc = (c << P.hbits) | __builtin_amdgcn_ubfe(lo, 12u, (uint32_t)P.hbits);
+    return __umul24(hc, 924u) + (uint32_t)colex[lo & 0xfffu];
+  };
   auto fetch = [&](W s) {  // x (/ sqrt(N)) of the canonical word s
     if constexpr (RANK) {
       const uint32_t lo = (uint32_t)s & ((1u << P.low_bits) - 1u);
       return x[((const uint32_t*)(lds + rank_low))[s >> P.low_bits] + (uint32_t)((const uint16_t*)lds)[lo]];
     }
-    const uint32_t top = (uint32_t)(s >> P.top_shift);
-    const uint32_t c = codes[top < top_max ? top : top_max];
-    const uint32_t lo = (uint32_t)s;
-    const uint32_t hc = (c << P.hbits) | __builtin_amdgcn_ubfe(lo, 12u, (uint32_t)P.hbits);
-    return ((const V*)P.values)[(uint64_t)(__umul24(hc, 924u) + (uint32_t)colex[lo & 0xfffu])];
+    return ((const V*)P.values)[(uint64_t)position(s)];
   };
   V acc = vzero<V>();
   auto add = [&](const V& xv, int t, const E& e, int bit) {
@@ -328,11 +351,31 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
       V xv[NW];
 #pragma unroll
       for (int k = 0; k < NW; ++k) {
-        e[k] = ent[t[k]];
-        S::canonical(tab, b ^ e[k].flip, P.n_bits, s[k], w[k]);
+        if constexpr (S::kPoint)
+          e[k].amp = ent[t[k]].amp;
+        else
+          e[k] = ent[t[k]];
+        if constexpr (S::kPoint)
+          S::canonical(tab, bw, ent[t[k]].flip, P.point_swap, s[k], w[k]);
+        else
+          S::canonical(tab, b ^ e[k].flip, P.n_bits, s[k], w[k]);
       }
+      if constexpr (S::kPoint) {  // both blocks, then both elements
+        uint32_t at[NW];
+        RankBlock blk[NW];
 #pragma unroll
-      for (int k = 0; k < NW; ++k) xv[k] = fetch(s[k]);
+        for (int k = 0; k < NW; ++k) blk[k] = rank_block(P.pos_blocks, at[k] = position(s[k]));
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+          uint64_t i;
+          const bool in = rank_in(blk[k], at[k], i);
+          xv[k] = ((const V*)P.values)[i];
+          if (!in) xv[k] = vzero<V>();
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < NW; ++k) xv[k] = fetch(s[k]);
+      }
       add(xv[0], t[0], e[0], w[0]);
 #pragma unroll
       for (int k = 1; k < NW; ++k)
@@ -355,7 +398,8 @@ template <typename V, int KIND, int LX, int LY>
 hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, void* y, hipStream_t st) {
   const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
   const dim3 grid((unsigned)((lanes + kMvBlock - 1) / kMvBlock));
-  const uint32_t dyn = win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest);
+  const uint32_t dyn =
+      win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest) + (KIND == kWinPoint ? 24u * (uint32_t)(P.n_lin + P.n_rest + 1) : 0u);
   // the column form only conjugates the phase
   constexpr bool kT = VT<V>::cx;
   if (unit)
@@ -377,6 +421,17 @@ hipError_t launch_win_v(const WinOp& P, int Lx, int Ly, int unit, int transpose,
   if (Lx == X && Ly == Y) return launch_win_t<V, K, X, Y>(P, unit, transpose, x, y, st);
   EDHIP_WIN_SHAPES(EDHIP_X)
 #undef EDHIP_X
+  return hipErrorInvalidValue;
+}
+
+template <typename V>
+hipError_t launch_win_other(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
+                            hipStream_t st) {
+  if (P.pos_blocks) {
+    if (Lx == 5 && Ly == 5) return launch_win_t<V, kWinPoint, 5, 5>(P, unit, transpose, x, y, st);
+    if (Lx == 6 && Ly == 6) return launch_win_t<V, kWinPoint, 6, 6>(P, unit, transpose, x, y, st);
+    return hipErrorInvalidValue;
+  }
   if (Ly == 0) {  // no group
     const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
     const dim3 grid((unsigned)((lanes + kMvBlock - 1) / kMvBlock));
@@ -395,7 +450,7 @@ hipError_t launch_win_v(const WinOp& P, int Lx, int Ly, int unit, int transpose,
   }
   if (Ly == 1 && Lx <= 32) return launch_win_t<V, kWinChain, 32, 1>(P, unit, transpose, x, y, st);
   if (Ly == 1 && Lx <= 48) return launch_win_t<V, kWinChain, 48, 1>(P, unit, transpose, x, y, st);
-  return hipErrorInvalidValue;
+  return launch_win_v<V>(P, Lx, Ly, unit, transpose, x, y, st);
 }
 
 template <typename V, int MODE>

@@ -10,7 +10,7 @@ hipError_t launch_product_c128(const OpDev& op, int transpose, int accumulate, c
 
 hipError_t launch_window_product_c128(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
                                     hipStream_t st) {
-  return launch_win_v<Cx<double>>(P, Lx, Ly, unit, transpose, x, y, st);
+  return launch_win_other<Cx<double>>(P, Lx, Ly, unit, transpose, x, y, st);
 }
 
 }  // namespace edhip

@@ -333,6 +333,14 @@ __global__ __launch_bounds__(kBlock) void k_xmap_fill(XMapDev X, const uint64_t*
   ((V*)X.values)[pos] = v;
 }
 
+__global__ __launch_bounds__(kBlock) void k_xmap_positions(XMapDev X, const uint64_t* __restrict__ keys, int64_t dim,
+                                                           uint64_t* __restrict__ pos) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= dim) return;
+  const uint64_t k = keys[i];
+  pos[i] = xmap_pos(X, X.colex, X.topcode[k >> X.top_shift], k);
+}
+
 __global__ void k_u32_to_u64(const uint32_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = in[i];
@@ -456,6 +464,13 @@ hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, 
     default:
       return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_xmap_positions(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t* d_pos,
+                                 hipStream_t st) {
+  if (dim == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_xmap_positions, dim3(grid_for((uint64_t)dim)), dim3(kBlock), 0, st, X, d_keys, dim, d_pos);
   return hipGetLastError();
 }
 

@@ -26,7 +26,7 @@
 
 namespace edhip {
 
-enum WinKind : int { kWinNone = 0, kWinPairs = 1, kWinRows = 2, kWinChain = 3 };
+enum WinKind : int { kWinNone = 0, kWinPairs = 1, kWinRows = 2, kWinChain = 3, kWinPoint = 4 };
 
 // Shapes compiled as their own kernels (lattices of up to 36 sites on which
 // products take long enough to matter; others run the general kernels).
@@ -62,10 +62,12 @@ struct WinWord<false> {
 template <int KIND, int LX, int LY>
 struct Win {
   static constexpr bool kChain = KIND == kWinChain;
+  static constexpr bool kPoint = false;
   static constexpr int NB = LX * LY;  // (a chain: the longest)
   static constexpr int MB = win_mask_bits(KIND);
   static constexpr int NW = kChain ? (LX + 5) / 6 : LY;  // windows
   static constexpr int kTab = 1 << win_index_bits(KIND, LX);
+  static constexpr uint32_t kTabBytes = 2u * kTab;
   static constexpr bool kWide = NB > 32;
   using W = typename WinWord<kWide>::T;
   using C = typename WinWord<(NW > 4)>::T;  // candidate mask
@@ -200,12 +202,147 @@ struct Win {
   }
 };
 
+// Translations and point operations of an L x L torus (L 5 or 6).  The images
+// of the pair window (row y, the row below) under the rows' reversal, their
+// exchange (the reflection in y shows the pair upside down) and both begin with
+// permuted copies of the same two rows, so that one table read gives the least
+// beginning over the four variants and all rotations: its rank (u16), and in a
+// second table, read for the windows that reach the least rank, the mask of
+// (variant, rotation) that reach it (8 bits per variant: bit 0 of the variant
+// reverses the rows' bits, bit 1 the order of the rows).  The other four point
+// operations are these after the transposition, whose windows are ranked
+// beside.  Each of these maps commutes with XOR, so the words of an image are
+// those of its row XORed with those of the flip, and nothing is permuted per
+// image.  (Bounding eight cosets one by one, each permuted by 4-bit tables:
+// 950 VALU instructions per image on the 6x6 A1 sector.)
+//
+// words: b, rows in reverse order, transposed, transposed and reversed.
+template <int L, int L2>
+struct Win<kWinPoint, L, L2> {
+  static constexpr bool kChain = false, kPoint = true;
+  static constexpr int NB = L * L;
+  static constexpr int kTab = 1 << (2 * L);
+  static constexpr uint32_t kTabBytes = 6u * kTab;  // ranks, then masks
+  using W = typename WinWord<(NB > 32)>::T;
+  using T = Win<kWinPairs, L, L>;
+
+  EDHIP_HD static W transposed(W b) {
+    W out = 0;
+#pragma unroll
+    for (int d = 1 - L; d < L; ++d) {  // the diagonal x - y = d moves by d (L - 1)
+      W m = 0;
+      for (int y = 0; y < L; ++y)
+        if (y + d >= 0 && y + d < L) m |= (W)1 << (y + d + L * y);
+      out |= d < 0 ? (b & m) >> (-d * (L - 1)) : (b & m) << (d * (L - 1));
+    }
+    return out;
+  }
+  EDHIP_HD static W rows_reversed(W b) {
+    W out = 0;
+#pragma unroll
+    for (int y = 0; y < L; ++y) out |= ((b >> (L * y)) & (((W)1 << L) - 1)) << (L * (L - 1 - y));
+    return out;
+  }
+  EDHIP_HD static uint32_t reversed32(uint32_t v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __brev(v);
+#else
+    uint32_t o = 0;
+    for (int i = 0; i < 32; ++i) o |= ((v >> i) & 1u) << (31 - i);
+    return o;
+#endif
+  }
+  EDHIP_HD static W reversed(W b) {
+    if constexpr (NB > 32)
+      return (((W)reversed32((uint32_t)b) << 32) | reversed32((uint32_t)(b >> 32))) >> (64 - NB);
+    else
+      return reversed32(b) >> (32 - NB);
+  }
+  EDHIP_HD static void words(W b, W* out) {
+    out[0] = b;
+    out[1] = rows_reversed(b);
+    out[2] = transposed(b);
+    out[3] = rows_reversed(out[2]);
+  }
+
+  // The smallest image s of the word whose words are b[] ^ f[], and the code
+  // (transposed, variant, 8 y + a) << ... of the first candidate giving it:
+  // bit 8: transposed, bits 6 and 7: variant, then 8 y + a as for translations.
+  // swap: the group holds the transposed variants too.
+  EDHIP_HD static void canonical(const uint16_t* tab, const W* b, const W* f, int swap, W& s, int& code) {
+    const uint32_t* masks = (const uint32_t*)(tab + kTab);
+    const W w = b[0] ^ f[0], wt = b[2] ^ f[2];
+    uint32_t cand;  // bit y: window y of w, bit 16 + y: of its transpose
+#ifdef __HIP_DEVICE_COMPILE__
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 p[L];
+#pragma unroll
+    for (int y = 0; y < L; ++y) {
+      p[y].x = tab[T::window(w, 0, y)];
+      p[y].y = swap ? tab[T::window(wt, 0, y)] : (uint16_t)0xffffu;
+    }
+    u16x2 m = p[0];
+#pragma unroll
+    for (int y = 1; y < L; ++y) m = __builtin_elementwise_min(m, p[y]);
+    const uint16_t lo = m.x < m.y ? m.x : m.y;
+    uint32_t other = 0;
+#pragma unroll
+    for (int y = 0; y < L; ++y) {
+      const u16x2 d = __builtin_elementwise_min((u16x2)(p[y] - (u16x2){lo, lo}), (u16x2){1, 1});
+      other |= __builtin_bit_cast(uint32_t, d) << y;
+    }
+    cand = ~other & (((1u << L) - 1u) * 0x10001u);
+#else
+    uint32_t p[2 * L], lo = 0xffffu;
+    for (int y = 0; y < 2 * L; ++y) {
+      p[y] = y < L ? tab[T::window(w, 0, y)] : swap ? tab[T::window(wt, 0, y - L)] : 0xffffu;
+      lo = p[y] < lo ? p[y] : lo;
+    }
+    cand = 0;
+    for (int y = 0; y < 2 * L; ++y)
+      if (p[y] == lo) cand |= 1u << (y < L ? y : 16 + y - L);
+#endif
+    s = (W)~(W)0;
+    code = 0;
+    uint32_t mask = 0;
+    int q = 0;
+    W src = 0;
+    do {
+      if (!mask) {
+        q = T::ctz(cand);
+        cand &= cand - 1;
+        src = q >= 16 ? wt : w;
+        mask = masks[T::window(src, 0, q & 15)];
+      }
+      const int r = T::ctz(mask), a = r & 7, v = r >> 3, y = q & 15;
+      mask &= mask - 1;
+      // the row after the beginning, against that of the least image so far
+      const int yn = v < 2 ? (y >= 2 ? y - 2 : y + L - 2) : (y + 1 < L ? y + 1 : 0);
+      uint32_t n = (uint32_t)(src >> (uint32_t)(yn * L)) & ((1u << L) - 1u);
+      n = (v & 1) ? reversed32(n) >> (32 - L) : n;
+      n = ((n << a) | (n >> (L - a))) & ((1u << L) - 1u);
+      if (n > ((uint32_t)(s >> ((L - 3) * L)) & ((1u << L) - 1u))) continue;
+      const int g = (q >= 16 ? 2 : 0) | ((v ^ (v >> 1)) & 1);
+      W u = (g & 1) ? ((g & 2) ? b[3] : b[1]) ^ f[g] : src;
+      if (v & 1) u = reversed(u);
+      const int bit = 8 * (v < 2 ? y : (y ? L - y : 0)) + a;
+      const W t = T::image(u, 0, bit);
+      code = t < s ? (q >= 16 ? 256 : 0) + 64 * v + bit : code;
+      s = t < s ? t : s;
+    } while (mask | cand);
+  }
+};
+
+// The window tables exist for square tori of these sides with point operations.
+inline bool win_point_side(int L) { return L == 5 || L == 6; }
+
 // No group: every word is its own image (LX: bits of the widest word).
 template <int LX, int LY>
 struct Win<kWinNone, LX, LY> {
   static constexpr bool kChain = true;  // (the number of word bits is a run-time value)
+  static constexpr bool kPoint = false;
   static constexpr int NB = LX;
-  static constexpr int kTab = 0;
+  static constexpr uint32_t kTabBytes = 0;
   using W = typename WinWord<(LX > 32)>::T;
   EDHIP_HD static void canonical(const uint16_t*, W b, int, W& s, int& bit) {
     s = b;

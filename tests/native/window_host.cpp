@@ -46,8 +46,59 @@ static int check(int Lx, int Ly, std::mt19937_64& rng) {
   return 0;
 }
 
+static uint64_t permuted(uint64_t b, const std::vector<int32_t>& perm) {
+  uint64_t out = 0;
+  for (size_t i = 0; i < perm.size(); ++i)
+    if ((b >> i) & 1) out |= 1ull << perm[i];
+  return out;
+}
+
+// Point operations: variants (bits) alone or with their transposes.
+template <int L>
+static int check_point(int variants, int swap, std::mt19937_64& rng) {
+  using S = Win<kWinPoint, L, L>;
+  using W = typename S::W;
+  const int n = L * L;
+  const std::vector<unsigned char> bytes = win_point_table(L, variants);
+  if (bytes.size() != S::kTabBytes) return std::printf("point %d: table size\n", L), 1;
+  std::vector<uint64_t> aligned(bytes.size() / 8);
+  std::copy(bytes.begin(), bytes.end(), (unsigned char*)aligned.data());
+  std::vector<std::vector<int32_t>> perms;
+  for (int code = 0; code < 512; ++code)
+    if ((code & 7) < L && ((code >> 3) & 7) < L && ((variants >> ((code >> 6) & 3)) & 1) && (swap || code < 256))
+      perms.push_back(win_point_perm(L, code));
+  const uint64_t full = (1ull << n) - 1;
+  for (int k = 0; k < 1500; ++k) {
+    uint64_t row = rng() & full;
+    if (k % 4 == 1) row &= rng();
+    if (k % 4 == 2) {  // symmetric: many candidates
+      const uint64_t line = rng() & ((1ull << L) - 1);
+      row = 0;
+      for (int y = 0; y < L; ++y) row |= line << (L * y);
+      row ^= (k & 4) ? 0 : S::transposed((W)row);
+    }
+    if (k < 2) row = k ? full : 0;
+    const uint64_t flip = (k % 3) ? (1ull << (rng() % n)) ^ (1ull << (rng() % n)) : 0;
+    W b[4], f[4];
+    S::words((W)row, b);
+    S::words((W)flip, f);
+    uint64_t want = ~0ull;
+    for (const auto& p : perms) want = std::min(want, permuted(row ^ flip, p));
+    W s;
+    int code;
+    S::canonical((const uint16_t*)aligned.data(), b, f, swap, s, code);
+    if ((uint64_t)s != want || permuted(row ^ flip, win_point_perm(L, code)) != want)
+      return std::printf("point %d, variants %d, swap %d: %llx -> %llx (code %d), not %llx\n", L, variants, swap,
+                         (unsigned long long)(row ^ flip), (unsigned long long)s, code, (unsigned long long)want), 1;
+  }
+  return 0;
+}
+
 int main() {
   std::mt19937_64 rng(3);
+  for (int swap = 0; swap < 2; ++swap)
+    for (int variants : {1, 3, 5, 9, 15})
+      if (check_point<5>(variants, swap, rng) || check_point<6>(variants, swap, rng)) return 1;
 #define EDHIP_X(K, X, Y) \
   if (check<K, X, Y>(X, Y, rng)) return 1;
   EDHIP_WIN_SHAPES(EDHIP_X)
