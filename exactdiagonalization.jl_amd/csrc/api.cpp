@@ -440,40 +440,28 @@ struct edhip_space {
     }
   }
 
-  // Rank blocks over the colex positions of the words (layout as the blocked
-  // rank index, 6 positions per byte): 6x6 A1, 172 MB against 5.7 GB over the
-  // words themselves.
-  mutable DevBuf pos_blocks;
+  // Ranks of the words' colex positions (6x6 A1: 258 MB, against 5.7 GB over the
+  // words themselves).
+  mutable DevBuf pos_bits;
   mutable bool pos_tried = false;
   mutable XMapDev pos_dev{};
   bool ensure_positions() const {
-    if (pos_tried) return pos_blocks.p != nullptr;
+    if (pos_tried) return pos_bits.p != nullptr;
     pos_tried = true;
-    if (dim == 0) return false;
+    if (dim == 0 || (uint64_t)dim >= 0xffffffffull) return false;
     const uint64_t n_pos = ensure_xtop();
     if (!xcolex_on || n_bits - xtop_shift > 32) return false;
-    const uint64_t n_blocks = (n_pos + kRankBlockWords - 1) / kRankBlockWords;
-    if (n_blocks * 64 > std::max<uint64_t>(kBitmapMaxRatio * (uint64_t)dim * 8ull, 1ull << 20)) return false;
+    const uint64_t n_blocks = (n_pos + 31) / 32, bytes = n_blocks * sizeof(RankBits);
+    if (bytes > std::max<uint64_t>(kBitmapMaxRatio * (uint64_t)dim * 8ull, 1ull << 20)) return false;
     pos_dev = XMapDev{nullptr, xtop.as<uint16_t>(), xcolex.as<uint16_t>(), xtop_K, xtop_bits, xtop_shift,
                       xtop_shift - 12, -1, 0, 1};
     try {
-      DevBuf pos, totals, base, tmp;
-      pos.alloc((size_t)dim * 8);
-      totals.alloc(n_blocks * 4);
-      base.alloc(n_blocks * 8);
-      pos_blocks.alloc(n_blocks * 64);
-      HIP_OR_THROW(hipMemsetAsync(pos_blocks.p, 0, n_blocks * 64, ctx->stream));
-      HIP_OR_THROW(launch_xmap_positions(pos_dev, keys.as<uint64_t>(), dim, pos.as<uint64_t>(), ctx->stream));
-      size_t tb = 0;
-      HIP_OR_THROW(launch_bitmap_build(pos.as<uint64_t>(), dim, pos_blocks.as<uint64_t>(), n_blocks,
-                                       totals.as<uint32_t>(), base.as<uint64_t>(), nullptr, tb, ctx->stream));
-      tmp.alloc(tb);
-      HIP_OR_THROW(launch_bitmap_build(pos.as<uint64_t>(), dim, pos_blocks.as<uint64_t>(), n_blocks,
-                                       totals.as<uint32_t>(), base.as<uint64_t>(), tmp.p, tb, ctx->stream));
-      ctx->sync();
+      pos_bits.alloc(bytes);
+      HIP_OR_THROW(launch_position_ranks(pos_dev, keys.as<uint64_t>(), dim, n_blocks, pos_bits.as<RankBits>(),
+                                         ctx->stream));
       return true;
     } catch (const Error& e) {
-      pos_blocks.release();
+      pos_bits.release();
       if (e.code != EDHIP_ERR_MEMORY) throw;
       (void)hipGetLastError();  // no room: the general kernels
       return false;
@@ -863,9 +851,11 @@ void build_group(GroupHost& gh, int nb, double tol, hipStream_t st) {
         variants[code >> 8] |= 1 << ((code >> 6) & 3);
         ++found;
       }
-      if (found == G && (variants[1] == 0 || variants[1] == variants[0])) {
+      const bool one_set = found == G && (variants[1] == 0 || variants[1] == variants[0]);
+      const std::vector<uint16_t> tab = one_set ? win_point_table(bestLx, variants[0]) : std::vector<uint16_t>();
+      if (!tab.empty()) {
         for (int32_t& e : elem) e = std::max(e, 0);
-        upload(gh.point_tab, win_point_table(bestLx, variants[0]), st);
+        upload(gh.point_tab, tab, st);
         upload(gh.point_elem, elem, st);
         d.point_tab = gh.point_tab.as<uint16_t>();
         d.point_elem = gh.point_elem.as<int32_t>();
@@ -1324,11 +1314,21 @@ constexpr uint64_t kAutoAsmMaxBytes = 16ull << 30;
 // Lanes per row and entries per lane per batch of the assembled product
 // (0: chosen from the mean entries per row)
 std::atomic<int> g_asm_lanes{0}, g_asm_batch{0};
-// Consecutive blocks per XCD and window in the products (xcd_chunked_block):
-// 32 measured at 6x6 against the plain order (1), same results bitwise:
-// term list FP32 82.3 / 83.1 ms, FP64 85.8 / 88.1 ms; assembled rows FP32
-// 69.1 / 70.2 ms, FP64 82.0 / 82.7 ms (2 to 64 in between or level)
+// Consecutive blocks per XCD and window in the products (xcd_chunked_block), for
+// grids of a few windows; every order gives the same results bitwise.
 std::atomic<int> g_xcd_chunk{32};
+
+// The same for a grid of n_blocks: as many times more, up to 16, as leave it 8
+// whole windows.  The more neighbouring rows an XCD holds at a time, the more of
+// their gathers meet in its L2 (32 against 512): 6x6 A1, assembled rows FP32 9.84
+// to 9.43 ms (L2 misses 5.3e8 to 4.5e8), FP64 11.39 to 10.69, matrix-free FP64
+// 19.88 to 19.28 ms; 6x6 (0,0) FP32 60.5 to 59.7 ms.  (Against the plain order,
+// 1: 6x6 assembled rows FP32 70.2 ms plain, 69.1 with 32.)
+int xcd_chunk_for(int64_t n_blocks) {
+  int c = g_xcd_chunk.load();
+  for (int k = 0; k < 4 && c > 1 && 128ll * c <= n_blocks; ++k) c *= 2;
+  return c;
+}
 
 void asm_shape(const edhip_op* op, int& lanes, int& batch) {
   const double mean = op->space->dim ? (double)op->asm_nnz / (double)op->space->dim : 0.0;
@@ -1336,6 +1336,14 @@ void asm_shape(const edhip_op* op, int& lanes, int& batch) {
   if (!lanes) lanes = mean < 12.0 ? 4 : mean < 40.0 ? 8 : mean < 160.0 ? 16 : 32;
   batch = g_asm_batch.load();
   if (!batch) batch = 8;
+}
+
+// Whether the images of the operator's rows are found through the window tables
+// of the point operations: their group, images that keep the popcount, ranks of
+// the positions and LDS room for the product's and the fill's tables.
+bool point_rows(const edhip_op* op, const OpDev& d) {
+  return d.g.point_tab && d.orbit && op->keeps_popcount &&
+         win_point_bytes(d.g.Lx, d.n_lin, d.n_chunk, d.n_rest) <= 64 * 1024 && op->space->ensure_positions();
 }
 
 // Assembled rows of the row form (strategy 3): the entry count of every row
@@ -1354,7 +1362,8 @@ bool ensure_assembled(edhip_op* op, uint64_t max_bytes = ~0ull) {
   while (col_bits < 32 && (1ull << col_bits) < (uint64_t)D) ++col_bits;
   if (col_bits > 31) fail(EDHIP_ERR_ARGUMENT, "assembled rows hold at most 2^31 basis states");
   OpDev d = op->dev_row;
-  d.ix = sp->index_dev(0);
+  const bool point = point_rows(op, d);
+  if (!point) d.ix = sp->index_dev(0);
   const std::vector<MvEntry>& terms = (d.ent == op->mv[0].ent.as<MvEntry>() ? op->mv[0] : op->mv_plain[0]).entries;
   const int nt = (int)terms.size();
   std::vector<std::complex<double>> amps, phs;
@@ -1418,7 +1427,10 @@ bool ensure_assembled(edhip_op* op, uint64_t max_bytes = ~0ull) {
     upload(op->asm_w, w, st);
     AsmFillDev f{op->asm_rowptr.as<uint64_t>(), op->asm_ent.as<uint32_t>(), op->asm_acls.as<uint32_t>(),
                  use_ph ? op->asm_pcls.as<uint32_t>() : nullptr, n_ph, col_bits};
-    HIP_OR_THROW(launch_asm_fill(d, f, st));
+    if (point)
+      HIP_OR_THROW(launch_asm_fill_point(d, f, sp->pos_dev, sp->pos_bits.as<RankBits>(), (uint32_t)D, st));
+    else
+      HIP_OR_THROW(launch_asm_fill(d, f, st));
     HIP_OR_THROW(hipStreamSynchronize(st));
   } catch (...) {
     (void)hipGetLastError();
@@ -1442,17 +1454,17 @@ void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) 
     d.diag_re = op->diag_re.as<double>();
     d.diag_im = op->diag_im.as<double>();
   }
-  d.xcd_chunk = g_xcd_chunk.load();
   const size_t es = elem_size(prec);
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
   const void* xt = x;
   if (d.orbit) {
-    op->asm_xt.ensure((size_t)sp->dim * es);
+    op->asm_xt.ensure((size_t)(sp->dim + 1) * es);
     HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, x, op->asm_xt.p, st));
     xt = op->asm_xt.p;
   }
   int lanes, batch;
   asm_shape(op, lanes, batch);
+  d.xcd_chunk = xcd_chunk_for(sp->dim * lanes / 256);
   HIP_OR_THROW(launch_asm_spmv(d, op->asm_dev, prec, lanes, batch, accumulate, x, xt, y, st));
   if (op->ctx->kernel_timing) {
     HIP_OR_THROW(hipEventRecord(op->ctx->ev[15], st));
@@ -1504,11 +1516,9 @@ bool rank_product(const edhip_op* op, const OpDev& d) {
 // the operator's buffer.
 bool point_product(edhip_op* op, const OpDev& d, int prec, const void* x) {
   const edhip_space* sp = op->space;
-  if (!d.g.point_tab || !d.orbit || !op->keeps_popcount || !(d.diag_re || op->n_diag == 0) ||
-      win_point_bytes(d.g.Lx, d.n_lin, d.n_chunk, d.n_rest) > 64 * 1024 || !sp->ensure_positions())
-    return false;
+  if (!(d.diag_re || op->n_diag == 0) || !point_rows(op, d)) return false;
   try {
-    op->asm_xt.ensure((size_t)sp->dim * elem_size(prec));
+    op->asm_xt.ensure((size_t)(sp->dim + 1) * elem_size(prec));
   } catch (const Error& e) {
     if (e.code != EDHIP_ERR_MEMORY) throw;
     (void)hipGetLastError();
@@ -1527,11 +1537,9 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   const bool rank_mode = sp->is_sector && !sp->group;
   const int idx_lookup = (op->strat_lookup == 2) ? 0 : op->strat_lookup;  // the hash applies to the pair kernel only
   OpDev d = transpose ? op->dev_col : op->dev_row;
-  d.xcd_chunk = g_xcd_chunk.load();
   d.row_begin = row_begin;
   d.dim = row_end;
   d.row_lanes = mv_row_lanes(sp->dim, d.n_lin + d.n_rest);
-  d.stripe = d.row_lanes == 0 ? ~0ull : ~0ull / ((1ull << (1 << d.row_lanes)) - 1ull);
   if (ensure_diag(op)) {
     d.diag_re = op->diag_re.as<double>();
     d.diag_im = op->diag_im.as<double>();
@@ -1539,6 +1547,12 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   op->used_kernel = 1;
   const bool point = idx_lookup == 0 && point_product(op, d, prec, x);
   if (!point) d.ix = sp->index_dev(idx_lookup == 4 ? 0 : idx_lookup);
+  // two lanes to a row at least: with half the rows in flight more of the two
+  // gathers per image hit the L2 (6x6 A1, FP64: 21.1 ms with one, 19.9 with two,
+  // 19.6 with four, 22.9 with eight)
+  if (point && d.n_lin + d.n_rest >= 2) d.row_lanes = std::max(d.row_lanes, 1);
+  d.stripe = d.row_lanes == 0 ? ~0ull : ~0ull / ((1ull << (1 << d.row_lanes)) - 1ull);
+  d.xcd_chunk = xcd_chunk_for(((row_end - row_begin) << d.row_lanes) / 512);
   op->used_lookup = rank_mode ? 1 : (point || d.ix.bm_bits ? 3 : 1);
   const bool ranked = idx_lookup <= 1 && rank_product(op, d);
   if (!point && !ranked && attach_spread(op, prec, d, d.mv_codes_lds, x, st, true)) op->used_lookup = 4;
@@ -1551,8 +1565,8 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
                   g.ph_im,     X.topcode, X.colex,     op->asm_xt.p, d.lin_tab, d.ent,      d.rest,
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, X.top_bits, X.top_shift,
-                  X.hbits,     nullptr,   nullptr,     0,          0,         sp->pos_blocks.as<uint64_t>(),
-                  g.point_swap};
+                  X.hbits,     nullptr,   nullptr,     0,          0,         sp->pos_bits.as<RankBits>(),
+                  (uint32_t)sp->dim, g.point_swap};
     HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
   } else if (ranked || window_product(op, d)) {
     const GroupDev& g = d.g;
@@ -1561,7 +1575,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, d.xm.top_bits, d.xm.top_shift,
                   d.xm.hbits,  ranked ? sp->rank_low.as<uint16_t>() : nullptr, sp->rank_base.as<uint32_t>(),
-                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes, nullptr, 0};
+                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes, nullptr, 0, 0};
     const bool none = g.mode == kGroupNone;
     HIP_OR_THROW(launch_window_product(P, none ? 0 : g.Lx, none ? 0 : g.Ly, none ? 1 : g.unit_phases, prec,
                                        transpose ? 1 : 0, x, y, st));

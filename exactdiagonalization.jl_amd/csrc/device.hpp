@@ -127,6 +127,29 @@ __device__ __forceinline__ uint64_t next_same_popcount(uint64_t v) {
   return (t + 1) | (((~t & (t + 1)) - 1) >> (__builtin_ctzll(v) + 1));
 }
 
+// Ranks of set positions: per 32 positions their bits and the number of set ones
+// below (one 8-byte load and three VALU instructions per rank).
+struct RankBits {
+  uint32_t bits, base;
+};
+// The rank of position pos among the set ones, or none.
+__device__ __forceinline__ uint32_t rank_of(RankBits r, uint32_t pos, uint32_t none) {
+  const uint32_t bit = pos & 31u;
+  const uint32_t rank = r.base + (uint32_t)__builtin_popcount(__builtin_amdgcn_ubfe(r.bits, 0u, bit));
+  return ((r.bits >> bit) & 1u) ? rank : none;
+}
+
+// LDS at a byte offset of the kernel's LDS block.  Kernels that have dynamic LDS
+// alone hold it from address 0: as an address space 3 pointer made from the
+// offset, a table at an offset known at compile time costs no address
+// arithmetic (through the extern array every read adds its base, 0, first).
+template <typename T>
+using LdsPtr = const __attribute__((address_space(3))) T*;
+template <typename T>
+__device__ __forceinline__ LdsPtr<T> lds_at(uint32_t offset) {
+  return (LdsPtr<T>)offset;
+}
+
 // ----------------------------------------------------------------------------
 // Lookup in a sorted key array behind a prefix table.
 //   bucket(key) = key >> shift; keys with that bucket live in
@@ -172,27 +195,6 @@ __device__ __forceinline__ int64_t bitmap_index(const IndexDev& ix, uint64_t key
   const uint32_t sub = w ? (uint32_t)(tail.y >> (9u * (w - 1u))) & 511u : 0u;
   const int64_t r = (int64_t)(tail.x + sub + (uint64_t)__builtin_popcountll(word & ((1ull << bit) - 1ull)));
   return ((word >> bit) & 1ull) ? r : -1;
-}
-
-// The same for a position below 2^32 in blocks of their own, the loads apart
-// from their use.
-struct RankBlock {
-  uint64_t word;
-  ulonglong2 tail;
-};
-__device__ __forceinline__ RankBlock rank_block(const uint64_t* blocks, uint32_t pos) {
-  const uint32_t j = __umulhi(pos >> 7, 0xAAAAAAABu) >> 1;
-  const uint64_t* blk = blocks + (uint64_t)j * 8u;
-  return RankBlock{blk[(pos - j * kRankBlockWords) >> 6], *(const ulonglong2*)(blk + 6)};
-}
-// Whether pos is a member; i: its rank, 0 if not.
-__device__ __forceinline__ bool rank_in(const RankBlock& r, uint32_t pos, uint64_t& i) {
-  const uint32_t j = __umulhi(pos >> 7, 0xAAAAAAABu) >> 1;
-  const uint32_t w = (pos - j * kRankBlockWords) >> 6, bit = pos & 63u;
-  const uint32_t sub = w ? (uint32_t)(r.tail.y >> (9u * (w - 1u))) & 511u : 0u;
-  const bool in = (r.word >> bit) & 1ull;
-  i = in ? r.tail.x + sub + (uint64_t)__builtin_popcountll(r.word & ((1ull << bit) - 1ull)) : 0ull;
-  return in;
 }
 
 __device__ __forceinline__ int64_t search_sorted(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ prefix,

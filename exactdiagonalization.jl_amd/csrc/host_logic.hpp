@@ -87,35 +87,54 @@ inline std::vector<int> win_positions(int Lx, int Ly) {
   return pos;
 }
 
-// Tables of Win<kWinPoint, L, L> for the variants in the mask (bit v), as bytes:
-// ranks, then masks.
-inline std::vector<unsigned char> win_point_table(int L, int variants) {
-  const int nv = 1 << (2 * L);
-  const uint32_t rm = (1u << L) - 1u;
-  auto rot = [&](uint32_t v, int a) { return ((v << a) | (v >> (L - a))) & rm; };
-  auto rev = [&](uint32_t v) {
+// Tables of Win<kWinPoint, L, L> for the variants in the mask (bit 0 of a variant
+// reverses the bits of the rows, bit 1 their order).
+inline std::vector<uint16_t> win_point_table(int L, int variants) {
+  const uint32_t nv = 1u << (2 * L), rm = (1u << L) - 1u;
+  auto framed = [&](uint32_t v, int f) {  // frame f = 8 reversed + rotation
     uint32_t o = 0;
-    for (int i = 0; i < L; ++i) o |= ((v >> i) & 1u) << (L - 1 - i);
+    for (int i = 0; i < L; ++i) o |= ((v >> i) & 1u) << (((f >> 3 ? L - 1 - i : i) + (f & 7)) % L);
     return o;
   };
-  std::vector<uint32_t> least((size_t)nv, ~0u), mask((size_t)nv, 0);
-  for (int w = 0; w < nv; ++w)
-    for (int v = 0; v < 4; ++v) {
-      if (!((variants >> v) & 1)) continue;
-      uint32_t hi = (uint32_t)w >> L, lo = (uint32_t)w & rm;
-      if (v & 2) std::swap(hi, lo);
-      if (v & 1) hi = rev(hi), lo = rev(lo);
+  // sets of frames (bit f), numbered as they occur
+  std::map<uint32_t, int> number{{0u, 0}};
+  std::vector<uint32_t> sets{0u};
+  auto class_of = [&](uint32_t set) {
+    auto it = number.emplace(set, (int)sets.size());
+    if (it.second) sets.push_back(set);
+    return it.first->second;
+  };
+  std::vector<uint16_t> tab((size_t)nv * 2 + ((size_t)kPointClasses << L) + kPointClasses, 0);
+  for (uint32_t w = 0; w < nv; ++w) {
+    uint32_t least = ~0u, set[2] = {0, 0};
+    for (int v = 0; v < 4; ++v)
       for (int a = 0; a < L; ++a) {
-        const uint32_t x = (rot(hi, a) << L) | rot(lo, a);
-        if (x < least[(size_t)w]) least[(size_t)w] = x, mask[(size_t)w] = 0;
-        if (x == least[(size_t)w]) mask[(size_t)w] |= 1u << (8 * v + a);
+        if (!((variants >> v) & 1)) continue;
+        const int f = 8 * (v & 1) + a;
+        const uint32_t hi = framed(v & 2 ? w & rm : w >> L, f), lo = framed(v & 2 ? w >> L : w & rm, f);
+        const uint32_t x = (hi << L) | lo;
+        if (x < least) least = x, set[0] = set[1] = 0;
+        if (x == least) set[v >> 1] |= 1u << f;
       }
+    tab[w] = (uint16_t)least;
+    tab[nv + w] = (uint16_t)(class_of(set[0]) | class_of(set[1]) << 8);
+  }
+  for (size_t c = 0; c < sets.size(); ++c) {  // (grows by the classes that the rows leave)
+    if (c >= (size_t)kPointClasses) return {};
+    const uint32_t set = sets[c];
+    for (uint32_t r = 0; r <= rm && set; ++r) {
+      uint32_t least = ~0u, left = 0;
+      for (int f = 0; f < 16; ++f) {
+        if (!((set >> f) & 1)) continue;
+        const uint32_t x = framed(r, f);
+        if (x < least) least = x, left = 0;
+        if (x == least) left |= 1u << f;
+      }
+      tab[2 * nv + (c << L) + r] = (uint16_t)((uint32_t)class_of(left) << L | least);
     }
-  std::vector<unsigned char> out((size_t)nv * 6);
-  uint16_t* rank = (uint16_t*)out.data();  // (the values themselves are below 2^12)
-  for (int w = 0; w < nv; ++w) rank[w] = (uint16_t)least[(size_t)w];
-  std::copy(mask.begin(), mask.end(), (uint32_t*)(out.data() + 2 * (size_t)nv));
-  return out;
+    tab[2 * nv + ((size_t)kPointClasses << L) + c] = (uint16_t)(set ? __builtin_ctz(set) : 0);
+  }
+  return tab;
 }
 
 // The bit permutation of a candidate code of Win<kWinPoint, L, L>.

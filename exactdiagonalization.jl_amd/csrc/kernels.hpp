@@ -29,8 +29,10 @@ hipError_t launch_mark_tops(const uint64_t* d_keys, int64_t dim, int shift, uint
 // x / sqrt(orbit) (the orbit factor of the images, X.scaled).
 hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, int64_t dim, const void* x,
                             const uint16_t* d_orbit, hipStream_t st);
-// positions of the keys in the spread X
-hipError_t launch_xmap_positions(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t* d_pos, hipStream_t st);
+// Ranks of the words' positions in the spread X, which ascend with the words:
+// n_blocks cleared blocks in.
+hipError_t launch_position_ranks(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t n_blocks,
+                                 RankBits* d_bits, hipStream_t st);
 // prefix[j] = lower_bound(keys, j << shift), j <= n_buckets
 hipError_t launch_build_prefix(const uint64_t* d_keys, int64_t dim, int shift, uint64_t n_buckets, uint32_t* d_prefix,
                                hipStream_t st);
@@ -168,8 +170,9 @@ struct WinOp {
   const uint32_t* rank_base;  // number of sector words with a smaller upper part
   int low_bits;
   uint32_t base_bytes;        // of rank_base, a multiple of 16
-  // point operations (values: x / sqrt(N) itself): rank blocks over the positions
-  const uint64_t* pos_blocks;
+  // point operations (values: x / sqrt(N) itself, 0 at the index none): ranks of the positions
+  const RankBits* pos_bits;
+  uint32_t none;
   int point_swap;
 };
 // Sectors of up to this many bits are ranked by two LDS tables (13 + 13 bits: 48 KiB)
@@ -185,10 +188,10 @@ inline uint32_t win_fixed_bytes(int kind, int Lx) {
 }
 
 // The same with point operations of an L x L torus, phases by candidate code
-// and the flip's four words included
+// and the flips' transposes included
 inline uint32_t win_point_bytes(int L, int n_lin, int n_chunk, int n_rest) {
-  return (6u << (2 * L)) + 512u * 16u + kXCodesBytesMax + 2u * 4096u + win_entries_bytes(n_lin, n_chunk, n_rest) +
-         24u * (uint32_t)(n_lin + n_rest + 1);
+  return 2u * ((2u << (2 * L)) + (kPointClasses << L) + kPointClasses) + 512u * 16u + kXCodesBytesMax + 2u * 4096u + win_entries_bytes(n_lin, n_chunk, n_rest) +
+         8u * (uint32_t)(n_lin + n_rest + 1);
 }
 
 enum Prec : int { kF64 = 0, kC128 = 1, kF32 = 2, kC64 = 3 };
@@ -237,7 +240,11 @@ struct AsmDev {
 // counts[r] = entries of row r (terms matching it)
 hipError_t launch_asm_count(const OpDev& op, uint32_t* d_counts, hipStream_t st);
 hipError_t launch_asm_fill(const OpDev& op, const AsmFillDev& a, hipStream_t st);
-// xt = x / sqrt(orbit) (orbit != nullptr), in precision prec
+// the same on a square torus with point operations (Win<kWinPoint>), the images
+// ranked by position
+hipError_t launch_asm_fill_point(const OpDev& op, const AsmFillDev& a, const XMapDev& X, const RankBits* pos_bits,
+                                 uint32_t none, hipStream_t st);
+// xt = x / sqrt(orbit) (orbit != nullptr), in precision prec; xt[dim] = 0
 hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, const void* x, void* xt, hipStream_t st);
 // y = (accumulate ? y : 0) + A x from the entries; xt = x scaled as above (x itself without orbits);
 // lanes = lanes per row (4, 8, 16 or 32), batch = entries per lane loaded together (4, 8 or 16)

@@ -623,11 +623,76 @@ __global__ __launch_bounds__(kMvBlock) void k_asm_fill(OpDev op, AsmFillDev a) {
   }
 }
 
-// xt[i] = x[i] / sqrt(N_i)
+// The same with the point operations of an L x L torus: canonical forms from the
+// window tables, images ranked by position (product.hpp, k_product_win), entries
+// written four at a time (one by one a wave's stores touch 64 lines each).  6x6
+// A1, 2.3e9 entries: 18.6 ms against 63.0 ms with the coset canonicaliser.
+template <int L, bool UNIT>
+__global__ __launch_bounds__(kMvBlock) void k_asm_fill_point(OpDev op, AsmFillDev a, XMapDev X,
+                                                             const RankBits* __restrict__ pos_bits, uint32_t none) {
+  using S = Win<kWinPoint, L, L>;
+  using W = typename S::W;
+  constexpr uint32_t at_codes = S::kTabBytes, at_colex = at_codes + kXCodesBytesMax, at_terms = at_colex + 2u * 4096u;
+  extern __shared__ unsigned char lds[];
+  lds_copy16(lds, op.g.point_tab, S::kTabBytes);
+  lds_copy16(lds + at_codes, X.topcode, xmap_codes_bytes(X.top_bits));
+  lds_copy16(lds + at_colex, X.colex, 2u * 4096u);
+  const MvTerms T = stage_mv_terms(op, lds, false, false);  // (op.mv_lds is at_terms here)
+  const uint32_t at_turned = at_terms + mv_layout(op.n_lin, op.n_chunk, op.n_rest, op.rest_paired).total;
+  W* turned = (W*)(lds + at_turned);
+  for (int t = threadIdx.x; t < op.n_lin + op.n_rest; t += kMvBlock) {
+    const W f = (W)op.ent[t].flip;
+    turned[t] = op.g.point_swap ? S::transposed(f) : f;
+  }
+  __syncthreads();
+  const int64_t row = (int64_t)blockIdx.x * kMvBlock + threadIdx.x;
+  if (row >= op.dim) return;
+  const W b = (W)op.rows[row];
+  const W bt = op.g.point_swap ? S::transposed(b) : b;
+  const LdsPtr<uint16_t> tab = lds_at<uint16_t>(0), codes = lds_at<uint16_t>(at_codes), colex = lds_at<uint16_t>(at_colex);
+  const uint32_t top_max = 1u << X.top_bits;
+  uint32_t* out = a.ent + a.rowptr[row];
+  uint32_t e[4] = {0, 0, 0, 0};
+  int n = 0;
+  const int n_seg = mv_segments(op);
+  for (int seg = 0; seg < n_seg; ++seg) {
+    int base;
+    uint64_t bits = mv_match(op, T, (uint64_t)b, seg, base);
+    while (bits) {
+      const int t = base + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      W s;
+      int code;
+      S::template canonical<!UNIT>(tab, b ^ (W)T.fa[2 * t], bt ^ turned[t], op.g.point_swap ? S::kWindows : S::kUpright,
+                                   s, code);
+      const uint32_t top = (uint32_t)(s >> X.top_shift), c = codes[top < top_max ? top : top_max];
+      const uint32_t hc = (c << X.hbits) | __builtin_amdgcn_ubfe((uint32_t)s, 12u, (uint32_t)X.hbits);
+      const uint32_t pos = __umul24(hc, 924u) + (uint32_t)colex[(uint32_t)s & 0xfffu];
+      const uint32_t idx = rank_of(pos_bits[pos >> 5], pos, none);
+      uint32_t cls = a.acls[t];
+      if (!UNIT && a.pcls) cls = 1u + (cls - 1u) * (uint32_t)a.n_ph + a.pcls[op.g.point_elem[code]];
+      e[0] = e[1];
+      e[1] = e[2];
+      e[2] = e[3];
+      e[3] = idx == none ? 0u : idx | (cls << a.col_bits);
+      if ((++n & 3) == 0) {
+        struct __attribute__((packed, aligned(4))) Four {
+          uint32_t v[4];
+        };
+        *(Four*)out = Four{{e[0], e[1], e[2], e[3]}};
+        out += 4;
+      }
+    }
+  }
+  for (int k = n & 3; k > 0; --k) *out++ = k == 3 ? e[1] : k == 2 ? e[2] : e[3];
+}
+
+// xt[i] = x[i] / sqrt(N_i), xt[dim] = 0 (the element of images outside the space)
 template <typename V>
 __global__ __launch_bounds__(kBlock) void k_asm_scale(int64_t dim, const uint16_t* __restrict__ orbit,
                                                       const V* __restrict__ x, V* __restrict__ xt) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i == dim) xt[i] = vzero<V>();
   if (i >= dim) return;
   using R = typename VT<V>::R;
   const double s = 1.0 / sqrt((double)orbit[i]);
@@ -795,9 +860,30 @@ hipError_t launch_asm_fill(const OpDev& op, const AsmFillDev& a, hipStream_t st)
   }
 }
 
+hipError_t launch_asm_fill_point(const OpDev& op, const AsmFillDev& a, const XMapDev& X, const RankBits* pos_bits,
+                                 uint32_t none, hipStream_t st) {
+  if (op.dim == 0) return hipSuccess;
+  const dim3 grid((unsigned)((op.dim + kMvBlock - 1) / kMvBlock));
+  OpDev o = op;
+#define EDHIP_FILL(L, U)                                                                                         \
+  {                                                                                                              \
+    o.mv_lds = Win<kWinPoint, L, L>::kTabBytes + kXCodesBytesMax + 2u * 4096u;                                   \
+    const uint32_t lds = o.mv_lds + mv_layout(o.n_lin, o.n_chunk, o.n_rest, o.rest_paired).total +               \
+                         8u * (uint32_t)(o.n_lin + o.n_rest);                                                    \
+    hipLaunchKernelGGL((k_asm_fill_point<L, U>), grid, dim3(kMvBlock), lds, st, o, a, X, pos_bits, none);        \
+    return hipGetLastError();                                                                                    \
+  }
+  if (op.g.Lx == 5 && op.g.unit_phases) EDHIP_FILL(5, true)
+  if (op.g.Lx == 5) EDHIP_FILL(5, false)
+  if (op.g.Lx == 6 && op.g.unit_phases) EDHIP_FILL(6, true)
+  if (op.g.Lx == 6) EDHIP_FILL(6, false)
+#undef EDHIP_FILL
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, const void* x, void* xt, hipStream_t st) {
   if (dim == 0) return hipSuccess;
-  dim3 grid((unsigned)((dim + kBlock - 1) / kBlock));
+  dim3 grid((unsigned)((dim + kBlock) / kBlock));
   switch (prec) {
     case kF64:
       hipLaunchKernelGGL(k_asm_scale<double>, grid, dim3(kBlock), 0, st, dim, d_orbit, (const double*)x, (double*)xt);

@@ -166,10 +166,10 @@ struct WinEntry {
   W flip;
   A amp;
 };
-// with point operations: the flip's words (Win<kWinPoint>)
+// with point operations: the flip's transpose too
 template <typename W, typename A>
 struct PointEntry {
-  W flip[4];
+  W flip, turned;
   A amp;
 };
 
@@ -192,8 +192,7 @@ struct PointEntry {
 // KIND = kWinPoint: translations and point operations.  These spaces are 8
 // times sparser in their words, so a spread would take a line per state (6x6
 // A1, FP64: 8.2 GB for 31.6M states): the position of the spread is ranked
-// through bits instead (blocks of 384 positions, 172 MB, which stay in the
-// last-level cache with x / sqrt(N) itself).
+// through bits instead (RankBits, 258 MB beside x / sqrt(N) itself).
 template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS, bool RANK = false>
 __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __restrict__ x, V* __restrict__ y) {
   using S = Win<KIND, LX, LY>;
@@ -226,18 +225,20 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   constexpr int n_chunk = S::kChain ? 0 : (((S::NB + 3) / 4 + 2) / 3) * 3;
   const int nch = n_chunk ? n_chunk : P.n_chunk;
   const uint32_t tab_bytes = (uint32_t)(((P.n_lin + 63) / 64) * nch) * 128u;
-  unsigned char* ptab = lds + (RANK ? rank_low + P.base_bytes : Lay::entries);
-  lds_copy16(ptab, P.lin_tab, tab_bytes);
-  E* ent = (E*)(ptab + tab_bytes);
+  const uint32_t at_ptab = RANK ? rank_low + P.base_bytes : Lay::entries;
+  lds_copy16(lds + at_ptab, P.lin_tab, tab_bytes);
   const int n_ent = P.n_lin + P.n_rest;
-  double* aim = (double*)(ent + ((n_ent + 1) & ~1));
-  uint64_t* mm = (uint64_t*)(aim + (CX ? n_ent : 0));
+  const uint32_t at_ent = at_ptab + tab_bytes;
+  const uint32_t at_aim = at_ent + (uint32_t)((n_ent + 1) & ~1) * (uint32_t)sizeof(E);
+  const uint32_t at_mm = at_aim + (CX ? 8u * (uint32_t)n_ent : 0u);
+  E* ent = (E*)(lds + at_ent);
+  double* aim = (double*)(lds + at_aim);
+  uint64_t* mm = (uint64_t*)(lds + at_mm);
 #pragma unroll 1
   for (int t = threadIdx.x; t < n_ent; t += kMvBlock) {
     const MvEntry e = P.ent[t];
     if constexpr (S::kPoint) {
-      S::words((W)e.flip, ent[t].flip);
-      ent[t].amp = (A)e.are;
+      ent[t] = E{(W)e.flip, P.point_swap ? S::transposed((W)e.flip) : (W)e.flip, (A)e.are};
     } else {
       ent[t] = E{(W)e.flip, (A)e.are};
     }
@@ -255,13 +256,13 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   const int sub = (int)threadIdx.x & ((1 << P.row_lanes) - 1);
   const W b = (W)P.rows[row];
 
-  const uint16_t* tab = (const uint16_t*)(lds + Lay::tab);
-  const uint16_t* codes = (const uint16_t*)(lds + Lay::codes);
-  const uint16_t* colex = (const uint16_t*)(lds + Lay::colex);
-  const double2* phase = (const double2*)(lds + Lay::phase);
+  const LdsPtr<uint16_t> tab = lds_at<uint16_t>(Lay::tab);
+  const LdsPtr<uint16_t> codes = lds_at<uint16_t>(Lay::codes);
+  const LdsPtr<uint16_t> colex = lds_at<uint16_t>(Lay::colex);
+  const LdsPtr<double> phase = lds_at<double>(Lay::phase);
   const uint32_t top_max = 1u << P.top_bits;
-  W bw[4];  // (point operations: the row's words)
-  if constexpr (S::kPoint) S::words(b, bw);
+  W turned = 0;  // (point operations: the row's transpose)
+  if constexpr (S::kPoint) turned = P.point_swap ? S::transposed(b) : b;
   auto position = [&](W s) {  // of the canonical word s in the spread
     const uint32_t top = (uint32_t)(s >> P.top_shift);
     const uint32_t c = codes[top < top_max ? top : top_max];
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   auto fetch = [&](W s) {  // x (/ sqrt(N)) of the canonical word s
     if constexpr (RANK) {
       const uint32_t lo = (uint32_t)s & ((1u << P.low_bits) - 1u);
-      return x[((const uint32_t*)(lds + rank_low))[s >> P.low_bits] + (uint32_t)((const uint16_t*)lds)[lo]];
+      return x[lds_at<uint32_t>(rank_low)[s >> P.low_bits] + (uint32_t)lds_at<uint16_t>(0)[lo]];
     }
     return ((const V*)P.values)[(uint64_t)position(s)];
   };
@@ -287,19 +288,19 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
           acc += (R)e.amp * xv;
         }
       } else {
-        vfma(acc, (R)e.amp, (R)aim[t], xv);
+        vfma(acc, (R)e.amp, (R)lds_at<double>(at_aim)[t], xv);
       }
     } else if constexpr (!CX) {
       if constexpr (kW32)
-        acc += e.amp * (float)phase[bit].x * xv;
+        acc += e.amp * (float)phase[2 * bit] * xv;
       else
-        acc += (R)(e.amp * phase[bit].x) * xv;
+        acc += (R)(e.amp * phase[2 * bit]) * xv;
     } else {
-      const double2 p = phase[bit];
+      const double2 p{phase[2 * bit], phase[2 * bit + 1]};
       if (P.real_amp) {
         vfma(acc, (R)(e.amp * p.x), (R)(e.amp * p.y), xv);
       } else {
-        const double ai = aim[t];
+        const double ai = lds_at<double>(at_aim)[t];
         vfma(acc, (R)(e.amp * p.x - ai * p.y), (R)(e.amp * p.y + ai * p.x), xv);
       }
     }
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
     int base;
     if (seg < n_ls) {  // parity entries (mv_match)
       base = 64 * seg;
-      const uint64_t* pt = (const uint64_t*)ptab + seg * (nch << 4);
+      const LdsPtr<uint64_t> pt = lds_at<uint64_t>(at_ptab) + seg * (nch << 4);
       if constexpr (n_chunk > 0) {
 #pragma unroll
         for (int k = 0; k < n_chunk; ++k)
@@ -351,27 +352,22 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
       V xv[NW];
 #pragma unroll
       for (int k = 0; k < NW; ++k) {
+        const uint32_t at = at_ent + __umul24((uint32_t)t[k], (uint32_t)sizeof(E));
+        e[k].flip = *lds_at<W>(at);
+        e[k].amp = *lds_at<A>(at + (uint32_t)offsetof(E, amp));
         if constexpr (S::kPoint)
-          e[k].amp = ent[t[k]].amp;
-        else
-          e[k] = ent[t[k]];
-        if constexpr (S::kPoint)
-          S::canonical(tab, bw, ent[t[k]].flip, P.point_swap, s[k], w[k]);
+          S::template canonical<!UNIT>(tab, b ^ e[k].flip, turned ^ *lds_at<W>(at + (uint32_t)sizeof(W)),
+                                       P.point_swap ? S::kWindows : S::kUpright, s[k], w[k]);
         else
           S::canonical(tab, b ^ e[k].flip, P.n_bits, s[k], w[k]);
       }
       if constexpr (S::kPoint) {  // both blocks, then both elements
         uint32_t at[NW];
-        RankBlock blk[NW];
+        RankBits r[NW];
 #pragma unroll
-        for (int k = 0; k < NW; ++k) blk[k] = rank_block(P.pos_blocks, at[k] = position(s[k]));
+        for (int k = 0; k < NW; ++k) r[k] = P.pos_bits[(at[k] = position(s[k])) >> 5];
 #pragma unroll
-        for (int k = 0; k < NW; ++k) {
-          uint64_t i;
-          const bool in = rank_in(blk[k], at[k], i);
-          xv[k] = ((const V*)P.values)[i];
-          if (!in) xv[k] = vzero<V>();
-        }
+        for (int k = 0; k < NW; ++k) xv[k] = ((const V*)P.values)[rank_of(r[k], at[k], P.none)];
       } else {
 #pragma unroll
         for (int k = 0; k < NW; ++k) xv[k] = fetch(s[k]);
@@ -399,7 +395,7 @@ hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, 
   const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
   const dim3 grid((unsigned)((lanes + kMvBlock - 1) / kMvBlock));
   const uint32_t dyn =
-      win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest) + (KIND == kWinPoint ? 24u * (uint32_t)(P.n_lin + P.n_rest + 1) : 0u);
+      win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest) + (KIND == kWinPoint ? 8u * (uint32_t)(P.n_lin + P.n_rest + 1) : 0u);
   // the column form only conjugates the phase
   constexpr bool kT = VT<V>::cx;
   if (unit)
@@ -427,7 +423,7 @@ hipError_t launch_win_v(const WinOp& P, int Lx, int Ly, int unit, int transpose,
 template <typename V>
 hipError_t launch_win_other(const WinOp& P, int Lx, int Ly, int unit, int transpose, const void* x, void* y,
                             hipStream_t st) {
-  if (P.pos_blocks) {
+  if (P.pos_bits) {
     if (Lx == 5 && Ly == 5) return launch_win_t<V, kWinPoint, 5, 5>(P, unit, transpose, x, y, st);
     if (Lx == 6 && Ly == 6) return launch_win_t<V, kWinPoint, 6, 6>(P, unit, transpose, x, y, st);
     return hipErrorInvalidValue;

@@ -333,12 +333,22 @@ __global__ __launch_bounds__(kBlock) void k_xmap_fill(XMapDev X, const uint64_t*
   ((V*)X.values)[pos] = v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_xmap_positions(XMapDev X, const uint64_t* __restrict__ keys, int64_t dim,
-                                                           uint64_t* __restrict__ pos) {
+// Ranks of the positions: a word sets its bit, and the first word of a block,
+// whose index is the rank below, the block's base.  (The bases of blocks without
+// words are never read.)  One pass over the words, no scan.
+__global__ __launch_bounds__(kBlock) void k_position_ranks(XMapDev X, const uint64_t* __restrict__ keys, int64_t dim,
+                                                           RankBits* __restrict__ blocks) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= dim) return;
   const uint64_t k = keys[i];
-  pos[i] = xmap_pos(X, X.colex, X.topcode[k >> X.top_shift], k);
+  const uint32_t pos = (uint32_t)xmap_pos(X, X.colex, X.topcode[k >> X.top_shift], k);
+  atomicOr(&blocks[pos >> 5].bits, 1u << (pos & 31u));
+  bool first = i == 0;
+  if (!first) {
+    const uint64_t p = keys[i - 1];
+    first = (uint32_t)xmap_pos(X, X.colex, X.topcode[p >> X.top_shift], p) >> 5 != pos >> 5;
+  }
+  if (first) blocks[pos >> 5].base = (uint32_t)i;
 }
 
 __global__ void k_u32_to_u64(const uint32_t* __restrict__ in, uint64_t* __restrict__ out, uint64_t n) {
@@ -467,10 +477,12 @@ hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, 
   return hipGetLastError();
 }
 
-hipError_t launch_xmap_positions(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t* d_pos,
-                                 hipStream_t st) {
+hipError_t launch_position_ranks(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t n_blocks,
+                                 RankBits* d_bits, hipStream_t st) {
   if (dim == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_xmap_positions, dim3(grid_for((uint64_t)dim)), dim3(kBlock), 0, st, X, d_keys, dim, d_pos);
+  hipError_t e = hipMemsetAsync(d_bits, 0, n_blocks * sizeof(RankBits), st);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_position_ranks, dim3(grid_for((uint64_t)dim)), dim3(kBlock), 0, st, X, d_keys, dim, d_bits);
   return hipGetLastError();
 }
 

@@ -91,7 +91,8 @@ struct Win {
   }
 
   // Candidates: bit 8 y + a for every (y, a) whose beginning is the smallest.
-  EDHIP_HD static C candidates(const uint16_t* tab, W b, int n) {
+  template <typename P>
+  EDHIP_HD static C candidates(P tab, W b, int n) {
     constexpr int NP = (NW + 1) / 2;
     constexpr uint32_t mask = (1u << MB) - 1u;
     C cand;
@@ -177,7 +178,8 @@ struct Win {
   EDHIP_HD static uint32_t next_row_of(W s) { return (uint32_t)(s >> ((LY - 1 - kNext) * LX)) & ((1u << LX) - 1u); }
 
   // The smallest image s of b and the first candidate that gives it.
-  EDHIP_HD static void canonical(const uint16_t* tab, W b, int n, W& s, int& bit) {
+  template <typename P>
+  EDHIP_HD static void canonical(P tab, W b, int n, W& s, int& bit) {
     C cand = candidates(tab, b, n);
     bit = ctz(cand);
     cand &= cand - 1;
@@ -206,23 +208,34 @@ struct Win {
 // of the pair window (row y, the row below) under the rows' reversal, their
 // exchange (the reflection in y shows the pair upside down) and both begin with
 // permuted copies of the same two rows, so that one table read gives the least
-// beginning over the four variants and all rotations: its rank (u16), and in a
-// second table, read for the windows that reach the least rank, the mask of
-// (variant, rotation) that reach it (8 bits per variant: bit 0 of the variant
-// reverses the rows' bits, bit 1 the order of the rows).  The other four point
+// beginning over these four variants and all rotations.  The other four point
 // operations are these after the transposition, whose windows are ranked
-// beside.  Each of these maps commutes with XOR, so the words of an image are
-// those of its row XORed with those of the flip, and nothing is permuted per
+// beside.  Each of these maps commutes with XOR, so the transposed image is
+// that of its row XORed with that of the flip, and nothing is permuted per
 // image.  (Bounding eight cosets one by one, each permuted by 4-bit tables:
 // 950 VALU instructions per image on the 6x6 A1 sector.)
 //
-// words: b, rows in reverse order, transposed, transposed and reversed.
+// The frames (reversed or not, rotation) that reach a window's least beginning
+// form one of few sets (cosets of subgroups of the dihedral group, at most 75),
+// its class.  A table over (class, row) gives the least image of the next row
+// over the frames of the class and the class of the frames that reach it: the
+// least image of a window is read off row by row, ties and all, with no
+// rotation (6x6 A1, FP64: 399 VALU instructions per image and 22.9 ms candidate
+// by candidate, 313 and 20.8 ms this way, 239 with every table read at a
+// compile-time LDS offset; what then bounds it is the L2 misses of its two
+// gathers, 0.5 per image, 7.2 TB/s).
+//
+// Tables (u16): least beginning by window, classes by window (upright in the
+// low byte, upside down in the high one, 0: none), next rows by class and row
+// (class << L | row), a frame of each class (bit 3: reversed; rotation).
+constexpr int kPointClasses = 80;
 template <int L, int L2>
 struct Win<kWinPoint, L, L2> {
   static constexpr bool kChain = false, kPoint = true;
   static constexpr int NB = L * L;
   static constexpr int kTab = 1 << (2 * L);
-  static constexpr uint32_t kTabBytes = 6u * kTab;  // ranks, then masks
+  static constexpr uint32_t kNext = 2 * kTab, kFrame = kNext + (kPointClasses << L);  // table offsets
+  static constexpr uint32_t kTabBytes = 2u * (kFrame + kPointClasses);
   using W = typename WinWord<(NB > 32)>::T;
   using T = Win<kWinPairs, L, L>;
 
@@ -237,99 +250,91 @@ struct Win<kWinPoint, L, L2> {
     }
     return out;
   }
-  EDHIP_HD static W rows_reversed(W b) {
-    W out = 0;
-#pragma unroll
-    for (int y = 0; y < L; ++y) out |= ((b >> (L * y)) & (((W)1 << L) - 1)) << (L * (L - 1 - y));
-    return out;
-  }
-  EDHIP_HD static uint32_t reversed32(uint32_t v) {
-#ifdef __HIP_DEVICE_COMPILE__
-    return __brev(v);
-#else
-    uint32_t o = 0;
-    for (int i = 0; i < 32; ++i) o |= ((v >> i) & 1u) << (31 - i);
-    return o;
-#endif
-  }
-  EDHIP_HD static W reversed(W b) {
-    if constexpr (NB > 32)
-      return (((W)reversed32((uint32_t)b) << 32) | reversed32((uint32_t)(b >> 32))) >> (64 - NB);
-    else
-      return reversed32(b) >> (32 - NB);
-  }
-  EDHIP_HD static void words(W b, W* out) {
-    out[0] = b;
-    out[1] = rows_reversed(b);
-    out[2] = transposed(b);
-    out[3] = rows_reversed(out[2]);
-  }
 
-  // The smallest image s of the word whose words are b[] ^ f[], and the code
-  // (transposed, variant, 8 y + a) << ... of the first candidate giving it:
-  // bit 8: transposed, bits 6 and 7: variant, then 8 y + a as for translations.
-  // swap: the group holds the transposed variants too.
-  EDHIP_HD static void canonical(const uint16_t* tab, const W* b, const W* f, int swap, W& s, int& code) {
-    const uint32_t* masks = (const uint32_t*)(tab + kTab);
-    const W w = b[0] ^ f[0], wt = b[2] ^ f[2];
-    uint32_t cand;  // bit y: window y of w, bit 16 + y: of its transpose
+  // The smallest image s of the word b, whose transpose is bt, and (CODE) the
+  // code of a candidate giving it: bit 8: transposed, bit 7: rows in reverse
+  // order, bit 6: their bits reversed, then 8 y + a as for translations.
+  // windows: the candidates to take, kWindows, or kUpright where the group
+  // transposes nothing (and bt is b).
+  static constexpr uint32_t kUpright = (1u << L) - 1u, kWindows = kUpright * 0x10001u;
+  template <bool CODE, typename P>
+  EDHIP_HD static void canonical(P tab, W b, W bt, uint32_t windows, W& s, int& code) {
+    constexpr int kRest = L * (L - 2);  // bits after the beginning, fewer than 32
+    uint32_t cand, lo;                  // bit y: window y of b, bit 16 + y: of bt
 #ifdef __HIP_DEVICE_COMPILE__
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     u16x2 p[L];
 #pragma unroll
-    for (int y = 0; y < L; ++y) {
-      p[y].x = tab[T::window(w, 0, y)];
-      p[y].y = swap ? tab[T::window(wt, 0, y)] : (uint16_t)0xffffu;
-    }
+    for (int y = 0; y < L; ++y) p[y] = u16x2{tab[T::window(b, 0, y)], tab[T::window(bt, 0, y)]};
     u16x2 m = p[0];
 #pragma unroll
     for (int y = 1; y < L; ++y) m = __builtin_elementwise_min(m, p[y]);
-    const uint16_t lo = m.x < m.y ? m.x : m.y;
+    lo = m.x < m.y ? m.x : m.y;
+    // a half is above the least (by less than 2^12) iff its sum with 0x7fff - least has bit 15
+    const uint32_t above = 0x7fff7fffu - lo * 0x10001u;
     uint32_t other = 0;
 #pragma unroll
-    for (int y = 0; y < L; ++y) {
-      const u16x2 d = __builtin_elementwise_min((u16x2)(p[y] - (u16x2){lo, lo}), (u16x2){1, 1});
-      other |= __builtin_bit_cast(uint32_t, d) << y;
-    }
-    cand = ~other & (((1u << L) - 1u) * 0x10001u);
+    for (int y = 0; y < L; ++y)
+      other = (other >> 1) | ((__builtin_bit_cast(uint32_t, p[y]) + above) & 0x80008000u);
+    cand = ~(other >> (16 - L)) & windows;
 #else
-    uint32_t p[2 * L], lo = 0xffffu;
+    uint32_t p[2 * L];
+    lo = 0xffffu;
     for (int y = 0; y < 2 * L; ++y) {
-      p[y] = y < L ? tab[T::window(w, 0, y)] : swap ? tab[T::window(wt, 0, y - L)] : 0xffffu;
+      p[y] = y < L ? tab[T::window(b, 0, y)] : tab[T::window(bt, 0, y - L)];
       lo = p[y] < lo ? p[y] : lo;
     }
     cand = 0;
     for (int y = 0; y < 2 * L; ++y)
       if (p[y] == lo) cand |= 1u << (y < L ? y : 16 + y - L);
+    cand &= windows;
 #endif
-    s = (W)~(W)0;
-    code = 0;
-    uint32_t mask = 0;
+    uint32_t best = ~0u;
+    uint32_t down = 0;  // class of the window's upside-down frames, to be taken next
+    uint32_t rows = 0;
     int q = 0;
-    W src = 0;
+    code = 0;
     do {
-      if (!mask) {
+      uint32_t c = down;
+      int at = 0, step = L;  // upside down: the rows from y + 1 up
+      if (!down) {
         q = T::ctz(cand);
         cand &= cand - 1;
-        src = q >= 16 ? wt : w;
-        mask = masks[T::window(src, 0, q & 15)];
+        const W w = q >= 16 ? bt : b;
+        const int n = ((q & 15) + 1) * L;  // row y to the top: the rows y - 2 down and y + 1 up are the low ones
+        const W t = (W)(w >> n) | (W)(w << (NB - n));
+        rows = (uint32_t)t;
+        const uint32_t e = tab[kTab + ((uint32_t)(t >> kRest) & (uint32_t)(kTab - 1))];
+        c = e & 255u;
+        down = e >> 8;
+        at = kRest - L;
+        step = -L;
+        if (c == 0) {
+          c = down;
+          at = 0;
+          step = L;
+          down = 0;
+        }
+      } else {
+        down = 0;
       }
-      const int r = T::ctz(mask), a = r & 7, v = r >> 3, y = q & 15;
-      mask &= mask - 1;
-      // the row after the beginning, against that of the least image so far
-      const int yn = v < 2 ? (y >= 2 ? y - 2 : y + L - 2) : (y + 1 < L ? y + 1 : 0);
-      uint32_t n = (uint32_t)(src >> (uint32_t)(yn * L)) & ((1u << L) - 1u);
-      n = (v & 1) ? reversed32(n) >> (32 - L) : n;
-      n = ((n << a) | (n >> (L - a))) & ((1u << L) - 1u);
-      if (n > ((uint32_t)(s >> ((L - 3) * L)) & ((1u << L) - 1u))) continue;
-      const int g = (q >= 16 ? 2 : 0) | ((v ^ (v >> 1)) & 1);
-      W u = (g & 1) ? ((g & 2) ? b[3] : b[1]) ^ f[g] : src;
-      if (v & 1) u = reversed(u);
-      const int bit = 8 * (v < 2 ? y : (y ? L - y : 0)) + a;
-      const W t = T::image(u, 0, bit);
-      code = t < s ? (q >= 16 ? 256 : 0) + 64 * v + bit : code;
-      s = t < s ? t : s;
-    } while (mask | cand);
+      uint32_t e = c << L, rest = 0;
+      constexpr uint32_t rm = (1u << L) - 1u;
+#pragma unroll
+      for (int k = 0; k < L - 2; ++k) {
+        e = tab[kNext + (e | ((rows >> at) & rm))];
+        rest = (rest << L) | (e & rm);
+        e &= ~rm;
+        at += step;
+      }
+      if constexpr (CODE)
+        if (rest < best) {
+          const int y = q & 15, f = tab[kFrame + (e >> L)];
+          code = (q >= 16 ? 256 : 0) + (step > 0 ? 128 + 8 * (y ? L - y : 0) : 8 * y) + 8 * (f & 8) + (f & 7);
+        }
+      best = rest < best ? rest : best;
+    } while (down | cand);
+    s = ((W)lo << kRest) | best;
   }
 };
 
@@ -344,7 +349,8 @@ struct Win<kWinNone, LX, LY> {
   static constexpr int NB = LX;
   static constexpr uint32_t kTabBytes = 0;
   using W = typename WinWord<(LX > 32)>::T;
-  EDHIP_HD static void canonical(const uint16_t*, W b, int, W& s, int& bit) {
+  template <typename P>
+  EDHIP_HD static void canonical(P, W b, int, W& s, int& bit) {
     s = b;
     bit = 0;
   }

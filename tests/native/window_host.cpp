@@ -59,10 +59,8 @@ static int check_point(int variants, int swap, std::mt19937_64& rng) {
   using S = Win<kWinPoint, L, L>;
   using W = typename S::W;
   const int n = L * L;
-  const std::vector<unsigned char> bytes = win_point_table(L, variants);
-  if (bytes.size() != S::kTabBytes) return std::printf("point %d: table size\n", L), 1;
-  std::vector<uint64_t> aligned(bytes.size() / 8);
-  std::copy(bytes.begin(), bytes.end(), (unsigned char*)aligned.data());
+  const std::vector<uint16_t> tab = win_point_table(L, variants);
+  if (2 * tab.size() != S::kTabBytes) return std::printf("point %d: table size\n", L), 1;
   std::vector<std::vector<int32_t>> perms;
   for (int code = 0; code < 512; ++code)
     if ((code & 7) < L && ((code >> 3) & 7) < L && ((variants >> ((code >> 6) & 3)) & 1) && (swap || code < 256))
@@ -79,14 +77,12 @@ static int check_point(int variants, int swap, std::mt19937_64& rng) {
     }
     if (k < 2) row = k ? full : 0;
     const uint64_t flip = (k % 3) ? (1ull << (rng() % n)) ^ (1ull << (rng() % n)) : 0;
-    W b[4], f[4];
-    S::words((W)row, b);
-    S::words((W)flip, f);
     uint64_t want = ~0ull;
     for (const auto& p : perms) want = std::min(want, permuted(row ^ flip, p));
     W s;
     int code;
-    S::canonical((const uint16_t*)aligned.data(), b, f, swap, s, code);
+    const W b = (W)(row ^ flip), bt = swap ? S::transposed((W)row) ^ S::transposed((W)flip) : b;
+    S::template canonical<true>(tab.data(), b, bt, swap ? S::kWindows : S::kUpright, s, code);
     if ((uint64_t)s != want || permuted(row ^ flip, win_point_perm(L, code)) != want)
       return std::printf("point %d, variants %d, swap %d: %llx -> %llx (code %d), not %llx\n", L, variants, swap,
                          (unsigned long long)(row ^ flip), (unsigned long long)s, code, (unsigned long long)want), 1;

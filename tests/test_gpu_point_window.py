@@ -44,3 +44,24 @@ def test_point_window_vs_general(ed, L, k, point, away, hop):
             ed.mul_(z, opr, x) if form == "row" else ed.mul_(z, x, opr)
             assert torch.linalg.norm(y - z) <= TOL[dt] * torch.linalg.norm(z), (dt, form)
     opr.set_strategy()
+
+
+@pytest.mark.parametrize("L,k,point,away", GROUPS)
+def test_assembled_point_rows(ed, L, k, point, away):
+    """The rows assembled through the window tables: the same products."""
+    hs, _ = ed.spin_half_system(L * L)
+    near, far = ed.square_bonds(L, L)
+    H = sum((ed.heisenberg_bond(hs, i, j, 1.0, 1.1) for i, j in near), ed.NullOperator())
+    H = H + sum((ed.heisenberg_bond(hs, i, j, 0.4) for i, j in far), ed.NullOperator())
+    space = ed.represent(ed.HilbertSpaceSector(hs, L * L % 2 + 2 * away))
+    opr = ed.represent(ed.symmetry_reduce(space, ed.SquareSpaceIrrep(L, k, point)), ed.simplify(H))
+    g = torch.Generator(device="cuda").manual_seed(L)
+    for dt in [torch.complex128, torch.complex64] if opr.is_complex else list(TOL):
+        x = torch.randn(opr.dimension, dtype=dt, device="cuda", generator=g)
+        y, z = torch.empty_like(x), torch.empty_like(x)
+        opr.set_strategy("assembled")
+        ed.mul_(y, opr, x)
+        opr.set_strategy("terms", "search")
+        ed.mul_(z, opr, x)
+        assert torch.linalg.norm(y - z) <= TOL[dt] * torch.linalg.norm(z), dt
+    opr.set_strategy()
