@@ -1008,6 +1008,9 @@ struct edhip_op {
   int64_t kt_n = 0;
   // assembled rows of the row form (strategy 3), built on first use
   bool asm_built = false;
+  DevBuf ex_steps, ex_lists, ex_sums;  // the term pass by rank (expect_by_rank)
+  int ex_rank = 0;                     // 0 not looked at, 1 by rank, -1 not
+  ExpectRank ex_rank_dev{};
   DevBuf asm_rowptr, asm_ent, asm_w, asm_acls, asm_pcls, asm_xt;
   AsmDev asm_dev{};
   uint64_t asm_nnz = 0;
@@ -3018,6 +3021,67 @@ int edhip_lanczos(edhip_op* op, const edhip_lanczos_opts* opts, double* evals, v
 }
 
 // ---- differentiation ------------------------------------------------------------------
+// The term pass by rank: sectors of one popcount without a group, up to
+// kRankBits bits, terms that keep the popcount, and diagonal terms that test at
+// most one lower bit beside upper ones.
+static bool expect_by_rank(edhip_op* op, ExpectRank& E) {
+  const edhip_space* sp = op->space;
+  if (op->strat_lookup > 1) return false;
+  if (op->ex_rank == 0) {
+    op->ex_rank = -1;
+    if (!op->keeps_popcount || sp->dim == 0 || sp->n_bits < 12 || !sp->ensure_rank_tables())
+      return false;
+    const OpDev& d = op->dev_row;
+    const int lb = sp->rank_low_bits;
+    const uint64_t lmask = (1ull << lb) - 1;
+    for (int64_t t : op->diag_ids) {
+      const uint64_t low = op->mask[t] & lmask;
+      if ((op->mask[t] >> lb) && (low & (low - 1))) return false;
+      if (op->row[t] & ~op->mask[t]) return false;
+    }
+    std::vector<ExpectStep> steps;
+    for (size_t j = 0; j < op->off_ids.size(); ++j) {
+      const int64_t t = op->off_ids[j];
+      const uint32_t mask = (uint32_t)op->mask[t], match = (uint32_t)op->row[t], flip = match ^ (uint32_t)op->col[t];
+      ExpectStep s{mask, {match, ~0u}, flip, {(int32_t)j, -1}};
+      if (j + 1 < op->off_ids.size()) {
+        const int64_t u = op->off_ids[j + 1];
+        if (op->mask[u] == op->mask[t] && (op->row[u] ^ op->col[u]) == (op->row[t] ^ op->col[t]) &&
+            op->row[u] != op->row[t]) {
+          s.match[1] = (uint32_t)op->row[u];
+          s.term[1] = (int32_t)++j;
+        }
+      }
+      steps.push_back(s);
+    }
+    while (steps.size() % kExpectWindow) steps.push_back(ExpectStep{0u, {~0u, ~0u}, 0u, {-1, -1}});
+    const int ub = std::max(0, sp->n_bits - lb);
+    const PopLists up = pop_lists(ub), lo = pop_lists(lb);
+    std::vector<int32_t> lists;
+    auto put = [&](const std::vector<int32_t>& v) {
+      const int32_t at = (int32_t)lists.size();
+      lists.insert(lists.end(), v.begin(), v.end());
+      return at;
+    };
+    std::vector<int32_t> items;
+    for (int p = 0; p <= lb; ++p)
+      for (int32_t k = 0; k < lo.off[(size_t)p + 1] - lo.off[(size_t)p]; k += 64) items.insert(items.end(), {p, k});
+    const int32_t at[5] = {put(up.list), put(up.off), put(lo.list), put(lo.off), put(items)};
+    hipStream_t st = op->ctx->stream;
+    upload(op->ex_steps, steps, st);
+    upload(op->ex_lists, lists, st);
+    op->ctx->sync();
+    const int32_t* l = op->ex_lists.as<int32_t>();
+    op->ex_rank_dev = ExpectRank{d.rows, sp->rank_low.as<uint16_t>(), sp->rank_base.as<uint32_t>(),
+                                 op->ex_steps.as<ExpectStep>(), l + at[0], l + at[1], l + at[2], l + at[3], l + at[4],
+                                 (uint32_t)sp->rank_base.bytes, lb, ub, 1 << ub, sp->popcounts[0], (int)op->off_ids.size(),
+                                 (int)steps.size(), (int)items.size() / 2};
+    op->ex_rank = 1;
+  }
+  E = op->ex_rank_dev;
+  return op->ex_rank == 1;
+}
+
 int edhip_term_expect(edhip_op* op, int prec, const void* phi, const void* psi, double* out) {
   if (!op || !out) return EDHIP_ERR_ARGUMENT;
   return guarded(op->ctx, [&] {
@@ -3030,14 +3094,26 @@ int edhip_term_expect(edhip_op* op, int prec, const void* phi, const void* psi, 
     const int nc = prec_is_complex(prec) ? 2 : 1;
     if (term_expect_window(op->dev_row, nc) < 1)
       fail(EDHIP_ERR_ARGUMENT, "operator and symmetry tables leave no LDS room for the fused expectation kernel");
+    OpDev d = op->dev_row;
+    ExpectRank E{};
+    const bool ranked = expect_by_rank(op, E);
+    if (ranked) {
+      const size_t x = (size_t)E.n_upper * (1 + 2 * E.low_bits) * 2, q = ((size_t)kExpectSplits << E.low_bits) * 2;
+      op->ex_sums.ensure((x + q) * 8);
+    }
     // psi of the images from its spread, as the products read x, where its
     // code table leaves LDS room for the bins
-    OpDev d = op->dev_row;
-    if (attach_spread(op, prec, d, d.codes_lds, psi, op->ctx->stream) && term_expect_window(d, nc) < 1) d.xm = XMapDev{};
+    if (!ranked && attach_spread(op, prec, d, d.codes_lds, psi, op->ctx->stream) && term_expect_window(d, nc) < 1) d.xm = XMapDev{};
     edhip_ctx* ctx = op->ctx;
     if (ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(ctx->ev[14], ctx->stream));
-    HIP_OR_THROW(launch_term_expect(d, prec, phi, psi, op->ex_partial.as<double>(), nb, op->ex_out.as<double>(),
-                                    ctx->stream));
+    if (ranked) {
+      double* X = op->ex_sums.as<double>();
+      HIP_OR_THROW(launch_term_expect_rank(E, d, prec, phi, psi, X, X + (size_t)E.n_upper * (1 + 2 * E.low_bits) * 2,
+                                           op->ex_partial.as<double>(), op->ex_out.as<double>(), ctx->stream));
+    } else {
+      HIP_OR_THROW(launch_term_expect(d, prec, phi, psi, op->ex_partial.as<double>(), nb, op->ex_out.as<double>(),
+                                      ctx->stream));
+    }
     if (ctx->kernel_timing) {
       HIP_OR_THROW(hipEventRecord(ctx->ev[15], ctx->stream));
       HIP_OR_THROW(hipEventSynchronize(ctx->ev[15]));

@@ -45,6 +45,21 @@ inline RankTables rank_tables(int n, int pop) {
   return T;
 }
 
+// The values of n bits by popcount, ascending, and the offset of each popcount.
+struct PopLists {
+  std::vector<int32_t> list, off;
+};
+inline PopLists pop_lists(int n) {
+  PopLists P;
+  for (int p = 0; p <= n; ++p) {
+    P.off.push_back((int32_t)P.list.size());
+    for (int32_t w = 0; w < (1 << n); ++w)
+      if (__builtin_popcount((unsigned)w) == p) P.list.push_back(w);
+  }
+  P.off.push_back((int32_t)P.list.size());
+  return P;
+}
+
 // Window table of an Lx x Ly torus (window.hpp): entry = rank << mask bits | mask.
 inline std::vector<uint16_t> win_table(int Lx, int Ly) {
   const int kind = win_kind(Lx, Ly);

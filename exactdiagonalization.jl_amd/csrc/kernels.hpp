@@ -285,6 +285,41 @@ int64_t term_expect_blocks(const OpDev& op);
 // components (0: the tables leave no LDS room)
 int64_t term_expect_scratch_rows(const OpDev& op);
 
+// The same on sectors that are ranked by two tables (expect.hip).  A step is one
+// off-diagonal term, or two that share mask and flip (term[1] < 0: one; a match of
+// all ones never occurs).
+struct ExpectStep {
+  uint32_t mask, match[2], flip;
+  int32_t term[2];
+};
+struct ExpectRank {
+  const uint64_t* rows;
+  const uint16_t* rank_low;   // as in WinOp
+  const uint32_t* rank_base;
+  const ExpectStep* steps;    // whole windows
+  // upper and lower parts by popcount: lists and their offsets; items: pairs
+  // (popcount, first) of every 64 lower parts
+  const int32_t *up_list, *up_off, *lo_list, *lo_off, *items;
+  uint32_t base_bytes;
+  int low_bits, upper_bits, n_upper, pop, n_off, n_steps, n_items;
+};
+constexpr int kExpectWindow = 6;  // steps per window (real vectors; half of it for complex ones)
+constexpr int kExpectSplits = 16;
+// Blocks of the steps' kernel per window, each with a row of 2 n_off partial sums:
+// all windows together three blocks per CU, which the chip holds at once (4x6 XXZ,
+// 8 windows: 110 us with 96 blocks, 124 with 64, 122 with 128, 140 with 384).
+inline int64_t expect_rank_blocks(int64_t dim, int windows) {
+  const int64_t n = (dim + 511) / 512, most = windows > 24 ? 32 : 768 / (windows < 1 ? 1 : windows);
+  return n < 1 ? 1 : n > most ? most : n;
+}
+// X: n_upper (1 + 2 low_bits) sums, Q: kExpectSplits 2^low_bits, each 2 doubles;
+// d_partial: expect_rank_blocks and their chunks (blocks / 64, rounded up) of 2 n_off doubles
+hipError_t launch_term_expect_rank(const ExpectRank& E, const OpDev& op, int prec, const void* phi, const void* psi,
+                                   double* X, double* Q, double* d_partial, double* d_out, hipStream_t st);
+// sums of the rows of d_partial (n_blocks x width), in a fixed order, by way of
+// the chunk sums behind them
+hipError_t launch_expect_reduce(double* d_partial, int64_t n_blocks, int width, double* d_out, hipStream_t st);
+
 // Fixed device scratch of the allocation-free term pass (one array per GPU,
 // held until the process ends): room for the per-block partial sums and the
 // result of at most kNoAllocMaxTerms terms.  term_expect_noalloc_setup runs

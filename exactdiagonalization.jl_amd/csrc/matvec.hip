@@ -415,6 +415,7 @@ __global__ __launch_bounds__(64) void k_sum_parts_chunks(const double* __restric
   const int64_t p0 = (int64_t)blockIdx.y * 64;
   const int64_t p1 = p0 + 64 < n_parts ? p0 + 64 : n_parts;
   double s = 0.0;
+#pragma unroll 16
   for (int64_t p = p0; p < p1; ++p) s += partial[p * width + col];
   inter[(int64_t)blockIdx.y * width + col] = s;
 }
@@ -424,6 +425,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce_partials(const double* __rest
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= width) return;
   double s = 0.0;
+#pragma unroll 8
   for (int64_t b = 0; b < n_blocks; ++b) s += partial[b * width + i];
   out[i] = s;
 }
@@ -532,17 +534,7 @@ hipError_t launch_expect_t(const OpDev& op, const void* phi, const void* psi, do
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  // fixed-order reduction of the per-block rows: chunks of 64 rows, then the chunks
-  const int width = n_terms * 2;
-  const int64_t n_chunks = (n_blocks + 63) / 64;
-  double* inter = d_partial + n_blocks * width;
-  hipLaunchKernelGGL(k_sum_parts_chunks, dim3((unsigned)((width + 63) / 64), (unsigned)n_chunks), dim3(64), 0, st,
-                     d_partial, n_blocks, width, inter);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((width + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, inter,
-                     n_chunks, width, d_out);
-  return hipGetLastError();
+  return launch_expect_reduce(d_partial, n_blocks, n_terms * 2, d_out, st);
 }
 
 template <typename V>
@@ -1041,6 +1033,19 @@ int term_expect_window(const OpDev& op, int nc) {
   const int n_terms = op.n_diag + op.n_off;
   if (nw < 1) return 0;
   return nw < n_terms ? (int)nw : n_terms;
+}
+
+// fixed-order reduction of the per-block rows: chunks of 64 rows, then the chunks
+hipError_t launch_expect_reduce(double* d_partial, int64_t n_blocks, int width, double* d_out, hipStream_t st) {
+  const int64_t n_chunks = (n_blocks + 63) / 64;
+  double* inter = d_partial + n_blocks * width;
+  hipLaunchKernelGGL(k_sum_parts_chunks, dim3((unsigned)((width + 63) / 64), (unsigned)n_chunks), dim3(64), 0, st,
+                     d_partial, n_blocks, width, inter);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_reduce_partials, dim3((unsigned)((width + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, inter,
+                     n_chunks, width, d_out);
+  return hipGetLastError();
 }
 
 int64_t term_expect_blocks(const OpDev& op) {
