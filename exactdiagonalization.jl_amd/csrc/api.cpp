@@ -482,16 +482,8 @@ struct edhip_space {
     const uint64_t bytes = n_blocks * 64;
     if (bytes > std::max<uint64_t>(kBitmapMaxRatio * (uint64_t)dim * 8ull, 1ull << 20)) return false;
     bitmap.alloc(bytes);
-    HIP_OR_THROW(hipMemsetAsync(bitmap.p, 0, bytes, ctx->stream));
-    DevBuf totals, base, tmp;
-    totals.alloc(n_blocks * 4);
-    base.alloc(n_blocks * 8);
-    size_t tb = 0;
-    HIP_OR_THROW(launch_bitmap_build(keys.as<uint64_t>(), dim, bitmap.as<uint64_t>(), n_blocks, totals.as<uint32_t>(),
-                                     base.as<uint64_t>(), nullptr, tb, ctx->stream));
-    tmp.alloc(tb);
-    HIP_OR_THROW(launch_bitmap_build(keys.as<uint64_t>(), dim, bitmap.as<uint64_t>(), n_blocks, totals.as<uint32_t>(),
-                                     base.as<uint64_t>(), tmp.p, tb, ctx->stream));
+    HIP_OR_THROW(launch_rank_blocks(keys.as<uint64_t>(), dim, prefix.as<uint32_t>(), shift, n_buckets,
+                                    bitmap.as<uint64_t>(), n_blocks, ctx->stream));
     ctx->sync();
     bm_bits = K;
     return true;
@@ -1258,6 +1250,34 @@ bool ensure_diag(edhip_op* op) {
   op->diag_im.p = pi;
   op->diag_im.bytes = pi ? (size_t)D * 8 : 0;
   const OpDev& d = op->dev_row;
+  if (!cx) {
+    std::vector<uint64_t> mask, match;
+    std::vector<double> amp;
+    for (int64_t t : op->diag_ids) {
+      mask.push_back(op->mask[t]);
+      match.push_back(op->row[t]);
+      amp.push_back(op->are[t]);
+    }
+    const DiagSplit D = diag_split(mask, match, amp);
+    std::vector<DiagSet> sets;
+    for (size_t i = 0; i < D.sets.size(); ++i) sets.push_back(DiagSet{D.sets[i], D.coefs[i]});
+    std::vector<DiagTerm> rest;
+    for (size_t t : D.rest) rest.push_back(DiagTerm{mask[t], match[t], amp[t], 0.0});
+    const std::vector<uint64_t> tab = mv_tables(D.entries, op->space->n_bits);
+    if (tab.size() * 8 <= 32 * 1024 && D.rest.size() < op->diag_ids.size()) {
+      hipStream_t st = op->ctx->stream;
+      DevBuf tab_d, sets_d, first_d, rest_d;
+      upload(tab_d, tab, st);
+      upload(sets_d, sets, st);
+      upload(first_d, D.first, st);
+      upload(rest_d, rest, st);
+      const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
+                         D.constant, (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
+      HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
+      op->ctx->sync();
+      return true;
+    }
+  }
   HIP_OR_THROW(launch_diag_values(d, op->diag_re.as<double>(), op->diag_im.as<double>(), op->ctx->stream));
   return true;
 }

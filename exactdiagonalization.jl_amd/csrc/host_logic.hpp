@@ -260,6 +260,59 @@ inline std::vector<uint64_t> mv_tables(const MvSplit& S, int nb) {
   return tab;
 }
 
+// A diagonal operator with real amplitudes, sum of a_t [b & mask_t == match_t], by
+// parities: masks of one or two sites whose summed amplitudes depend on the
+// parity of the masked bits alone, m + h for even and m - h for odd, give m to a
+// constant and an entry (parity mask, h), the others stay terms.  The entries of
+// one h then sum to h (even ones - odd ones): for exchange and fields, whose m
+// is 0, a product with an integer and no cancellation.
+struct DiagSplit {
+  double constant = 0.0;
+  MvSplit entries;            // q, c and one lin entry (are: h) each
+  std::vector<size_t> rest;   // terms left
+  std::vector<uint64_t> sets; // per segment and coefficient: the entries' bits
+  std::vector<double> coefs;
+  std::vector<int32_t> first; // offsets of the segments
+};
+inline DiagSplit diag_split(const std::vector<uint64_t>& mask, const std::vector<uint64_t>& match,
+                            const std::vector<double>& amp) {
+  DiagSplit D;
+  std::map<uint64_t, std::vector<size_t>> by_mask;
+  for (size_t t = 0; t < mask.size(); ++t) by_mask[mask[t]].push_back(t);
+  long double constant = 0.0L;
+  std::vector<std::pair<double, uint64_t>> found;  // h, parity mask
+  for (const auto& [m, ts] : by_mask) {
+    const uint64_t lowest = m & (~m + 1);
+    double f[4] = {0, 0, 0, 0};  // by (upper bit, lower bit)
+    for (size_t t : ts) f[((match[t] & lowest) ? 1 : 0) + ((match[t] & m & ~lowest) ? 2 : 0)] += amp[t];
+    const int n = __builtin_popcountll(m);
+    if (n == 0) {
+      constant += f[0];
+    } else if (n == 1 || (n == 2 && f[0] == f[3] && f[1] == f[2])) {
+      constant += 0.5L * ((long double)f[0] + f[1]);
+      if (f[1] != f[0]) found.emplace_back(0.5 * (f[0] - f[1]), m);
+    } else {
+      D.rest.insert(D.rest.end(), ts.begin(), ts.end());
+    }
+  }
+  D.constant = (double)constant;
+  std::sort(D.rest.begin(), D.rest.end());
+  std::sort(found.begin(), found.end());  // equal coefficients together
+  for (size_t e = 0; e < found.size(); ++e) {
+    if (e % 64 == 0) D.first.push_back((int32_t)D.sets.size());
+    if (e % 64 == 0 || found[e].first != D.coefs.back()) {
+      D.sets.push_back(0);
+      D.coefs.push_back(found[e].first);
+    }
+    D.sets.back() |= 1ull << (e % 64);
+    D.entries.q.push_back(found[e].second);
+    D.entries.c.push_back(0);
+    D.entries.lin.push_back(MvEntry{0, found[e].first, 0.0});
+  }
+  D.first.push_back((int32_t)D.sets.size());
+  return D;
+}
+
 // Householder reduction of a dense symmetric matrix (row-major, n x n) to
 // tridiagonal form A = Q T Q^T; returns d (diagonal), e (e[i] = T[i][i+1]).
 inline void householder_tridiag(int n, std::vector<double>& A, std::vector<double>& Q, std::vector<double>& d,

@@ -71,12 +71,10 @@ hipError_t launch_vec_reduce(const uint64_t* d_reps, const uint16_t* d_orbit, in
                              const GroupLdsLayout& lay, const IndexDev& parent_index, int prec, const void* d_large,
                              void* d_small, hipStream_t st);
 
-// Blocked rank index over the words [0, 384 n_blocks) (zeroed blocks in,
-// layout as in IndexDev); d_totals (u32) and d_base (u64) hold n_blocks
-// entries of scratch.  Two-phase: call with d_tmp == nullptr to size the
-// scan's scratch.
-hipError_t launch_bitmap_build(const uint64_t* d_keys, int64_t dim, uint64_t* d_blocks, uint64_t n_blocks,
-                               uint32_t* d_totals, uint64_t* d_base, void* d_tmp, size_t& tmp_bytes, hipStream_t st);
+// Blocked rank index over the words [0, 384 n_blocks), layout as in IndexDev, from
+// the sorted keys and their prefix table.
+hipError_t launch_rank_blocks(const uint64_t* d_keys, int64_t dim, const uint32_t* d_prefix, int shift,
+                              uint64_t n_buckets, uint64_t* d_blocks, uint64_t n_blocks, hipStream_t st);
 hipError_t exclusive_scan_u32_to_u64(const uint32_t* d_in, uint64_t* d_out, uint64_t n, void* d_tmp, size_t& tmp_bytes,
                                      hipStream_t st);
 hipError_t exclusive_scan_i64(const int64_t* d_in, int64_t* d_out, uint64_t n, void* d_tmp, size_t& tmp_bytes,
@@ -254,6 +252,23 @@ hipError_t launch_asm_spmv(const OpDev& op, const AsmDev& a, int prec, int lanes
 // Diagonal element of every row: re[r] (+ i im[r] when im != nullptr) = sum of
 // the amplitudes of the diagonal terms that match row r.
 hipError_t launch_diag_values(const OpDev& op, double* d_re, double* d_im, hipStream_t st);
+
+// The same for real amplitudes by parities (DiagSplit): constant + the coefficient
+// of every set of entries (mask within its segment) times the number of them whose
+// parity is even less that of those whose is odd + the terms left (rest).
+struct DiagSet {
+  uint64_t mask;
+  double coef;
+};
+struct DiagParity {
+  const uint64_t* tab;   // as OpDev::lin_tab, n_seg segments of n_chunk chunks
+  const DiagSet* sets;   // by segment
+  const int32_t* first;  // n_seg + 1 offsets into sets
+  const DiagTerm* rest;
+  double constant;
+  int n_seg, n_chunk, n_rest;
+};
+hipError_t launch_diag_parity(const DiagParity& P, const uint64_t* d_rows, int64_t dim, double* d_re, hipStream_t st);
 
 // Total number of off-diagonal images the row form generates (atomic u64 add).
 hipError_t launch_count_images(const OpDev& op, unsigned long long* d_total, hipStream_t st);
