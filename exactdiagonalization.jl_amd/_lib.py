@@ -156,6 +156,7 @@ SIGNATURES = {
     "edhip_op_assembled_info": (_i32, [_vp, _P(_u64), _P(_u64), _P(_dbl)]),
     "edhip_iterate": (_i32, [_vp, _i32, _i64, _P(_i64), _P(_i64), _P(_dbl), _P(_dbl)]),
     "edhip_sparse_build": (_i32, [_vp, _dbl, _P(_i64)]),
+    "edhip_sparse_export_csc": (_i32, [_vp, _i32, _vp, _vp, _P(_dbl)]),
     "edhip_sparse_export": (_i32, [_vp, _P(_i64), _P(_i64), _P(_dbl), _P(_dbl)]),
     "edhip_get_vectors": (_i32, [_vp, _i32, _i64, _P(_i64), _dbl, _P(_i64), _P(_i64), _P(_dbl), _P(_dbl)]),
     "edhip_matrix": (_i32, [_vp, _vp]),

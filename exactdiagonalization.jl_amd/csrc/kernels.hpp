@@ -286,6 +286,10 @@ hipError_t launch_sparse_columns(const OpDev& op, int transpose, double tol, int
 // Dense column-major matrix (column form operator) added into a cleared
 // dim x dim buffer of doubles (complex_out: interleaved re, im pairs).
 hipError_t launch_dense_columns(const OpDev& op, int complex_out, double* d_out, hipStream_t st);
+// For the host: colptr then rowval in 4 bytes (idx32, where given), the values
+// interleaved (cplx, where given).
+hipError_t launch_sparse_pack(int64_t dim, int64_t nnz, const int64_t* d_colptr, const int64_t* d_rowval,
+                              const double* d_re, const double* d_im, int32_t* d_idx32, double* d_cplx, hipStream_t st);
 hipError_t launch_sparse_compact(int64_t dim, int slot, const int64_t* d_colptr, const int64_t* d_scratch_idx,
                                  const double* d_scratch_re, const double* d_scratch_im, int64_t* d_rowval,
                                  double* d_re, double* d_im, hipStream_t st);

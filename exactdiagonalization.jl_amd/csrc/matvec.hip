@@ -1,5 +1,7 @@
 // The other kernels that walk an operator: diagonal elements, raw iterators,
 // sparse and dense export, term expectations, assembled rows, pair groups.
+#include <algorithm>
+
 #include "opterms.hpp"
 
 namespace edhip {
@@ -232,6 +234,17 @@ __global__ __launch_bounds__(kBlock) void k_sparse_compact(int64_t dim, int slot
     re[o + k] = sre[col * (int64_t)slot + k];
     im[o + k] = sim[col * (int64_t)slot + k];
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_sparse_pack(int64_t dim, int64_t nnz, const int64_t* __restrict__ colptr,
+                                                        const int64_t* __restrict__ rowval,
+                                                        const double* __restrict__ re, const double* __restrict__ im,
+                                                        int32_t* __restrict__ idx32, double2* __restrict__ cplx) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (idx32 && i <= dim) idx32[i] = (int32_t)colptr[i];
+  if (i >= nnz) return;
+  if (idx32) idx32[dim + 1 + i] = (int32_t)rowval[i];
+  if (cplx) cplx[i] = double2{re[i], im[i]};
 }
 
 // ---------------------------------------------------------------------------
@@ -1047,6 +1060,14 @@ hipError_t launch_dense_columns(const OpDev& op, int complex_out, double* d_out,
     if (complex_out) EDHIP_DC(kGroupTorus, true); else EDHIP_DC(kGroupTorus, false);
   }
 #undef EDHIP_DC
+  return hipGetLastError();
+}
+
+hipError_t launch_sparse_pack(int64_t dim, int64_t nnz, const int64_t* d_colptr, const int64_t* d_rowval,
+                              const double* d_re, const double* d_im, int32_t* d_idx32, double* d_cplx, hipStream_t st) {
+  const int64_t n = std::max(dim + 1, nnz);
+  hipLaunchKernelGGL(k_sparse_pack, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dim, nnz, d_colptr,
+                     d_rowval, d_re, d_im, d_idx32, (double2*)d_cplx);
   return hipGetLastError();
 }
 

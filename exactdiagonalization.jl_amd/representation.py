@@ -734,16 +734,16 @@ class AbstractOperatorRepresentation:
             self.ctx.check(_lib.lib().edhip_sparse_build(self._handle, key, ctypes.byref(nnz)))
             n = self.dimension
             k = int(nnz.value)
-            colptr = np.empty(n + 1, np.int64)
-            rowval = np.empty(max(k, 1), np.int64)
-            re = np.empty(max(k, 1))
-            im = np.empty(max(k, 1))
+            # the index type that scipy settles on for such a matrix
+            index = np.int32 if max(n, k) <= np.iinfo(np.int32).max else np.int64
+            colptr = np.empty(n + 1, index)
+            rowval = np.empty(k, index)
+            data = np.empty(k, np.complex128 if self.is_complex else np.float64)
             self.ctx.check(
-                _lib.lib().edhip_sparse_export(self._handle, ptr(colptr, ctypes.c_int64), ptr(rowval, ctypes.c_int64),
-                                               ptr(re, ctypes.c_double), ptr(im, ctypes.c_double))
+                _lib.lib().edhip_sparse_export_csc(self._handle, colptr.itemsize, colptr.ctypes.data_as(ctypes.c_void_p),
+                                                   rowval.ctypes.data_as(ctypes.c_void_p), ptr(data, ctypes.c_double))
             )
-            data = (re[:k] + 1j * im[:k]) if self.is_complex else re[:k].copy()
-            self._sparse_cache[key] = sp.csc_matrix((data, rowval[:k].copy(), colptr), shape=(n, n))
+            self._sparse_cache[key] = sp.csc_matrix((data, rowval, colptr), shape=(n, n))
         return self._sparse_cache[key]
 
     sparse_serial = sparse

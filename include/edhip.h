@@ -269,6 +269,12 @@ int edhip_sparse_build(edhip_op* op, double tol, int64_t* nnz);
 int edhip_sparse_export(edhip_op* op, int64_t* colptr_host, int64_t* rowval_host, double* re_host,
                         double* im_host);
 
+/* The same for a host that keeps the matrix as it comes: indices in 4 or 8 bytes
+ * (4 where dimension and nnz are below 2^31), colptr[dim + 1], rowval[nnz], and
+ * values[nnz] (real operators) or interleaved (re, im) pairs (complex operators,
+ * edhip_op_is_complex), through pinned staging buffers of the context. */
+int edhip_sparse_export_csc(edhip_op* op, int index_bytes, void* colptr_host, void* rowval_host, double* values_host);
+
 /* get_row / get_column (abstract_operator_representation.jl:217-243) and the
  * column sums behind get_element (operator_representation.jl:109-119,
  * reduced_operator_representation.jl:120-138): for each of the n indices in

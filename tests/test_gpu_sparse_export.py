@@ -1,0 +1,37 @@
+"""The sparse matrix as it comes to the host through the staging buffers, against
+the plain export of the same matrix (exactly), in both index sizes, real and
+complex, over several staging parts and a last partial one (GPU)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Lx,Ly,k", [(4, 4, (1, 0)), (4, 5, (1, 2)), (4, 6, (2, 0)), (5, 5, (1, 1))])
+def test_staged_export(ed, Lx, Ly, k):
+    from edhip import _lib
+
+    hs, _ = ed.spin_half_system(Lx * Ly)
+    near, far = ed.square_bonds(Lx, Ly)
+    H = sum((ed.heisenberg_bond(hs, i, j) for i, j in near), ed.NullOperator())
+    H = ed.simplify(H + sum((ed.heisenberg_bond(hs, i, j, 0.3) for i, j in far), ed.NullOperator()))
+    space = ed.represent(ed.HilbertSpaceSector(hs, Lx * Ly % 2))
+    opr = ed.represent(ed.symmetry_reduce(space, ed.TranslationIrrep((Lx, Ly), k)), H)
+    A = opr.sparse()
+    n, nnz = opr.dimension, A.nnz
+    assert A.indices.dtype == np.int32 and A.indptr.dtype == np.int32 and A.has_sorted_indices
+    colptr, rowval = np.empty(n + 1, np.int64), np.empty(nnz, np.int64)
+    re, im = np.empty(nnz), np.empty(nnz)
+    L, i64, dbl = _lib.lib(), ctypes.c_int64, ctypes.c_double
+    opr.ctx.check(L.edhip_sparse_export(opr._handle, _lib.ptr(colptr, i64), _lib.ptr(rowval, i64), _lib.ptr(re, dbl),
+                                        _lib.ptr(im, dbl)))
+    assert np.array_equal(A.indptr, colptr) and np.array_equal(A.indices, rowval)
+    assert np.array_equal(A.data.real, re) and (not opr.is_complex or np.array_equal(A.data.imag, im))
+    wide_ptr, wide_row, data = np.empty_like(colptr), np.empty_like(rowval), np.empty_like(A.data)
+    opr.ctx.check(L.edhip_sparse_export_csc(opr._handle, 8, wide_ptr.ctypes.data_as(ctypes.c_void_p),
+                                            wide_row.ctypes.data_as(ctypes.c_void_p), _lib.ptr(data, dbl)))
+    assert np.array_equal(wide_ptr, colptr) and np.array_equal(wide_row, rowval) and np.array_equal(data, A.data)
+    assert L.edhip_sparse_export_csc(opr._handle, 2, wide_ptr.ctypes.data_as(ctypes.c_void_p),
+                                     wide_row.ctypes.data_as(ctypes.c_void_p), _lib.ptr(data, dbl)) != 0
