@@ -221,15 +221,160 @@ __global__ __launch_bounds__(kBlock) void k_dense_columns(OpDev op, double* __re
   }
 }
 
+// The same with a wave per vector, for slot <= kSparseSlots: the matching terms are
+// listed in order, 64 images are found at a time, and every entry finds its place
+// by counting the entries before it (index, then term order) in LDS, so that the
+// sums of duplicates run in the same order as above: the same values to the bit.
+// 4x6 (pi, 0), 112,792 columns of up to 193 entries: 1.07 ms, 3.97 ms with a lane
+// per column, which sorts in memory (1762 waves, every access a line of its own).
+constexpr int kSparseSlots = 256;
+constexpr uint32_t sparse_wave_bytes(int slot) { return (uint32_t)((slot + 63) & ~63) * 26u; }
+// LDS written by a wave's lanes before is read by its other lanes after.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+template <int MODE, bool TRANS>
+__global__ __launch_bounds__(kBlock) void k_sparse_waves(OpDev op, double tol, int slot, int64_t n_sel,
+                                                         const int64_t* __restrict__ sel, int64_t* __restrict__ sidx,
+                                                         double* __restrict__ sre, double* __restrict__ sim,
+                                                         int64_t* __restrict__ count) {
+  extern __shared__ unsigned char lds[];
+  Staged S = stage_op<MODE>(op, lds);
+  __syncthreads();
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+  const int64_t k = (int64_t)blockIdx.x * (kBlock / 64) + wave;
+  if (k >= n_sel) return;  // (no barrier below: waves are on their own)
+  const int cap = (slot + 63) & ~63;
+  unsigned char* mine = lds + op.lds_total + (uint32_t)wave * sparse_wave_bytes(slot);
+  int64_t* I = (int64_t*)mine;
+  double* Re = (double*)(I + cap);
+  double* Im = Re + cap;
+  uint16_t* list = (uint16_t*)(Im + cap);
+  const int64_t col = sel ? sel[k] : k;
+  const uint64_t bl = op.rows[col];
+  const uint64_t b = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(bl >> 32)) << 32) |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bl);  // the same in all lanes
+  int n = 0;
+  double dre = 0.0, dim_ = 0.0;
+  bool any_diag = false;
+  for (int t = 0; t < op.n_diag; ++t) {
+    const DiagTerm d = op.diag[t];
+    if ((b & d.mask) == d.match) {
+      dre += d.are;
+      dim_ += d.aim;
+      any_diag = true;
+    }
+  }
+  if (any_diag) {
+    if (lane == 0) {
+      I[0] = col;
+      Re[0] = dre;
+      Im[0] = dim_;
+    }
+    n = 1;
+  }
+  auto below = [&](uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  };
+  int n_match = 0;
+  for (int t0 = 0; t0 < op.n_off; t0 += 64) {
+    const int t = t0 + lane;
+    const bool hit = t < op.n_off && (b & S.off[t].mask) == S.off[t].match;
+    const uint64_t m = __ballot(hit);
+    if (hit) list[n_match + below(m)] = (uint16_t)t;
+    n_match += __builtin_popcountll(m);
+  }
+  double sqrt_own = 1.0;
+  if constexpr (MODE != kGroupNone) sqrt_own = sqrt((double)op.orbit[col]);
+  wave_lds_sync();
+  for (int i0 = 0; i0 < n_match; i0 += 64) {
+    int64_t idx = -1;
+    double wr = 0.0, wi = 0.0;
+    if (i0 + lane < n_match) {
+      const OffTerm t = S.off[list[i0 + lane]];
+      uint64_t s;
+      int h, cnt;
+      Canon<MODE>::run(op.g, S.L, (b & ~t.mask) | t.image, s, h, cnt);
+      idx = index_of(op.ix, S.W, s);
+      if (idx >= 0) element_weight<MODE, TRANS>(op, S, t, h, cnt, sqrt_own, wr, wi);
+    }
+    const uint64_t m = __ballot(idx >= 0);
+    if (idx >= 0) {
+      const int at = n + below(m);
+      I[at] = idx;
+      Re[at] = wr;
+      Im[at] = wi;
+    }
+    n += __builtin_popcountll(m);
+  }
+  wave_lds_sync();
+  // ascending, equal indices in term order
+  constexpr int E = kSparseSlots / 64;
+  int64_t key[E];
+  double vr[E], vi[E];
+  int place[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = e * 64 + lane;
+    if (e * 64 < n) {
+      key[e] = i < n ? I[i] : 0;
+      vr[e] = i < n ? Re[i] : 0.0;
+      vi[e] = i < n ? Im[i] : 0.0;
+      int p = 0;
+      for (int j = 0; j < n; ++j) {
+        const int64_t o = I[j];
+        p += (o < key[e] || (o == key[e] && j < i)) ? 1 : 0;
+      }
+      place[e] = p;
+    }
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e * 64 + lane < n) {
+      I[place[e]] = key[e];
+      Re[place[e]] = vr[e];
+      Im[place[e]] = vi[e];
+    }
+  wave_lds_sync();
+  // sums of duplicates, chop
+  int m = 0;
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    const int i = i0 + lane;
+    bool keep = false;
+    int64_t r = 0;
+    double sr = 0.0, si = 0.0;
+    if (i < n && (i == 0 || I[i - 1] != I[i])) {
+      r = I[i];
+      for (int j = i; j < n && I[j] == r; ++j) {
+        sr += Re[j];
+        si += Im[j];
+      }
+      keep = !(hypot(sr, si) < tol);
+    }
+    const uint64_t kept = __ballot(keep);
+    if (keep) {
+      const int64_t at = k * (int64_t)slot + m + below(kept);
+      sidx[at] = r;
+      sre[at] = sr;
+      sim[at] = si;
+    }
+    m += __builtin_popcountll(kept);
+  }
+  if (lane == 0) count[k] = m;
+}
+
+// (a wave per column: its entries are copied side by side; 0.06 ms, 0.54 with a lane)
 __global__ __launch_bounds__(kBlock) void k_sparse_compact(int64_t dim, int slot, const int64_t* __restrict__ colptr,
                                                            const int64_t* __restrict__ sidx, const double* __restrict__ sre,
                                                            const double* __restrict__ sim, int64_t* __restrict__ rowval,
                                                            double* __restrict__ re, double* __restrict__ im) {
-  const int64_t col = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t col = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
   if (col >= dim) return;
   const int64_t o = colptr[col];
   const int64_t n = colptr[col + 1] - o;
-  for (int64_t k = 0; k < n; ++k) {
+  for (int64_t k = threadIdx.x & 63; k < n; k += 64) {
     rowval[o + k] = sidx[col * (int64_t)slot + k];
     re[o + k] = sre[col * (int64_t)slot + k];
     im[o + k] = sim[col * (int64_t)slot + k];
@@ -1033,16 +1178,23 @@ hipError_t launch_sparse_columns(const OpDev& op, int transpose, double tol, int
                                  const int64_t* d_sel, int64_t* d_scratch_idx, double* d_scratch_re,
                                  double* d_scratch_im, int64_t* d_count, hipStream_t st) {
   if (n_sel == 0) return hipSuccess;
-  dim3 grid((unsigned)((n_sel + kBlock - 1) / kBlock));
+  const uint32_t wave_lds = op.lds_total + kBlock / 64 * sparse_wave_bytes(slot);
+  const bool waves = slot <= kSparseSlots && wave_lds <= 64 * 1024;
+  const int per_block = waves ? kBlock / 64 : kBlock;
+  dim3 grid((unsigned)((n_sel + per_block - 1) / per_block));
 #define EDHIP_SC(M, T)                                                                                                 \
-  hipLaunchKernelGGL((k_sparse_columns<M, T>), grid, dim3(kBlock), op.lds_total, st, op, tol, slot, n_sel, d_sel,     \
-                     d_scratch_idx, d_scratch_re, d_scratch_im, d_count)
+  if (waves)                                                                                                           \
+    hipLaunchKernelGGL((k_sparse_waves<M, T>), grid, dim3(kBlock), wave_lds, st, op, tol, slot, n_sel, d_sel,         \
+                       d_scratch_idx, d_scratch_re, d_scratch_im, d_count);                                           \
+  else                                                                                                                 \
+    hipLaunchKernelGGL((k_sparse_columns<M, T>), grid, dim3(kBlock), op.lds_total, st, op, tol, slot, n_sel, d_sel,   \
+                       d_scratch_idx, d_scratch_re, d_scratch_im, d_count)
   if (op.g.mode == kGroupNone) {
-    if (transpose) EDHIP_SC(kGroupNone, true); else EDHIP_SC(kGroupNone, false);
+    if (transpose) { EDHIP_SC(kGroupNone, true); } else { EDHIP_SC(kGroupNone, false); }
   } else if (op.g.mode == kGroupGeneric) {
-    if (transpose) EDHIP_SC(kGroupGeneric, true); else EDHIP_SC(kGroupGeneric, false);
+    if (transpose) { EDHIP_SC(kGroupGeneric, true); } else { EDHIP_SC(kGroupGeneric, false); }
   } else {
-    if (transpose) EDHIP_SC(kGroupTorus, true); else EDHIP_SC(kGroupTorus, false);
+    if (transpose) { EDHIP_SC(kGroupTorus, true); } else { EDHIP_SC(kGroupTorus, false); }
   }
 #undef EDHIP_SC
   return hipGetLastError();
@@ -1075,7 +1227,7 @@ hipError_t launch_sparse_compact(int64_t dim, int slot, const int64_t* d_colptr,
                                  const double* d_scratch_re, const double* d_scratch_im, int64_t* d_rowval,
                                  double* d_re, double* d_im, hipStream_t st) {
   if (dim == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sparse_compact, dim3((unsigned)((dim + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dim, slot,
+  hipLaunchKernelGGL(k_sparse_compact, dim3((unsigned)((dim + kBlock / 64 - 1) / (kBlock / 64))), dim3(kBlock), 0, st, dim, slot,
                      d_colptr, d_scratch_idx, d_scratch_re, d_scratch_im, d_rowval, d_re, d_im);
   return hipGetLastError();
 }
