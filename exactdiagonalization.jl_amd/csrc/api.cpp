@@ -1607,7 +1607,7 @@ void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) 
   }
   int lanes, batch;
   asm_shape(op, lanes, batch);
-  d.xcd_chunk = xcd_chunk_for(sp->dim * lanes / 256);
+  d.xcd_chunk = xcd_chunk_for(sp->dim * lanes / kAsmBlock);
   HIP_OR_THROW(launch_asm_spmv(d, op->asm_dev, prec, lanes, batch, accumulate, x, xt, y, st));
   if (op->ctx->kernel_timing) {
     HIP_OR_THROW(hipEventRecord(op->ctx->ev[15], st));

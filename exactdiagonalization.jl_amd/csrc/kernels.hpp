@@ -219,6 +219,7 @@ hipError_t launch_window_product_c128(const WinOp& P, int Lx, int Ly, int unit, 
 
 // ---- assembled rows (row form): entries col | cls << col_bits per image ----
 constexpr int kAsmMaxClasses = 256;
+constexpr int kAsmBlock = 512;  // lanes per block of the assembled product
 struct AsmFillDev {
   const uint64_t* rowptr;  // dim + 1 offsets of the rows' entries
   uint32_t* ent;
