@@ -111,7 +111,7 @@ struct DevBuf {
 struct UploadArena {
   static constexpr size_t kBytes = 256 * 1024;
   DevBuf dev;
-  std::vector<char> host;
+  std::unique_ptr<char[]> host;  // (not cleared)
   size_t used = 0;
 };
 thread_local UploadArena* t_arena = nullptr;
@@ -120,16 +120,16 @@ struct ArenaScope {
   UploadArena* before;
   explicit ArenaScope(UploadArena& a) : arena(a), before(t_arena) {
     arena.dev.alloc(UploadArena::kBytes);
-    arena.host.resize(UploadArena::kBytes);
+    arena.host.reset(new char[UploadArena::kBytes]);
     t_arena = &arena;
   }
   ~ArenaScope() { t_arena = before; }
   // waits: the host copy ends here
   void flush(hipStream_t st) {
     t_arena = before;
-    if (arena.used) HIP_OR_THROW(hipMemcpyAsync(arena.dev.p, arena.host.data(), arena.used, hipMemcpyHostToDevice, st));
+    if (arena.used) HIP_OR_THROW(hipMemcpyAsync(arena.dev.p, arena.host.get(), arena.used, hipMemcpyHostToDevice, st));
     HIP_OR_THROW(hipStreamSynchronize(st));
-    std::vector<char>().swap(arena.host);
+    arena.host.reset();
   }
 };
 
@@ -141,7 +141,7 @@ void upload(DevBuf& b, const std::vector<T>& v, hipStream_t st) {
     b.p = t_arena->dev.as<char>() + t_arena->used;
     b.bytes = std::max<size_t>(n, 16);
     b.view = true;
-    if (n) std::memcpy(t_arena->host.data() + t_arena->used, v.data(), n);
+    if (n) std::memcpy(t_arena->host.get() + t_arena->used, v.data(), n);
     t_arena->used += room;
     return;
   }
@@ -1386,11 +1386,14 @@ bool ensure_diag(edhip_op* op) {
     const std::vector<uint64_t> tab = mv_tables(D.entries, op->space->n_bits);
     if (tab.size() * 8 <= 32 * 1024 && D.rest.size() < op->diag_ids.size()) {
       hipStream_t st = op->ctx->stream;
+      UploadArena arena;
+      ArenaScope tables(arena);
       DevBuf tab_d, sets_d, first_d, rest_d;
       upload(tab_d, tab, st);
       upload(sets_d, sets, st);
       upload(first_d, D.first, st);
       upload(rest_d, rest, st);
+      tables.flush(st);
       const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
                          D.constant, (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
       HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
