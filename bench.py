@@ -650,7 +650,7 @@ def main():
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,
-            "kernel": "k_matvec<float> (term list, 6x6 row-pair canonicaliser, x / sqrt(N) spread over word positions)",
+            "kernel": "k_product_win<float> (6x6 window canonicaliser, x / sqrt(N) spread over word positions)",
             "kernel_ms": kms32,
             # measured HBM bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated) over this run's kernel time
             "traffic_GBps": traffic / (kms32 * 1e-3) / 1e9 if traffic else None,

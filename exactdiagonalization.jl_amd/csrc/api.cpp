@@ -1427,7 +1427,7 @@ bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const v
   // a dense spread only for vectors larger than the last-level cache: where x
   // itself fits it, the rank index's x gathers hit it and the index was
   // measured faster (6x6 space-group A1 sector, 31.6M words, 126 MB of FP32
-  // x: 57.8 ms against 67.0 ms through its spread)
+  // x, with the general kernel: 57.8 ms against 67.0 ms through its spread)
   const uint64_t ratio = es == 4 ? kXMapDenseRatio32 : kXMapDenseRatio;
   const bool dense = sp->ensure_xtop() <= ratio * (uint64_t)sp->dim && (uint64_t)sp->dim * es > kXMapCachedBytes;
   // the products on the shapes of window.hpp read x only through the spread and
@@ -1454,7 +1454,7 @@ bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const v
 // The eigensolver assembles the rows of a reduced space over 2^22 words for
 // the time of a solve (kernel auto) when their arrays take at most this much
 // and fit beside its workspace (6x6 space-group A1 sector: 9.6 GB built in
-// 0.1 s, products 57.9 -> 9.8 ms, mixed time to E0 3.40 -> 0.61 s)
+// 0.02 s, FP32 products 17.6 -> 9.1 ms, mixed time to E0 1.07 -> 0.59 s)
 constexpr uint64_t kAutoAsmMaxBytes = 16ull << 30;
 
 // Lanes per row and entries per lane per batch of the assembled product
