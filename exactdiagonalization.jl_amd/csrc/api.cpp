@@ -1386,19 +1386,27 @@ bool ensure_diag(edhip_op* op) {
     const std::vector<uint64_t> tab = mv_tables(D.entries, op->space->n_bits);
     if (tab.size() * 8 <= 32 * 1024 && D.rest.size() < op->diag_ids.size()) {
       hipStream_t st = op->ctx->stream;
-      UploadArena arena;
-      ArenaScope tables(arena);
-      DevBuf tab_d, sets_d, first_d, rest_d;
-      upload(tab_d, tab, st);
-      upload(sets_d, sets, st);
-      upload(first_d, D.first, st);
-      upload(rest_d, rest, st);
-      tables.flush(st);
-      const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
-                         D.constant, (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
-      HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
-      op->ctx->sync();
-      return true;
+      try {
+        UploadArena arena;
+        ArenaScope tables(arena);
+        DevBuf tab_d, sets_d, first_d, rest_d;
+        upload(tab_d, tab, st);
+        upload(sets_d, sets, st);
+        upload(first_d, D.first, st);
+        upload(rest_d, rest, st);
+        tables.flush(st);
+        const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
+                           D.constant, (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
+        HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
+        op->ctx->sync();
+        return true;
+      } catch (const Error& e) {
+        if (e.code != EDHIP_ERR_MEMORY) {
+          op->diag_re.release();
+          throw;
+        }
+        (void)hipGetLastError();  // no room for the tables: term by term
+      }
     }
   }
   HIP_OR_THROW(launch_diag_values(d, op->diag_re.as<double>(), op->diag_im.as<double>(), op->ctx->stream));
