@@ -1396,7 +1396,7 @@ bool ensure_diag(edhip_op* op) {
         upload(rest_d, rest, st);
         tables.flush(st);
         const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
-                           D.constant, (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
+                           (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
         HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
         op->ctx->sync();
         return true;

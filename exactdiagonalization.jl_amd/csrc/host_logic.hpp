@@ -260,14 +260,49 @@ inline std::vector<uint64_t> mv_tables(const MvSplit& S, int nb) {
   return tab;
 }
 
+// Diagonal term: adds its amplitude to the rows b with (b & mask) == match.
+struct DiagTerm {
+  uint64_t mask, match;
+  double are, aim;
+};
+
+// A sum of doubles whose rounding errors are kept beside it: the result is the
+// exact sum rounded about once.  An infinite or NaN sum is that of plain addition.
+struct CarriedSum {
+  double hi = 0.0, lo = 0.0;
+  EDHIP_HD void add(double x) {
+#ifdef __clang__
+#pragma clang fp contract(off)
+#endif
+    const double s = hi + x, t = s - hi;
+    lo += (hi - (s - t)) + (x - t);
+    hi = s;
+  }
+  // coef * count
+  EDHIP_HD void add_multiple(double coef, int count) {
+#ifdef __clang__
+#pragma clang fp contract(off)
+#endif
+    const double p = coef * (double)count;
+    const double rest = __builtin_fma(coef, (double)count, -p);
+    add(p);
+    lo += rest;
+  }
+  EDHIP_HD double value() const {
+    const double v = hi + lo;
+    return v - v == 0.0 ? v : hi;
+  }
+};
+
 // A diagonal operator with real amplitudes, sum of a_t [b & mask_t == match_t], by
-// parities: masks of one or two sites whose summed amplitudes depend on the
-// parity of the masked bits alone, m + h for even and m - h for odd, give m to a
-// constant and an entry (parity mask, h), the others stay terms.  The entries of
-// one h then sum to h (even ones - odd ones): for exchange and fields, whose m
-// is 0, a product with an integer and no cancellation.
+// parities: masks of one or two sites whose amplitudes are +h where the parity of
+// the masked bits is even and -h where it is odd (exchange, fields) become entries
+// (parity mask, h); the entries of one h sum to h (even ones - odd ones), a product
+// with an integer.  All other masks stay terms: split into a mean and +-h, a term
+// would add its mean to rows that it does not touch and take it away again, and a
+// row's element would carry the rounding of amplitudes that are not its own (a
+// penalty of 1e8 on parallel pairs: 7e-8 on the rows without one).
 struct DiagSplit {
-  double constant = 0.0;
   MvSplit entries;            // q, c and one lin entry (are: h) each
   std::vector<size_t> rest;   // terms left
   std::vector<uint64_t> sets; // per segment and coefficient: the entries' bits
@@ -279,23 +314,26 @@ inline DiagSplit diag_split(const std::vector<uint64_t>& mask, const std::vector
   DiagSplit D;
   std::map<uint64_t, std::vector<size_t>> by_mask;
   for (size_t t = 0; t < mask.size(); ++t) by_mask[mask[t]].push_back(t);
-  long double constant = 0.0L;
   std::vector<std::pair<double, uint64_t>> found;  // h, parity mask
   for (const auto& [m, ts] : by_mask) {
     const uint64_t lowest = m & (~m + 1);
     double f[4] = {0, 0, 0, 0};  // by (upper bit, lower bit)
-    for (size_t t : ts) f[((match[t] & lowest) ? 1 : 0) + ((match[t] & m & ~lowest) ? 2 : 0)] += amp[t];
+    bool exact = true;           // several amplitudes of one pattern add up without rounding
+    for (size_t t : ts) {
+      double& s = f[((match[t] & lowest) ? 1 : 0) + ((match[t] & m & ~lowest) ? 2 : 0)];
+      CarriedSum c;
+      c.add(s);
+      c.add(amp[t]);
+      exact = exact && c.lo == 0.0;  // (false for infinities and NaN)
+      s = c.hi;
+    }
     const int n = __builtin_popcountll(m);
-    if (n == 0) {
-      constant += f[0];
-    } else if (n == 1 || (n == 2 && f[0] == f[3] && f[1] == f[2])) {
-      constant += 0.5L * ((long double)f[0] + f[1]);
-      if (f[1] != f[0]) found.emplace_back(0.5 * (f[0] - f[1]), m);
+    if (exact && f[0] == -f[1] && (n == 1 || (n == 2 && f[0] == f[3] && f[1] == f[2]))) {
+      if (f[0] != 0.0) found.emplace_back(f[0], m);
     } else {
       D.rest.insert(D.rest.end(), ts.begin(), ts.end());
     }
   }
-  D.constant = (double)constant;
   std::sort(D.rest.begin(), D.rest.end());
   std::sort(found.begin(), found.end());  // equal coefficients together
   for (size_t e = 0; e < found.size(); ++e) {
@@ -311,6 +349,31 @@ inline DiagSplit diag_split(const std::vector<uint64_t>& mask, const std::vector
   }
   D.first.push_back((int32_t)D.sets.size());
   return D;
+}
+
+// Entries of one segment (bits of mask) that share a coefficient.
+struct DiagSet {
+  uint64_t mask;
+  double coef;
+};
+
+// The diagonal element of the word b from the entries' tables (mv_tables, n_seg
+// segments of n_chunk chunks), their sets by segment and the terms left.
+template <typename P>
+EDHIP_HD double diag_value(P tab, const DiagSet* sets, const int32_t* first, int n_seg, int n_chunk,
+                           const DiagTerm* rest, int n_rest, uint64_t b) {
+  CarriedSum v;
+  for (int seg = 0; seg < n_seg; ++seg) {
+    uint64_t bits = 0;
+    for (int k = 0; k < n_chunk; ++k)
+      bits ^= tab[((seg * n_chunk + k) << 4) + (int)((b >> ((4 * k) & 63)) & 15ull)];
+    for (int i = first[seg]; i < first[seg + 1]; ++i)
+      v.add_multiple(sets[i].coef,
+                     __builtin_popcountll(sets[i].mask) - 2 * __builtin_popcountll(bits & sets[i].mask));
+  }
+  for (int t = 0; t < n_rest; ++t)
+    if ((b & rest[t].mask) == rest[t].match) v.add(rest[t].are);
+  return v.value();
 }
 
 // Householder reduction of a dense symmetric matrix (row-major, n x n) to

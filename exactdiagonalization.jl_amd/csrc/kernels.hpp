@@ -81,11 +81,6 @@ hipError_t exclusive_scan_i64(const int64_t* d_in, int64_t* d_out, uint64_t n, v
                               hipStream_t st);
 
 // ---- matvec.hip, product_*.hip ---------------------------------------------
-struct DiagTerm {
-  uint64_t mask, match;
-  double are, aim;
-};
-
 // LDS offsets of the products' entries, from mv_lds.
 struct MvLayout {
   uint32_t off_mm, off_fa, off_ai, total;
@@ -254,19 +249,14 @@ hipError_t launch_asm_spmv(const OpDev& op, const AsmDev& a, int prec, int lanes
 // the amplitudes of the diagonal terms that match row r.
 hipError_t launch_diag_values(const OpDev& op, double* d_re, double* d_im, hipStream_t st);
 
-// The same for real amplitudes by parities (DiagSplit): constant + the coefficient
-// of every set of entries (mask within its segment) times the number of them whose
-// parity is even less that of those whose is odd + the terms left (rest).
-struct DiagSet {
-  uint64_t mask;
-  double coef;
-};
+// The same for real amplitudes by parities (DiagSplit): the coefficient of every
+// set of entries (mask within its segment) times the number of them whose parity
+// is even less that of those whose is odd, and the terms left (rest).
 struct DiagParity {
   const uint64_t* tab;   // as OpDev::lin_tab, n_seg segments of n_chunk chunks
   const DiagSet* sets;   // by segment
   const int32_t* first;  // n_seg + 1 offsets into sets
   const DiagTerm* rest;
-  double constant;
   int n_seg, n_chunk, n_rest;
 };
 hipError_t launch_diag_parity(const DiagParity& P, const uint64_t* d_rows, int64_t dim, double* d_re, hipStream_t st);

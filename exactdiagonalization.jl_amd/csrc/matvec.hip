@@ -30,19 +30,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_parity(DiagParity P, const uint
   __syncthreads();
   const LdsPtr<uint64_t> tab = lds_at<uint64_t>(0);
   for (int64_t row = (int64_t)blockIdx.x * kBlock + threadIdx.x; row < dim; row += (int64_t)gridDim.x * kBlock) {
-    const uint64_t b = rows[row];
-    double v = P.constant;
-    for (int seg = 0; seg < P.n_seg; ++seg) {
-      uint64_t bits = 0;
-      for (int k = 0; k < P.n_chunk; ++k)
-        bits ^= tab[((seg * P.n_chunk + k) << 4) + (int)((b >> ((4 * k) & 63)) & 15ull)];
-      for (int i = P.first[seg]; i < P.first[seg + 1]; ++i)
-        v += P.sets[i].coef *
-             (double)(__builtin_popcountll(P.sets[i].mask) - 2 * __builtin_popcountll(bits & P.sets[i].mask));
-    }
-    for (int t = 0; t < P.n_rest; ++t)
-      if ((b & P.rest[t].mask) == P.rest[t].match) v += P.rest[t].are;
-    re[row] = v;
+    re[row] = diag_value(tab, P.sets, P.first, P.n_seg, P.n_chunk, P.rest, P.n_rest, rows[row]);
   }
 }
 
