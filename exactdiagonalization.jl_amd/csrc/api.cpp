@@ -354,6 +354,8 @@ constexpr size_t kNibLdsMax = 40 * 1024;
 struct edhip_space {
   edhip_ctx* ctx = nullptr;
   int n_bits = 0;
+  int list_bits = 0;  // of the largest word of a basis list, which may have bits past n_bits
+  int word_bits() const { return std::max(n_bits, list_bits); }
   int64_t dim = 0;
   // sector description (popcount sector)
   bool is_sector = false;
@@ -1184,7 +1186,7 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   }
   d.n_off = op->n_off;
   d.n_diag = op->n_diag;
-  d.word_bits = sp->n_bits;
+  d.word_bits = sp->word_bits();
   for (int i = 0; i < op->n_diag; ++i) {
     const int64_t t = op->diag_ids[i];
     d.word_bits = std::max({d.word_bits, bit_length(op->mask[t]), bit_length(op->row[t])});
@@ -1195,7 +1197,7 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
   const uint32_t group_bytes = align_up(d.lay.total, 16);
   const int form = transpose ? 1 : 0;
-  d.n_chunk = mv_chunks(sp->n_bits);
+  d.n_chunk = mv_chunks(sp->word_bits());
   const MvLayout full = mv_layout(op->mv[form].n_lin, d.n_chunk, op->mv[form].n_rest, 1);
   const bool no_room = group_bytes + std::max(full.total, plain_bytes) + w_bytes > 64 * 1024 &&
                        group_bytes + plain_bytes + w_bytes <= 64 * 1024;
@@ -1383,7 +1385,7 @@ bool ensure_diag(edhip_op* op) {
     for (size_t i = 0; i < D.sets.size(); ++i) sets.push_back(DiagSet{D.sets[i], D.coefs[i]});
     std::vector<DiagTerm> rest;
     for (size_t t : D.rest) rest.push_back(DiagTerm{mask[t], match[t], amp[t], 0.0});
-    const std::vector<uint64_t> tab = mv_tables(D.entries, op->space->n_bits);
+    const std::vector<uint64_t> tab = mv_tables(D.entries, op->space->word_bits());
     if (tab.size() * 8 <= 32 * 1024 && D.rest.size() < op->diag_ids.size()) {
       hipStream_t st = op->ctx->stream;
       try {
@@ -1396,7 +1398,7 @@ bool ensure_diag(edhip_op* op) {
         upload(rest_d, rest, st);
         tables.flush(st);
         const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
-                           (int)D.first.size() - 1, mv_chunks(op->space->n_bits), (int)rest.size()};
+                           (int)D.first.size() - 1, mv_chunks(op->space->word_bits()), (int)rest.size()};
         HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
         op->ctx->sync();
         return true;
@@ -2370,6 +2372,7 @@ int edhip_space_from_list(edhip_ctx* ctx, int n_bits, int64_t n, const uint64_t*
       if (basis[i - 1] == basis[i]) fail(EDHIP_ERR_ARGUMENT, "vals contains duplicates");
     sp->ctx = ctx;
     sp->n_bits = n_bits;
+    sp->list_bits = n ? bit_length(basis[n - 1]) : 0;
     sp->dim = n;
     sp->keys.alloc((size_t)std::max<int64_t>(n, 1) * 8);
     if (n) HIP_OR_THROW(hipMemcpyAsync(sp->keys.p, basis, (size_t)n * 8, hipMemcpyHostToDevice, ctx->stream));
@@ -2535,6 +2538,7 @@ int edhip_space_reduce_ex(edhip_ctx* ctx, const edhip_space* parent, int n_group
     n_threads = (NW + chunk - 1) / chunk;
     sp->ctx = ctx;
     sp->n_bits = nb;
+    sp->list_bits = parent->list_bits;
     sp->parent = parent;
     if (n_threads == 0) {
       sp->dim = 0;
@@ -2756,7 +2760,7 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
       M.n_rest = (int)S.rest.size();
       M.entries = S.lin;
       for (const OffTerm& o : S.rest) M.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});
-      upload(M.tab, mv_tables(S, space->n_bits), ctx->stream);
+      upload(M.tab, mv_tables(S, space->word_bits()), ctx->stream);
       upload(M.rest, S.rest, ctx->stream);
       upload(M.ent, M.entries, ctx->stream);
       edhip_op::MvHost& P = op->mv_plain[form];
