@@ -1087,7 +1087,7 @@ struct edhip_op {
   std::vector<uint64_t> mask, row, col;
   std::vector<double> are, aim;
   bool complex_amp = false;
-  bool keeps_popcount = true;  // every off-diagonal term's image has its row's popcount
+  bool keeps_popcount = true;  // every off-diagonal term's images have their rows' popcount (off_term)
   // device terms
   DevBuf off_row, off_col, diag, all_row, all_col;
   // the products' entries, row form [0] and column form [1] (OpDev)
@@ -2736,9 +2736,9 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
         dg.push_back(DiagTerm{mask[t], row[t], are[t], aim[t]});
         op->diag_ids.push_back(t);
       } else {
-        if (__builtin_popcountll(row[t]) != __builtin_popcountll(col[t])) op->keeps_popcount = false;
-        offr.push_back(OffTerm{mask[t], row[t], col[t], are[t], aim[t]});
-        offc.push_back(OffTerm{mask[t], col[t], row[t], are[t], aim[t]});
+        offr.push_back(off_term(mask[t], row[t], col[t], are[t], aim[t], space->word_bits()));
+        offc.push_back(off_term(mask[t], col[t], row[t], are[t], aim[t], space->word_bits()));
+        if (__builtin_popcountll(offr.back().match) != __builtin_popcountll(offr.back().image)) op->keeps_popcount = false;
         op->off_ids.push_back(t);
       }
     }
@@ -3231,6 +3231,9 @@ static bool expect_by_rank(edhip_op* op, ExpectRank& E) {
       if ((op->mask[t] >> lb) && (low & (low - 1))) return false;
       if (op->row[t] & ~op->mask[t]) return false;
     }
+    // (terms that lead out of the words stay with the general kernels, as off_term makes them)
+    for (int64_t t : op->off_ids)
+      if ((op->row[t] | op->col[t]) >> sp->n_bits) return false;
     std::vector<ExpectStep> steps;
     for (size_t j = 0; j < op->off_ids.size(); ++j) {
       const int64_t t = op->off_ids[j];

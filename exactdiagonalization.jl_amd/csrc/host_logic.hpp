@@ -174,6 +174,15 @@ struct OffTerm {
   double are, aim;
 };
 
+// A term as it acts on words of n_bits bits: one whose match or image has a bit
+// past them takes no word to another, and is made to match none.  (The kernels that
+// find an image by its position alone need every image to be such a word.)
+inline OffTerm off_term(uint64_t mask, uint64_t match, uint64_t image, double are, double aim, int n_bits) {
+  const uint64_t past = n_bits >= 64 ? 0ull : ~0ull << n_bits;
+  if ((match | image) & past) return OffTerm{0, 1, 1, 0.0, 0.0};
+  return OffTerm{mask, match, image, are, aim};
+}
+
 // One entry of the products: a matching row b has the image b ^ flip.
 struct MvEntry {
   uint64_t flip;

@@ -1,0 +1,14 @@
+"""The images of the products' entries stay words of the space (CPU, with
+AddressSanitizer and UndefinedBehaviorSanitizer): tests/native/images_host.cpp."""
+import os
+import subprocess
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def test_images_are_words(tmp_path):
+    exe = str(tmp_path / "images")
+    subprocess.check_call(["g++", "-O1", "-g", "-std=c++17", "-fsanitize=address,undefined", "-fno-sanitize-recover=all",
+                           "-o", exe, os.path.join(HERE, "native", "images_host.cpp")])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
