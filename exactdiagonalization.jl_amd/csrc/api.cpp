@@ -3229,7 +3229,8 @@ static bool expect_by_rank(edhip_op* op, ExpectRank& E) {
     for (int64_t t : op->diag_ids) {
       const uint64_t low = op->mask[t] & lmask;
       if ((op->mask[t] >> lb) && (low & (low - 1))) return false;
-      if (op->row[t] & ~op->mask[t]) return false;
+      // (32-bit masks: a bit past the words, which no row has, stays with the general kernels)
+      if (op->row[t] >> sp->n_bits) return false;
     }
     // (terms that lead out of the words stay with the general kernels, as off_term makes them)
     for (int64_t t : op->off_ids)

@@ -93,3 +93,25 @@ def test_term_pass(ed, oracle, n, up, shape, k):
     ref = _forms(oracle, ospace, ed.terms_arrays(H), phi, psi)
     got = ed.term_expectations(opr, torch.tensor(phi).cuda(), torch.tensor(psi).cuda())
     assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("n,up", [(16, 8), (24, 4), (26, 3)])
+@pytest.mark.parametrize("top", [0, 4, 35, 40, 62])
+def test_diagonal_terms_past_the_words(ed, oracle, n, up, top):
+    """Diagonal terms that test such a bit beside the forms by rank: no row has it set."""
+    import torch
+
+    hs, space, basis = _spaces(ed, oracle, n, up)
+    P, bit, last = ed.PureOperator, 1 << (top if top > n else n + top), 1 << (n - 1)
+    H = sum((ed.heisenberg_bond(hs, i, j) for i, j in ed.chain_bonds(n)[:4]), ed.NullOperator())
+    H = ed.SumOperator(list(H.terms) + [P(1 | bit, 1 | bit, 1 | bit, 1.0), P(bit, bit, bit, 1.0), P(last | bit, bit, bit, 1.0),
+                                        P(last | bit, last, last, 1.0), P(bit, 0, 0, 1.0), P(1 | bit, 0, 0, 1.0)])
+    opr = ed.represent(space, H)
+    rng = np.random.default_rng(n)
+    phi, psi = rng.standard_normal((2, opr.dimension))
+    ref = _forms(oracle, basis, ed.terms_arrays(H), phi, psi)
+    got = ed.term_expectations(opr, torch.tensor(phi).cuda(), torch.tensor(psi).cuda())
+    assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+    y = opr @ psi
+    ref = oracle.Opr(basis, ed.terms_arrays(H)).matvec(psi)
+    assert np.linalg.norm(y - ref) <= 1e-13 * np.linalg.norm(ref)
