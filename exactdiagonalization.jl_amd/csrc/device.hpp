@@ -60,6 +60,9 @@ __device__ __forceinline__ int64_t xcd_chunked_block(int64_t b, int64_t n_blocks
   return b - r + (r & 7) * C + (r >> 3);
 }
 
+// Number of the block in a grid of block_grid.
+__device__ __forceinline__ int64_t flat_block() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 template <typename V>
 __device__ __forceinline__ V vzero() {
   if constexpr (VT<V>::cx) {

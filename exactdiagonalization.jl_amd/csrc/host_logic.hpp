@@ -18,6 +18,17 @@
 
 namespace edhip {
 
+// A launch of n_blocks blocks in two grid dimensions (numbered x first, the last
+// row partly past n_blocks): a dimension holds fewer than 2^32 lanes, which one
+// alone passes at 2^26 columns with a wave each.
+struct BlockGrid {
+  uint32_t x, y;
+};
+inline BlockGrid block_grid(uint64_t n_blocks) {
+  const uint64_t x = std::min<uint64_t>(std::max<uint64_t>(n_blocks, 1), 1ull << 22);
+  return BlockGrid{(uint32_t)x, (uint32_t)((n_blocks + x - 1) / x)};
+}
+
 // Rank tables of the n-bit words of popcount pop: rank(w) = base[w >> low_bits]
 // + low[w & mask], low the rank of a low_bits-bit word among those of its
 // popcount, base the number of words whose upper part is smaller.  base is

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(kBlock) void k_sparse_columns(OpDev op, double tol,
   extern __shared__ unsigned char lds[];
   Staged S = stage_op<MODE>(op, lds);
   __syncthreads();
-  const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t k = flat_block() * kBlock + threadIdx.x;
   if (k >= n_sel) return;
   const int64_t col = sel ? sel[k] : k;
   const uint64_t b = op.rows[col];
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_sparse_waves(OpDev op, double tol, i
   Staged S = stage_op<MODE>(op, lds);
   __syncthreads();
   const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
-  const int64_t k = (int64_t)blockIdx.x * (kBlock / 64) + wave;
+  const int64_t k = flat_block() * (kBlock / 64) + wave;
   if (k >= n_sel) return;  // (no barrier below: waves are on their own)
   const int cap = (slot + 63) & ~63;
   unsigned char* mine = lds + op.lds_total + (uint32_t)wave * sparse_wave_bytes(slot);
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void k_sparse_compact(int64_t dim, int slot
                                                            const int64_t* __restrict__ sidx, const double* __restrict__ sre,
                                                            const double* __restrict__ sim, int64_t* __restrict__ rowval,
                                                            double* __restrict__ re, double* __restrict__ im) {
-  const int64_t col = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const int64_t col = flat_block() * (kBlock / 64) + (threadIdx.x >> 6);
   if (col >= dim) return;
   const int64_t o = colptr[col];
   const int64_t n = colptr[col + 1] - o;
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kBlock) void k_sparse_pack(int64_t dim, int64_t nnz
                                                         const int64_t* __restrict__ rowval,
                                                         const double* __restrict__ re, const double* __restrict__ im,
                                                         int32_t* __restrict__ idx32, double2* __restrict__ cplx) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  const int64_t i = flat_block() * kBlock + threadIdx.x;
   if (idx32 && i <= dim) idx32[i] = (int32_t)colptr[i];
   if (i >= nnz) return;
   if (idx32) idx32[dim + 1 + i] = (int32_t)rowval[i];
@@ -1172,7 +1172,8 @@ hipError_t launch_sparse_columns(const OpDev& op, int transpose, double tol, int
   const uint32_t wave_lds = op.lds_total + kBlock / 64 * sparse_wave_bytes(slot);
   const bool waves = slot <= kSparseSlots && wave_lds <= 64 * 1024;
   const int per_block = waves ? kBlock / 64 : kBlock;
-  dim3 grid((unsigned)((n_sel + per_block - 1) / per_block));
+  const BlockGrid g2 = block_grid((uint64_t)(n_sel + per_block - 1) / (uint64_t)per_block);
+  const dim3 grid(g2.x, g2.y);
 #define EDHIP_SC(M, T)                                                                                                 \
   if (waves)                                                                                                           \
     hipLaunchKernelGGL((k_sparse_waves<M, T>), grid, dim3(kBlock), wave_lds, st, op, tol, slot, n_sel, d_sel,         \
@@ -1209,7 +1210,8 @@ hipError_t launch_dense_columns(const OpDev& op, int complex_out, double* d_out,
 hipError_t launch_sparse_pack(int64_t dim, int64_t nnz, const int64_t* d_colptr, const int64_t* d_rowval,
                               const double* d_re, const double* d_im, int32_t* d_idx32, double* d_cplx, hipStream_t st) {
   const int64_t n = std::max(dim + 1, nnz);
-  hipLaunchKernelGGL(k_sparse_pack, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, dim, nnz, d_colptr,
+  const BlockGrid g2 = block_grid((uint64_t)(n + kBlock - 1) / kBlock);
+  hipLaunchKernelGGL(k_sparse_pack, dim3(g2.x, g2.y), dim3(kBlock), 0, st, dim, nnz, d_colptr,
                      d_rowval, d_re, d_im, d_idx32, (double2*)d_cplx);
   return hipGetLastError();
 }
@@ -1218,8 +1220,8 @@ hipError_t launch_sparse_compact(int64_t dim, int slot, const int64_t* d_colptr,
                                  const double* d_scratch_re, const double* d_scratch_im, int64_t* d_rowval,
                                  double* d_re, double* d_im, hipStream_t st) {
   if (dim == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_sparse_compact, dim3((unsigned)((dim + kBlock / 64 - 1) / (kBlock / 64))), dim3(kBlock), 0, st, dim, slot,
-                     d_colptr, d_scratch_idx, d_scratch_re, d_scratch_im, d_rowval, d_re, d_im);
+  const BlockGrid g2 = block_grid((uint64_t)(dim + kBlock / 64 - 1) / (kBlock / 64));
+  hipLaunchKernelGGL(k_sparse_compact, dim3(g2.x, g2.y), dim3(kBlock), 0, st, dim, slot, d_colptr, d_scratch_idx, d_scratch_re, d_scratch_im, d_rowval, d_re, d_im);
   return hipGetLastError();
 }
 
