@@ -103,46 +103,116 @@ struct DevBuf {
   }
 };
 
-// Tables that live and die with one object, in one allocation and one copy: while
-// an ArenaScope is open, this thread's uploads that fit go to its arena, whose
-// memory the scope's flush copies to the device (a 28-site reduction and its
-// operator: 45 small allocations, copies and frees, 20 to 30 us each).  Inside a
-// scope only buffers of the arena's own object are uploaded.
-struct UploadArena {
-  static constexpr size_t kBytes = 256 * 1024;
+// Tables that live and die with one object, copied to the device at once: while an
+// ArenaScope is open, this thread's uploads to the buffers of the scope's object that
+// fit go to its arena, whose part of the device memory the scope's flush fills (a
+// 28-site reduction and its operator: 45 small allocations, copies and frees, 20 to
+// 30 us each).  Uploads to any other object's buffers, which may live longer, take
+// memory of their own as always.
+//
+// The device memory is a part of a slab that the objects made one after the other
+// share (an operator on 8 sites: 21 kB of its own instead of a 256 kB block); a slab
+// is freed with the last of them.  Parts are never used again before that, so no
+// kernel still reading one needs to be waited for when its object ends.
+constexpr size_t kSlabBytes = 256 * 1024;
+struct Slab {
   DevBuf dev;
-  std::unique_ptr<char[]> host;  // (not cleared)
   size_t used = 0;
 };
-thread_local UploadArena* t_arena = nullptr;
+// The slab with room left, at most one per context.
+struct OpenSlab {
+  std::mutex lock;
+  std::shared_ptr<Slab> slab;
+  // one with the bytes wanted (at most a whole slab), for the caller alone until given back
+  std::shared_ptr<Slab> take(size_t bytes) {
+    {
+      std::lock_guard<std::mutex> hold(lock);
+      if (slab && kSlabBytes - slab->used >= std::min(bytes, kSlabBytes)) return std::move(slab);
+    }
+    auto fresh = std::make_shared<Slab>();
+    fresh->dev.alloc(kSlabBytes);
+    return fresh;
+  }
+  void give_back(const std::shared_ptr<Slab>& s) {
+    std::lock_guard<std::mutex> hold(lock);
+    if (!slab || slab->used > s->used) slab = s;
+  }
+};
+struct UploadArena {
+  std::shared_ptr<Slab> slab;  // (part of it)
+  std::unique_ptr<char[]> host;  // (not cleared)
+  size_t begin = 0, used = 0;
+};
+struct ArenaScope;
+thread_local ArenaScope* t_arena = nullptr;
 struct ArenaScope {
   UploadArena& arena;
-  UploadArena* before;
-  explicit ArenaScope(UploadArena& a) : arena(a), before(t_arena) {
-    arena.dev.alloc(UploadArena::kBytes);
-    arena.host.reset(new char[UploadArena::kBytes]);
-    t_arena = &arena;
+  OpenSlab& open;
+  const char *object, *object_end;
+  ArenaScope* before;
+  // object: whose members' buffers go to the arena; bytes: about what they take
+  template <typename T>
+  ArenaScope(OpenSlab& o, UploadArena& a, const T* owner, size_t bytes)
+      : arena(a), open(o), object((const char*)owner), object_end((const char*)(owner + 1)), before(t_arena) {
+    arena.slab = open.take(bytes);
+    arena.begin = arena.slab->used;
+    arena.host.reset(new char[kSlabBytes - arena.begin]);
+    t_arena = this;
   }
   ~ArenaScope() { t_arena = before; }
+  static size_t room(size_t n) { return (std::max<size_t>(n, 16) + 255) / 256 * 256; }
+  bool takes(const DevBuf& b, size_t n) const {
+    return (const char*)&b >= object && (const char*)&b < object_end &&
+           arena.begin + arena.used + room(n) <= kSlabBytes;
+  }
+  void put(DevBuf& b, const void* v, size_t n) {
+    b.release();
+    b.p = arena.slab->dev.as<char>() + arena.begin + arena.used;
+    b.bytes = std::max<size_t>(n, 16);
+    b.view = true;
+    if (n) std::memcpy(arena.host.get() + arena.used, v, n);
+    arena.used += room(n);
+  }
   // waits: the host copy ends here
   void flush(hipStream_t st) {
     t_arena = before;
-    if (arena.used) HIP_OR_THROW(hipMemcpyAsync(arena.dev.p, arena.host.get(), arena.used, hipMemcpyHostToDevice, st));
+    if (arena.used)
+      HIP_OR_THROW(hipMemcpyAsync(arena.slab->dev.as<char>() + arena.begin, arena.host.get(), arena.used,
+                                  hipMemcpyHostToDevice, st));
     HIP_OR_THROW(hipStreamSynchronize(st));
     arena.host.reset();
+    arena.slab->used = arena.begin + arena.used;
+    open.give_back(arena.slab);
+  }
+};
+
+// Tables of one call, in one allocation and one copy.
+struct PackedTables {
+  std::vector<char> host;
+  DevBuf dev;
+  template <typename T>
+  size_t add(const std::vector<T>& v) {
+    const size_t at = host.size();
+    host.resize(at + ArenaScope::room(v.size() * sizeof(T)));
+    if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+  // waits: the host copy may end after it
+  void send(hipStream_t st) {
+    dev.alloc(host.size());
+    HIP_OR_THROW(hipMemcpyAsync(dev.p, host.data(), host.size(), hipMemcpyHostToDevice, st));
+    HIP_OR_THROW(hipStreamSynchronize(st));
+  }
+  template <typename T>
+  const T* at(size_t offset) const {
+    return (const T*)((const char*)dev.p + offset);
   }
 };
 
 template <typename T>
 void upload(DevBuf& b, const std::vector<T>& v, hipStream_t st) {
-  const size_t n = v.size() * sizeof(T), room = (std::max<size_t>(n, 16) + 255) / 256 * 256;
-  if (t_arena && t_arena->used + room <= UploadArena::kBytes) {
-    b.release();
-    b.p = t_arena->dev.as<char>() + t_arena->used;
-    b.bytes = std::max<size_t>(n, 16);
-    b.view = true;
-    if (n) std::memcpy(t_arena->host.get() + t_arena->used, v.data(), n);
-    t_arena->used += room;
+  if (t_arena && t_arena->takes(b, v.size() * sizeof(T))) {
+    t_arena->put(b, v.data(), v.size() * sizeof(T));
     return;
   }
   b.alloc(v.size() * sizeof(T));
@@ -183,6 +253,7 @@ struct edhip_ctx {
     return small.as<double>();
   }
   void sync() { HIP_OR_THROW(hipStreamSynchronize(stream)); }
+  OpenSlab open_slab;  // of the tables of its objects (ArenaScope)
 
   // Large results on their way to host memory: two pinned buffers, allocated on
   // first use and freed with the context.
@@ -1168,6 +1239,21 @@ void check_flip_closed(const edhip_space* p) {
       fail(EDHIP_ERR_ARGUMENT, "the global bit flip maps the basis outside itself");
 }
 
+uint32_t rank_table_bytes(const edhip_space* sp) {
+  return sp->is_sector && !sp->group ? (uint32_t)((sp->n_bits + 1) * (sp->n_bits + 1) * 8) : 0u;
+}
+
+// Whether the tables of the products' entries leave no LDS room where the plain
+// list of the terms still does.
+bool mv_no_room(const edhip_op* op, int form) {
+  const edhip_space* sp = op->space;
+  const uint32_t group_bytes = align_up(sp->group ? sp->group->lay.total : 0u, 16), w_bytes = rank_table_bytes(sp);
+  const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
+  const MvLayout full = mv_layout(op->mv[form].n_lin, mv_chunks(sp->word_bits()), op->mv[form].n_rest, 1);
+  return group_bytes + std::max(full.total, plain_bytes) + w_bytes > 64 * 1024 &&
+         group_bytes + plain_bytes + w_bytes <= 64 * 1024;
+}
+
 OpDev make_opdev(edhip_op* op, bool transpose) {
   const edhip_space* sp = op->space;
   OpDev d{};
@@ -1193,14 +1279,12 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   }
   d.off = transpose ? op->off_col.as<OffTerm>() : op->off_row.as<OffTerm>();
   d.diag = op->diag.as<DiagTerm>();
-  const uint32_t w_bytes = d.ix.rank_mode ? (uint32_t)((sp->n_bits + 1) * (sp->n_bits + 1) * 8) : 0u;
+  const uint32_t w_bytes = rank_table_bytes(sp);
   const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
   const uint32_t group_bytes = align_up(d.lay.total, 16);
   const int form = transpose ? 1 : 0;
   d.n_chunk = mv_chunks(sp->word_bits());
-  const MvLayout full = mv_layout(op->mv[form].n_lin, d.n_chunk, op->mv[form].n_rest, 1);
-  const bool no_room = group_bytes + std::max(full.total, plain_bytes) + w_bytes > 64 * 1024 &&
-                       group_bytes + plain_bytes + w_bytes <= 64 * 1024;
+  const bool no_room = mv_no_room(op, form);
   const auto& mv = no_room ? op->mv_plain[form] : op->mv[form];
   d.ent = mv.ent.as<MvEntry>();
   d.lin_tab = mv.tab.as<uint64_t>();
@@ -1389,15 +1473,10 @@ bool ensure_diag(edhip_op* op) {
     if (tab.size() * 8 <= 32 * 1024 && D.rest.size() < op->diag_ids.size()) {
       hipStream_t st = op->ctx->stream;
       try {
-        UploadArena arena;
-        ArenaScope tables(arena);
-        DevBuf tab_d, sets_d, first_d, rest_d;
-        upload(tab_d, tab, st);
-        upload(sets_d, sets, st);
-        upload(first_d, D.first, st);
-        upload(rest_d, rest, st);
-        tables.flush(st);
-        const DiagParity P{tab_d.as<uint64_t>(), sets_d.as<DiagSet>(), first_d.as<int32_t>(), rest_d.as<DiagTerm>(),
+        PackedTables T;
+        const size_t at[4] = {T.add(tab), T.add(sets), T.add(D.first), T.add(rest)};
+        T.send(st);
+        const DiagParity P{T.at<uint64_t>(at[0]), T.at<DiagSet>(at[1]), T.at<int32_t>(at[2]), T.at<DiagTerm>(at[3]),
                            (int)D.first.size() - 1, mv_chunks(op->space->word_bits()), (int)rest.size()};
         HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
         op->ctx->sync();
@@ -2519,7 +2598,8 @@ int edhip_space_reduce_ex(edhip_ctx* ctx, const edhip_space* parent, int n_group
     gh->chi.resize(n_group);
     for (int g = 0; g < n_group; ++g) gh->chi[g] = {chi_re[g], chi_im[g]};
     {
-      ArenaScope tables(gh->arena);
+      // (translations of a torus take 10 to 30 kB, more goes to allocations of its own)
+      ArenaScope tables(ctx->open_slab, gh->arena, gh.get(), 64 * 1024);
       build_group(*gh, nb, tol, ctx->stream);
       tables.flush(ctx->stream);
     }
@@ -2744,7 +2824,8 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
     }
     op->n_off = (int)offr.size();
     op->n_diag = (int)dg.size();
-    ArenaScope tables(op->arena);
+    // 40 bytes a term in each of four lists and in the products' entries, and their tables
+    ArenaScope tables(ctx->open_slab, op->arena, op.get(), (size_t)n_terms * 400 + 32 * 1024);
     upload(op->off_row, offr, ctx->stream);
     upload(op->off_col, offc, ctx->stream);
     for (int form = 0; form < 2; ++form) {
@@ -2763,10 +2844,12 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
       upload(M.tab, mv_tables(S, space->word_bits()), ctx->stream);
       upload(M.rest, S.rest, ctx->stream);
       upload(M.ent, M.entries, ctx->stream);
-      edhip_op::MvHost& P = op->mv_plain[form];
-      P.n_rest = (int)v.size();
-      for (const OffTerm& o : v) P.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});
-      upload(P.ent, P.entries, ctx->stream);
+      if (mv_no_room(op.get(), form)) {
+        edhip_op::MvHost& P = op->mv_plain[form];
+        P.n_rest = (int)v.size();
+        for (const OffTerm& o : v) P.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});
+        upload(P.ent, P.entries, ctx->stream);
+      }
     }
     upload(op->diag, dg, ctx->stream);
     upload(op->all_row, allr, ctx->stream);
