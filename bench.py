@@ -295,7 +295,7 @@ def assembled_times(ed, opr, elems, steps, warmup, e0=True):
                     "checksum": cs32},
             "f64": {"ms_per_step": ms64, "kernel_ms": k64, "Gelem_per_s": elems / (ms64 * 1e-3) / 1e9,
                     "checksum": cs64},
-            "kernels": "k_asm_scale (x / sqrt(N)) + k_asm_spmv (16 lanes per row, 8 entries per lane per batch)",
+            "kernels": "k_asm_scale (x sqrt(G / N)) + k_asm_spmv (16 lanes per row, 8 entries per lane per batch)",
         }
         te = {}
         for mode in ("fp64", "mixed") if e0 else ():
@@ -650,7 +650,7 @@ def main():
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": traffic,
-            "kernel": "k_product_win<float> (6x6 window canonicaliser, x / sqrt(N) spread over word positions)",
+            "kernel": "k_product_win<float> (6x6 window canonicaliser, x sqrt(G / N) spread over word positions)",
             "kernel_ms": kms32,
             # measured HBM bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated) over this run's kernel time
             "traffic_GBps": traffic / (kms32 * 1e-3) / 1e9 if traffic else None,

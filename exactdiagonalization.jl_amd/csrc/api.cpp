@@ -1504,7 +1504,7 @@ bool ensure_diag(edhip_op* op) {
 // spaces: 6x6 FP64 127 -> 91 ms, where the sparser plain form, 18 positions
 // per word, is no faster than the blocked rank index) and x itself does not
 // fit the last-level cache.  scaled: the spread holds
-// x / sqrt(N) on reduced spaces (the products then weigh an image without
+// x sqrt(G / N) on reduced spaces (the products then weigh an image without
 // its orbit size, and their canonicalisers skip counting the stabiliser).
 // Returns whether it did.
 bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const void* x, hipStream_t st,
@@ -1531,7 +1531,7 @@ bool attach_spread(edhip_op* op, int prec, OpDev& d, uint32_t codes_lds, const v
   const edhip_space::XMapHost* X = sp->ensure_xmap(es);
   if (!X) return false;
   const uint16_t* orbit = (scaled && sp->group) ? sp->orbit.as<uint16_t>() : nullptr;
-  HIP_OR_THROW(launch_xmap_fill(prec, X->dev, sp->keys.as<uint64_t>(), sp->dim, x, orbit, st));
+  HIP_OR_THROW(launch_xmap_fill(prec, X->dev, sp->keys.as<uint64_t>(), sp->dim, x, orbit, d.g.G, st));
   d.xm = X->dev;
   d.xm.scaled = orbit ? 1 : 0;
   // every image of a term that keeps the popcount has the space's popcount:
@@ -1679,7 +1679,7 @@ bool ensure_assembled(edhip_op* op, uint64_t max_bytes = ~0ull) {
   return true;
 }
 
-// Row-form product from the assembled rows: x / sqrt(N) first (reduced spaces),
+// Row-form product from the assembled rows: x sqrt(G / N) first (reduced spaces),
 // then the streaming product.
 void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) {
   hipStream_t st = op->ctx->stream;
@@ -1694,7 +1694,7 @@ void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) 
   const void* xt = x;
   if (d.orbit) {
     op->asm_xt.ensure((size_t)(sp->dim + 1) * es);
-    HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, x, op->asm_xt.p, st));
+    HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, d.g.G, x, op->asm_xt.p, st));
     xt = op->asm_xt.p;
   }
   int lanes, batch;
@@ -1747,7 +1747,7 @@ bool rank_product(const edhip_op* op, const OpDev& d) {
                  win_entries_bytes(d.n_lin, d.n_chunk, d.n_rest) <= 64 * 1024;
 }
 
-// Whether it runs the kernel of the torus's point operations, and x / sqrt(N) in
+// Whether it runs the kernel of the torus's point operations, and x sqrt(G / N) in
 // the operator's buffer.
 bool point_product(edhip_op* op, const OpDev& d, int prec, const void* x) {
   const edhip_space* sp = op->space;
@@ -1759,7 +1759,7 @@ bool point_product(edhip_op* op, const OpDev& d, int prec, const void* x) {
     (void)hipGetLastError();
     return false;
   }
-  HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, x, op->asm_xt.p, op->ctx->stream));
+  HIP_OR_THROW(launch_asm_scale(prec, sp->dim, d.orbit, d.g.G, x, op->asm_xt.p, op->ctx->stream));
   return true;
 }
 
@@ -1801,7 +1801,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, X.top_bits, X.top_shift,
                   X.hbits,     nullptr,   nullptr,     0,          0,         sp->pos_bits.as<RankBits>(),
-                  (uint32_t)sp->dim, g.point_swap};
+                  (uint32_t)sp->dim, g.point_swap, g.G};
     HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
   } else if (ranked || window_product(op, d)) {
     const GroupDev& g = d.g;
@@ -1810,7 +1810,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
                   d.stripe,    d.dim,     d.row_begin, sp->n_bits, d.n_lin,   d.n_chunk,  d.n_rest,
                   op->complex_amp ? 0 : 1, d.row_lanes, d.xcd_chunk, accumulate ? 1 : 0, d.xm.top_bits, d.xm.top_shift,
                   d.xm.hbits,  ranked ? sp->rank_low.as<uint16_t>() : nullptr, sp->rank_base.as<uint32_t>(),
-                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes, nullptr, 0, 0};
+                  sp->rank_low_bits, (uint32_t)sp->rank_base.bytes, nullptr, 0, 0, g.G};
     const bool none = g.mode == kGroupNone;
     HIP_OR_THROW(launch_window_product(P, none ? 0 : g.Lx, none ? 0 : g.Ly, none ? 1 : g.unit_phases, prec,
                                        transpose ? 1 : 0, x, y, st));

@@ -26,9 +26,9 @@ hipError_t launch_enumerate_qn(uint64_t count, int n_sites, const QnSite* d_site
 // flags[key >> shift] = 1 for every key
 hipError_t launch_mark_tops(const uint64_t* d_keys, int64_t dim, int shift, uint32_t* d_flags, hipStream_t st);
 // x spread over the word positions of X (before each product); with d_orbit,
-// x / sqrt(orbit) (the orbit factor of the images, X.scaled).
+// x sqrt(G / orbit) (the orbit factor of the images, X.scaled).
 hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, int64_t dim, const void* x,
-                            const uint16_t* d_orbit, hipStream_t st);
+                            const uint16_t* d_orbit, int G, hipStream_t st);
 // Ranks of the words' positions in the spread X, which ascend with the words:
 // n_blocks cleared blocks in.
 hipError_t launch_position_ranks(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t n_blocks,
@@ -149,7 +149,7 @@ struct WinOp {
   const double* ph_im;
   const uint16_t* topcode;
   const uint16_t* colex;
-  const void* values;     // the spread x / sqrt(N)
+  const void* values;     // the spread x sqrt(G / N)
   const uint64_t* lin_tab;
   const MvEntry* ent;
   const OffTerm* rest;
@@ -163,10 +163,11 @@ struct WinOp {
   const uint32_t* rank_base;  // number of sector words with a smaller upper part
   int low_bits;
   uint32_t base_bytes;        // of rank_base, a multiple of 16
-  // point operations (values: x / sqrt(N) itself, 0 at the index none): ranks of the positions
+  // point operations (values: x sqrt(G / N) itself, 0 at the index none): ranks of the positions
   const RankBits* pos_bits;
   uint32_t none;
   int point_swap;
+  int G;                  // order of the group (1: none)
 };
 // Sectors of up to this many bits are ranked by two LDS tables (13 + 13 bits: 48 KiB)
 constexpr int kRankBits = 26;
@@ -238,8 +239,9 @@ hipError_t launch_asm_fill(const OpDev& op, const AsmFillDev& a, hipStream_t st)
 // ranked by position
 hipError_t launch_asm_fill_point(const OpDev& op, const AsmFillDev& a, const XMapDev& X, const RankBits* pos_bits,
                                  uint32_t none, hipStream_t st);
-// xt = x / sqrt(orbit) (orbit != nullptr), in precision prec; xt[dim] = 0
-hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, const void* x, void* xt, hipStream_t st);
+// xt = x sqrt(G / orbit) (orbit != nullptr), in precision prec; xt[dim] = 0
+hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, int G, const void* x, void* xt,
+                            hipStream_t st);
 // y = (accumulate ? y : 0) + A x from the entries; xt = x scaled as above (x itself without orbits);
 // lanes = lanes per row (4, 8, 16 or 32), batch = entries per lane loaded together (4, 8 or 16)
 hipError_t launch_asm_spmv(const OpDev& op, const AsmDev& a, int prec, int lanes, int batch, int accumulate,

@@ -730,8 +730,8 @@ hipError_t launch_expect_v(const OpDev& op, const void* phi, const void* psi, do
 // in the matvec's term order, rows one after another (rowptr).  Class 0 is an
 // image outside the space (weight 0); class c > 0 weighs a * phase, the term's
 // amplitude times the character phase of the element reaching the image.  The
-// orbit factor sqrt(N_r / N_s) is not stored: a product reads x / sqrt(N_s)
-// (prepared once per product) and scales each row's sum by sqrt(N_r).
+// orbit factor sqrt(N_r / N_s) is not stored: a product reads x sqrt(G / N_s)
+// (prepared once per product) and scales each row's sum by sqrt(N_r / G).
 // ---------------------------------------------------------------------------
 
 // counts[r] = number of terms matching row r (the entries it will hold)
@@ -852,15 +852,15 @@ __global__ __launch_bounds__(kMvBlock) void k_asm_fill_point(OpDev op, AsmFillDe
   for (int k = n & 3; k > 0; --k) *out++ = k == 3 ? e[1] : k == 2 ? e[2] : e[3];
 }
 
-// xt[i] = x[i] / sqrt(N_i), xt[dim] = 0 (the element of images outside the space)
+// xt[i] = x[i] sqrt(G / N_i), xt[dim] = 0 (the element of images outside the space)
 template <typename V>
-__global__ __launch_bounds__(kBlock) void k_asm_scale(int64_t dim, const uint16_t* __restrict__ orbit,
+__global__ __launch_bounds__(kBlock) void k_asm_scale(int64_t dim, const uint16_t* __restrict__ orbit, int G,
                                                       const V* __restrict__ x, V* __restrict__ xt) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i == dim) xt[i] = vzero<V>();
   if (i >= dim) return;
   using R = typename VT<V>::R;
-  const double s = 1.0 / sqrt((double)orbit[i]);
+  const double s = sqrt((double)G / (double)orbit[i]);
   V v = x[i];
   if constexpr (VT<V>::cx) {
     v.re = (R)((double)v.re * s);
@@ -880,7 +880,7 @@ __device__ __forceinline__ V vshfl_xor(const V& v, int o, int width) {
   }
 }
 
-// y[r] = (accumulate ? y[r] : 0) + d_r x[r] + sqrt(N_r) sum_e W[cls_e] xt[col_e]:
+// y[r] = (accumulate ? y[r] : 0) + d_r x[r] + sqrt(N_r / G) sum_e W[cls_e] xt[col_e]:
 // GL lanes per row stride over its entries (a wave reads whole runs of
 // neighbouring rows' entries) in batches of U entries per lane, every load of
 // a batch issued before any is used (entries past the row's end are not
@@ -934,7 +934,7 @@ __global__ __launch_bounds__(kAsmBlock) void k_asm_spmv(OpDev op, AsmDev a, cons
   }
   V out = vzero<V>();
   vfma(out, (R)dre, (R)dim_, x[row]);
-  const R so = op.orbit ? (R)sqrt((double)op.orbit[row]) : (R)1;
+  const R so = op.orbit ? (R)sqrt((double)op.orbit[row] / (double)op.g.G) : (R)1;
   vfma(out, so, (R)0, acc);
   y[row] = accumulate ? vadd(y[row], out) : out;
 }
@@ -1049,22 +1049,23 @@ hipError_t launch_asm_fill_point(const OpDev& op, const AsmFillDev& a, const XMa
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, const void* x, void* xt, hipStream_t st) {
+hipError_t launch_asm_scale(int prec, int64_t dim, const uint16_t* d_orbit, int G, const void* x, void* xt,
+                            hipStream_t st) {
   if (dim == 0) return hipSuccess;
   dim3 grid((unsigned)((dim + kBlock) / kBlock));
   switch (prec) {
     case kF64:
-      hipLaunchKernelGGL(k_asm_scale<double>, grid, dim3(kBlock), 0, st, dim, d_orbit, (const double*)x, (double*)xt);
+      hipLaunchKernelGGL(k_asm_scale<double>, grid, dim3(kBlock), 0, st, dim, d_orbit, G, (const double*)x, (double*)xt);
       break;
     case kC128:
-      hipLaunchKernelGGL(k_asm_scale<Cx<double>>, grid, dim3(kBlock), 0, st, dim, d_orbit, (const Cx<double>*)x,
+      hipLaunchKernelGGL(k_asm_scale<Cx<double>>, grid, dim3(kBlock), 0, st, dim, d_orbit, G, (const Cx<double>*)x,
                          (Cx<double>*)xt);
       break;
     case kF32:
-      hipLaunchKernelGGL(k_asm_scale<float>, grid, dim3(kBlock), 0, st, dim, d_orbit, (const float*)x, (float*)xt);
+      hipLaunchKernelGGL(k_asm_scale<float>, grid, dim3(kBlock), 0, st, dim, d_orbit, G, (const float*)x, (float*)xt);
       break;
     case kC64:
-      hipLaunchKernelGGL(k_asm_scale<Cx<float>>, grid, dim3(kBlock), 0, st, dim, d_orbit, (const Cx<float>*)x,
+      hipLaunchKernelGGL(k_asm_scale<Cx<float>>, grid, dim3(kBlock), 0, st, dim, d_orbit, G, (const Cx<float>*)x,
                          (Cx<float>*)xt);
       break;
     default:

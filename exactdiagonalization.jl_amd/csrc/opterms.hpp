@@ -105,8 +105,9 @@ struct MvTerms {
 };
 
 // amp32: the real amplitude is kept as an FP32 value in the low half of its
-// slot.  with_im: imaginary parts are staged.
-__device__ __forceinline__ MvTerms stage_mv_terms(const OpDev& op, unsigned char* lds, bool amp32, bool with_im) {
+// slot.  with_im: imaginary parts are staged.  Amplitudes are staged times scale.
+__device__ __forceinline__ MvTerms stage_mv_terms(const OpDev& op, unsigned char* lds, bool amp32, bool with_im,
+                                                  double scale = 1.0) {
   const MvLayout Y = mv_layout(op.n_lin, op.n_chunk, op.n_rest, op.rest_paired);
   unsigned char* base = lds + op.mv_lds;
   uint64_t* mm = (uint64_t*)(base + Y.off_mm);
@@ -126,7 +127,9 @@ __device__ __forceinline__ MvTerms stage_mv_terms(const OpDev& op, unsigned char
     }
   }
   for (int t = threadIdx.x; t < op.n_lin + op.n_rest; t += blockDim.x) {
-    const MvEntry e = op.ent[t];
+    MvEntry e = op.ent[t];
+    e.are *= scale;
+    e.aim *= scale;
     fa[2 * t] = e.flip;
     fa[2 * t + 1] = amp32 ? (uint64_t)__float_as_uint((float)e.are) : (uint64_t)__double_as_longlong(e.are);
     if (with_im) ai[t] = e.aim;
@@ -180,7 +183,7 @@ __device__ __forceinline__ uint64_t mv_match(const OpDev& op, const MvTerms& T, 
 
 // Weight of an off-diagonal element without the row's own sqrt(N_r), which the
 // products multiply into the finished sum: a * phase^(conj if TRANS) / sqrt(N_img)
-// (SCALED: without 1 / sqrt(N_img), which the spread x / sqrt(N) carries)
+// (SCALED: without 1 / sqrt(N_img), which the spread x sqrt(G / N) carries)
 template <int MODE, bool TRANS, bool UNIT = false, bool SCALED = false>
 __device__ __forceinline__ void element_weight_a(const OpDev& op, const GroupLds& L, double are, double aim, int h,
                                                  int cnt, double& wr, double& wi) {

@@ -34,7 +34,7 @@ __device__ __forceinline__ V row_lanes_sum(V acc, int lg) {
 
 // UNIT: every character is 1 (op.g.unit_phases): the weight needs no phase,
 // so the canonicaliser does not track the element reaching the image.
-// SCALED: x is read from its spread holding x / sqrt(N) (op.xm.scaled), so the
+// SCALED: x is read from its spread holding x sqrt(G / N) (op.xm.scaled), so the
 // weight needs no orbit size of the image and the stabiliser goes uncounted.
 // 2^op.row_lanes lanes share a row and take its matched entries in turn
 // (op.stripe): one lane per row on spaces that fill the chip by themselves,
@@ -48,7 +48,9 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
   // spread) weighs each image in FP32, from FP32 amplitudes and phases of +-1
   // (no FP64 multiply and conversion per image)
   constexpr bool kW32 = SCALED && std::is_same<V, float>::value;
-  const MvTerms T = stage_mv_terms(op, lds, kW32, VT<V>::cx);
+  // the weights of single precision carry sqrt(G) (row_result)
+  constexpr bool kUnitScale = MODE != kGroupNone && (SCALED || std::is_same<typename VT<V>::R, float>::value);
+  const MvTerms T = stage_mv_terms(op, lds, kW32, VT<V>::cx, kUnitScale && !SCALED ? sqrt((double)op.g.G) : 1.0);
   lds_copy(lds + op.mv_w_lds, op.ix.W, op.w_bytes);
   const uint64_t* W = (const uint64_t*)(lds + op.mv_w_lds);
   // code table of the spread x (the host sets xm only with room for it)
@@ -62,7 +64,10 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
   using R = typename VT<V>::R;
   const uint64_t b = op.rows[row];
 
-  V acc = vzero<V>();
+  // single precision sums the two images of a step apart (k_product_win); without
+  // the spread the registers of a second sum would cost a wave (6x6, C64)
+  constexpr bool kTwoSums = SCALED && std::is_same<R, float>::value;
+  V sums[2] = {vzero<V>(), vzero<V>()};
   const int n_seg = mv_segments(op);
   for (int seg = 0; seg < n_seg; ++seg) {
     int base;
@@ -112,18 +117,18 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
           if constexpr (kW32) {
             float w = __uint_as_float((uint32_t)fa[k].y);
             if constexpr (!UNIT) w *= (float)L.ph_re[hk[k]];
-            vfma(acc, w, 0.f, xv[k]);
+            vfma(sums[kTwoSums ? k : 0], w, 0.f, xv[k]);
           } else {
             double wr, wi;
             element_weight_a<MODE, TRANS, UNIT, SCALED>(op, L, __longlong_as_double((long long)fa[k].y),
                                                         VT<V>::cx ? T.ai[t[k]] : 0.0, hk[k], ck[k], wr, wi);
-            vfma(acc, (R)wr, (R)wi, xv[k]);
+            vfma(sums[kTwoSums ? k : 0], (R)wr, (R)wi, xv[k]);
           }
         }
       }
     }
   }
-  acc = row_lanes_sum(acc, op.row_lanes);
+  const V acc = row_lanes_sum(kTwoSums ? vadd(sums[0], sums[1]) : sums[0], op.row_lanes);
   if (sub != 0) return;
   // diagonal terms (C == R): the element is the summed amplitude (U[b]/U[b] = 1)
   double dre = 0.0, dim_ = 0.0;
@@ -133,12 +138,15 @@ __global__ __launch_bounds__(kMvBlock) void k_matvec(OpDev op, const V* __restri
   } else {
     diag_sum(op, b, dre, dim_);
   }
-  V out = vzero<V>();
-  vfma(out, (R)dre, (R)dim_, x[row]);
-  if constexpr (MODE != kGroupNone)
-    vfma(out, (R)sqrt((double)op.orbit[row]), (R)0, acc);
-  else
+  V out;
+  if constexpr (MODE != kGroupNone) {
+    const double n = kUnitScale ? (double)op.orbit[row] / (double)op.g.G : (double)op.orbit[row];
+    out = row_result(dre, dim_, x[row], sqrt(n), acc);
+  } else {
+    out = vzero<V>();
+    vfma(out, (R)dre, (R)dim_, x[row]);
     out = vadd(out, acc);
+  }
   V* yr = y + (row - op.row_begin);
   *yr = accumulate ? vadd(*yr, out) : out;
 }
@@ -174,7 +182,7 @@ struct PointEntry {
 };
 
 // The product for translation groups on the shapes of window.hpp, x read from
-// its colex spread x / sqrt(N) (XMapDev: every image keeps the popcount, narrow).
+// its colex spread x sqrt(G / N) (XMapDev: every image keeps the popcount, narrow).
 // It is bound by instruction issue and by the line fills of the x gathers
 // together, so what counts is the number of instructions per image: the shape,
 // the word width (32 bits up to 32 sites) and the LDS offsets are fixed at
@@ -192,7 +200,7 @@ struct PointEntry {
 // KIND = kWinPoint: translations and point operations.  These spaces are 8
 // times sparser in their words, so a spread would take a line per state (6x6
 // A1, FP64: 8.2 GB for 31.6M states): the position of the spread is ranked
-// through bits instead (RankBits, 258 MB beside x / sqrt(N) itself).
+// through bits instead (RankBits, 258 MB beside x sqrt(G / N) itself).
 template <typename V, int KIND, int LX, int LY, bool UNIT, bool TRANS, bool RANK = false>
 __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __restrict__ x, V* __restrict__ y) {
   using S = Win<KIND, LX, LY>;
@@ -270,15 +278,19 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
     const uint32_t hc = (c << P.hbits) | __builtin_amdgcn_ubfe(lo, 12u, (uint32_t)P.hbits);
     return __umul24(hc, 924u) + (uint32_t)colex[lo & 0xfffu];
   };
-  auto fetch = [&](W s) {  // x (/ sqrt(N)) of the canonical word s
+  auto fetch = [&](W s) {  // x (sqrt(G / N)) of the canonical word s
     if constexpr (RANK) {
       const uint32_t lo = (uint32_t)s & ((1u << P.low_bits) - 1u);
       return x[lds_at<uint32_t>(rank_low)[s >> P.low_bits] + (uint32_t)lds_at<uint16_t>(0)[lo]];
     }
     return ((const V*)P.values)[(uint64_t)position(s)];
   };
-  V acc = vzero<V>();
-  auto add = [&](const V& xv, int t, const E& e, int bit) {
+  // single precision sums the two images of a step apart: half as many roundings in
+  // either sum (5x6 (1,2), C64, x > 0: 1.44e-7 off in the norm with one sum, 9e-8
+  // with two)
+  constexpr bool kTwoSums = std::is_same<R, float>::value;
+  V sums[2] = {vzero<V>(), vzero<V>()};
+  auto add = [&](V& acc, const V& xv, int t, const E& e, int bit) {
     if constexpr (UNIT) {
       if (!CX || P.real_amp) {
         if constexpr (CX) {
@@ -372,20 +384,23 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
 #pragma unroll
         for (int k = 0; k < NW; ++k) xv[k] = fetch(s[k]);
       }
-      add(xv[0], t[0], e[0], w[0]);
+      add(sums[0], xv[0], t[0], e[0], w[0]);
 #pragma unroll
       for (int k = 1; k < NW; ++k)
-        if (ok[k]) add(xv[k], t[k], e[k], w[k]);
+        if (ok[k]) add(sums[kTwoSums ? k : 0], xv[k], t[k], e[k], w[k]);
     }
   }
-  acc = row_lanes_sum(acc, P.row_lanes);
+  const V acc = row_lanes_sum(kTwoSums ? vadd(sums[0], sums[1]) : sums[0], P.row_lanes);
   if (sub != 0) return;
   V out = vzero<V>();
-  if (P.diag_re) vfma(out, (R)P.diag_re[row], (R)(P.diag_im ? P.diag_im[row] : 0.0), x[row]);
-  if constexpr (KIND != kWinNone)
-    vfma(out, (R)sqrt((double)P.orbit[row]), (R)0, acc);
-  else
+  if constexpr (KIND != kWinNone) {
+    const bool diag = P.diag_re != nullptr;
+    out = row_result(diag ? P.diag_re[row] : 0.0, diag && P.diag_im ? P.diag_im[row] : 0.0, diag ? x[row] : out,
+                     sqrt((double)P.orbit[row] / (double)P.G), acc);
+  } else {
+    if (P.diag_re) vfma(out, (R)P.diag_re[row], (R)(P.diag_im ? P.diag_im[row] : 0.0), x[row]);
     out = vadd(out, acc);
+  }
   V* yr = y + (row - P.row_begin);
   *yr = P.accumulate ? vadd(*yr, out) : out;
 }

@@ -397,15 +397,15 @@ __global__ __launch_bounds__(kBlock) void k_mark_tops(const uint64_t* __restrict
 // Before a product: x spread over the word positions (XMapDev).
 template <typename V>
 __global__ __launch_bounds__(kBlock) void k_xmap_fill(XMapDev X, const uint64_t* __restrict__ keys, int64_t dim,
-                                                      const V* __restrict__ x, const uint16_t* __restrict__ orbit) {
+                                                      const V* __restrict__ x, const uint16_t* __restrict__ orbit, int G) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= dim) return;
   const uint64_t k = keys[i];
   const uint64_t pos = xmap_pos(X, X.colex, X.topcode[k >> X.top_shift], k);
   V v = x[i];
-  if (orbit) {  // x / sqrt(N), scaled in double
+  if (orbit) {  // x sqrt(G / N), scaled in double
     using R = typename VT<V>::R;
-    const double sc = 1.0 / sqrt((double)orbit[i]);
+    const double sc = sqrt((double)G / (double)orbit[i]);
     if constexpr (VT<V>::cx) {
       v.re = (R)((double)v.re * sc);
       v.im = (R)((double)v.im * sc);
@@ -527,23 +527,23 @@ hipError_t launch_mark_tops(const uint64_t* d_keys, int64_t dim, int shift, uint
 }
 
 hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, int64_t dim, const void* x,
-                            const uint16_t* d_orbit, hipStream_t st) {
+                            const uint16_t* d_orbit, int G, hipStream_t st) {
   if (dim == 0) return hipSuccess;
   dim3 grid(grid_for((uint64_t)dim));
   switch (prec) {
     case kF64:
-      hipLaunchKernelGGL(k_xmap_fill<double>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const double*)x, d_orbit);
+      hipLaunchKernelGGL(k_xmap_fill<double>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const double*)x, d_orbit, G);
       break;
     case kC128:
       hipLaunchKernelGGL(k_xmap_fill<Cx<double>>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const Cx<double>*)x,
-                         d_orbit);
+                         d_orbit, G);
       break;
     case kF32:
-      hipLaunchKernelGGL(k_xmap_fill<float>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const float*)x, d_orbit);
+      hipLaunchKernelGGL(k_xmap_fill<float>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const float*)x, d_orbit, G);
       break;
     case kC64:
       hipLaunchKernelGGL(k_xmap_fill<Cx<float>>, grid, dim3(kBlock), 0, st, X, d_keys, dim, (const Cx<float>*)x,
-                         d_orbit);
+                         d_orbit, G);
       break;
     default:
       return hipErrorInvalidValue;
