@@ -1243,15 +1243,16 @@ uint32_t rank_table_bytes(const edhip_space* sp) {
   return sp->is_sector && !sp->group ? (uint32_t)((sp->n_bits + 1) * (sp->n_bits + 1) * 8) : 0u;
 }
 
-// Whether the tables of the products' entries leave no LDS room where the plain
-// list of the terms still does.
-bool mv_no_room(const edhip_op* op, int form) {
+// The LDS room of an operator's terms, row form (0) or column form (1).
+LdsPlan op_lds_plan(const edhip_op* op, int form) {
   const edhip_space* sp = op->space;
-  const uint32_t group_bytes = align_up(sp->group ? sp->group->lay.total : 0u, 16), w_bytes = rank_table_bytes(sp);
-  const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
+  GroupLdsLayout lay{};
+  if (sp->group) lay = sp->group->lay;
+  const uint32_t group = align_up(lay.total, 16);
+  const bool pairs = sp->group && sp->group->dev.pair_table;
   const MvLayout full = mv_layout(op->mv[form].n_lin, mv_chunks(sp->word_bits()), op->mv[form].n_rest, 1);
-  return group_bytes + std::max(full.total, plain_bytes) + w_bytes > 64 * 1024 &&
-         group_bytes + plain_bytes + w_bytes <= 64 * 1024;
+  return lds_plan(group, pairs ? align_up(lay.off_pair, 16) : group,
+                  align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16), align_up(full.total, 16), rank_table_bytes(sp));
 }
 
 OpDev make_opdev(edhip_op* op, bool transpose) {
@@ -1281,10 +1282,10 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   d.diag = op->diag.as<DiagTerm>();
   const uint32_t w_bytes = rank_table_bytes(sp);
   const uint32_t plain_bytes = align_up((uint32_t)(op->n_off * sizeof(OffTerm)), 16);
-  const uint32_t group_bytes = align_up(d.lay.total, 16);
   const int form = transpose ? 1 : 0;
   d.n_chunk = mv_chunks(sp->word_bits());
-  const bool no_room = mv_no_room(op, form);
+  const LdsPlan plan = op_lds_plan(op, form);
+  const bool no_room = plan.one_by_one;
   const auto& mv = no_room ? op->mv_plain[form] : op->mv[form];
   d.ent = mv.ent.as<MvEntry>();
   d.lin_tab = mv.tab.as<uint64_t>();
@@ -1294,7 +1295,7 @@ OpDev make_opdev(edhip_op* op, bool transpose) {
   d.rest_paired = no_room ? 0 : 1;
   d.stripe = ~0ull;
   const uint32_t mv_bytes = align_up(mv_layout(d.n_lin, d.n_chunk, d.n_rest, d.rest_paired).total, 16);
-  if (d.g.pair_table && group_bytes + std::max(plain_bytes, mv_bytes) + w_bytes > 64 * 1024) {
+  if (plan.drop_pairs) {
     // not enough LDS next to this operator's terms: use the per-row table path
     d.g.pair_table = 0;
     d.lay.bytes_pair = 0;
@@ -2844,7 +2845,7 @@ int edhip_op_create(edhip_ctx* ctx, const edhip_space* space, int64_t n_terms, c
       upload(M.tab, mv_tables(S, space->word_bits()), ctx->stream);
       upload(M.rest, S.rest, ctx->stream);
       upload(M.ent, M.entries, ctx->stream);
-      if (mv_no_room(op.get(), form)) {
+      if (op_lds_plan(op.get(), form).one_by_one) {
         edhip_op::MvHost& P = op->mv_plain[form];
         P.n_rest = (int)v.size();
         for (const OffTerm& o : v) P.entries.push_back(MvEntry{o.match ^ o.image, o.are, o.aim});

@@ -280,6 +280,36 @@ inline std::vector<uint64_t> mv_tables(const MvSplit& S, int nb) {
   return tab;
 }
 
+// LDS offsets of the products' entries, from mv_lds.
+struct MvLayout {
+  uint32_t off_mm, off_fa, off_ai, total;
+};
+EDHIP_HD MvLayout mv_layout(int n_lin, int n_chunk, int n_rest, int paired) {
+  MvLayout Y;
+  Y.off_mm = (uint32_t)(((n_lin + 63) / 64) * n_chunk) * 128u;
+  Y.off_fa = (Y.off_mm + (uint32_t)(paired ? n_rest / 2 * 24 : n_rest * 16) + 15u) & ~15u;
+  Y.off_ai = Y.off_fa + (uint32_t)(n_lin + n_rest) * 16u;
+  Y.total = Y.off_ai + (uint32_t)(n_lin + n_rest) * 8u;
+  return Y;
+}
+
+// How an operator's terms find room in the 64 KiB of LDS beside its group's tables
+// (group bytes, fewer without the row-pair table) and the rank table (rank bytes):
+// plain, the list of the terms, always staged by the kernels that walk it, and full,
+// the products' entries with their tables.  Entries, else the terms one by one, else
+// the same without the row-pair table; what is accepted is decided by the plain list
+// alone.
+struct LdsPlan {
+  bool one_by_one, drop_pairs;
+};
+inline LdsPlan lds_plan(uint32_t group, uint32_t group_without_pairs, uint32_t plain, uint32_t full, uint32_t rank) {
+  const uint32_t most = std::max(plain, full);
+  auto fits = [&](uint32_t g, uint32_t terms) { return g + terms + rank <= 64u * 1024u; };
+  if (fits(group, most)) return {false, false};
+  if (fits(group, plain)) return {true, false};
+  return {!fits(group_without_pairs, most) && fits(group_without_pairs, plain), group_without_pairs != group};
+}
+
 // Diagonal term: adds its amplitude to the rows b with (b & mask) == match.
 struct DiagTerm {
   uint64_t mask, match;

@@ -81,19 +81,6 @@ hipError_t exclusive_scan_i64(const int64_t* d_in, int64_t* d_out, uint64_t n, v
                               hipStream_t st);
 
 // ---- matvec.hip, product_*.hip ---------------------------------------------
-// LDS offsets of the products' entries, from mv_lds.
-struct MvLayout {
-  uint32_t off_mm, off_fa, off_ai, total;
-};
-__host__ __device__ __forceinline__ MvLayout mv_layout(int n_lin, int n_chunk, int n_rest, int paired) {
-  MvLayout Y;
-  Y.off_mm = (uint32_t)(((n_lin + 63) / 64) * n_chunk) * 128u;
-  Y.off_fa = (Y.off_mm + (uint32_t)(paired ? n_rest / 2 * 24 : n_rest * 16) + 15u) & ~15u;
-  Y.off_ai = Y.off_fa + (uint32_t)(n_lin + n_rest) * 16u;
-  Y.total = Y.off_ai + (uint32_t)(n_lin + n_rest) * 8u;
-  return Y;
-}
-
 struct OpDev {
   IndexDev ix;           // lookup of canonical images
   GroupDev g;            // symmetry group
