@@ -171,11 +171,24 @@ __device__ __forceinline__ uint32_t rank_of(RankBits r, uint32_t pos, uint32_t n
 // alone hold it from address 0: as an address space 3 pointer made from the
 // offset, a table at an offset known at compile time costs no address
 // arithmetic (through the extern array every read adds its base, 0, first).
+// Their launches ask lds_from_zero.
 template <typename T>
 using LdsPtr = const __attribute__((address_space(3))) T*;
 template <typename T>
 __device__ __forceinline__ LdsPtr<T> lds_at(uint32_t offset) {
   return (LdsPtr<T>)offset;
+}
+
+// Whether the kernel has dynamic LDS alone, as lds_at needs (asked of the runtime
+// once per kernel): a __shared__ variable would take address 0.
+template <auto Kernel>
+inline hipError_t lds_from_zero() {
+  static const hipError_t error = [] {
+    hipFuncAttributes a{};
+    const hipError_t e = hipFuncGetAttributes(&a, reinterpret_cast<const void*>(Kernel));
+    return e != hipSuccess ? e : a.sharedSizeBytes != 0 ? hipErrorInvalidConfiguration : hipSuccess;
+  }();
+  return error;
 }
 
 // ----------------------------------------------------------------------------

@@ -259,6 +259,7 @@ hipError_t launch_rank_v(const ExpectRank& E, const OpDev& op, const void* phi, 
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (E.n_steps > 0) {
+    if ((e = lds_from_zero<k_expect_steps<V, KT>>()) != hipSuccess) return e;
     const int windows = E.n_steps / KT;
     const int64_t blocks = expect_rank_blocks(op.dim, windows);
     const uint32_t tables = (2u << E.low_bits) + E.base_bytes, sums = kMvBlock / 64 * KT * 4 * 8;

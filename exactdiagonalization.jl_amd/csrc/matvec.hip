@@ -1035,6 +1035,8 @@ hipError_t launch_asm_fill_point(const OpDev& op, const AsmFillDev& a, const XMa
   OpDev o = op;
 #define EDHIP_FILL(L, U)                                                                                         \
   {                                                                                                              \
+    const hipError_t e = lds_from_zero<k_asm_fill_point<L, U>>();                                                \
+    if (e != hipSuccess) return e;                                                                               \
     o.mv_lds = Win<kWinPoint, L, L>::kTabBytes + kXCodesBytesMax + 2u * 4096u;                                   \
     const uint32_t lds = o.mv_lds + mv_layout(o.n_lin, o.n_chunk, o.n_rest, o.rest_paired).total +               \
                          8u * (uint32_t)(o.n_lin + o.n_rest);                                                    \
@@ -1108,6 +1110,8 @@ hipError_t launch_diag_values(const OpDev& op, double* d_re, double* d_im, hipSt
 
 hipError_t launch_diag_parity(const DiagParity& P, const uint64_t* d_rows, int64_t dim, double* d_re, hipStream_t st) {
   if (dim == 0) return hipSuccess;
+  const hipError_t e = lds_from_zero<k_diag_parity>();
+  if (e != hipSuccess) return e;
   const int64_t blocks = (dim + 4 * kBlock - 1) / (4 * kBlock);  // (4 rows a lane, for the staging)
   hipLaunchKernelGGL(k_diag_parity, dim3((unsigned)blocks), dim3(kBlock), (uint32_t)(P.n_seg * P.n_chunk) * 128u, st, P,
                      d_rows, dim, d_re);

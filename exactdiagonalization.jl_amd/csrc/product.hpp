@@ -405,6 +405,14 @@ __global__ __launch_bounds__(kMvBlock) void k_product_win(WinOp P, const V* __re
   *yr = P.accumulate ? vadd(*yr, out) : out;
 }
 
+template <auto Kernel, typename V>
+hipError_t launch_win_kernel(dim3 grid, uint32_t lds, hipStream_t st, const WinOp& P, const void* x, void* y) {
+  const hipError_t e = lds_from_zero<Kernel>();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(Kernel, grid, dim3(kMvBlock), lds, st, P, (const V*)x, (V*)y);
+  return hipGetLastError();
+}
+
 template <typename V, int KIND, int LX, int LY>
 hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, void* y, hipStream_t st) {
   const uint64_t lanes = (uint64_t)(P.dim - P.row_begin) << P.row_lanes;
@@ -413,16 +421,10 @@ hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, 
       win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest) + (KIND == kWinPoint ? 8u * (uint32_t)(P.n_lin + P.n_rest + 1) : 0u);
   // the column form only conjugates the phase
   constexpr bool kT = VT<V>::cx;
-  if (unit)
-    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, true, false>), grid, dim3(kMvBlock),
-                       (WinLds<KIND, LX, LY, true>::entries + dyn), st, P, (const V*)x, (V*)y);
-  else if (transpose)
-    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, false, kT>), grid, dim3(kMvBlock),
-                       (WinLds<KIND, LX, LY, false>::entries + dyn), st, P, (const V*)x, (V*)y);
-  else
-    hipLaunchKernelGGL((k_product_win<V, KIND, LX, LY, false, false>), grid, dim3(kMvBlock),
-                       (WinLds<KIND, LX, LY, false>::entries + dyn), st, P, (const V*)x, (V*)y);
-  return hipGetLastError();
+  if (unit) return launch_win_kernel<k_product_win<V, KIND, LX, LY, true, false>, V>(grid, WinLds<KIND, LX, LY, true>::entries + dyn, st, P, x, y);
+  constexpr uint32_t below = WinLds<KIND, LX, LY, false>::entries;
+  if (transpose) return launch_win_kernel<k_product_win<V, KIND, LX, LY, false, kT>, V>(grid, below + dyn, st, P, x, y);
+  return launch_win_kernel<k_product_win<V, KIND, LX, LY, false, false>, V>(grid, below + dyn, st, P, x, y);
 }
 
 template <typename V>
@@ -449,15 +451,11 @@ hipError_t launch_win_other(const WinOp& P, int Lx, int Ly, int unit, int transp
     const uint32_t dyn = win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest);
     constexpr uint32_t fixed = WinLds<kWinNone, 32, 1, true>::entries;
     if (P.rank_low)
-      hipLaunchKernelGGL((k_product_win<V, kWinNone, 32, 1, true, false, true>), grid, dim3(kMvBlock),
-                         ((2u << P.low_bits) + P.base_bytes + dyn), st, P, (const V*)x, (V*)y);
-    else if (P.n_bits <= 32)
-      hipLaunchKernelGGL((k_product_win<V, kWinNone, 32, 1, true, false>), grid, dim3(kMvBlock), (fixed + dyn), st, P,
-                         (const V*)x, (V*)y);
-    else
-      hipLaunchKernelGGL((k_product_win<V, kWinNone, 64, 1, true, false>), grid, dim3(kMvBlock), (fixed + dyn), st, P,
-                         (const V*)x, (V*)y);
-    return hipGetLastError();
+      return launch_win_kernel<k_product_win<V, kWinNone, 32, 1, true, false, true>, V>(
+          grid, (2u << P.low_bits) + P.base_bytes + dyn, st, P, x, y);
+    if (P.n_bits <= 32)
+      return launch_win_kernel<k_product_win<V, kWinNone, 32, 1, true, false>, V>(grid, fixed + dyn, st, P, x, y);
+    return launch_win_kernel<k_product_win<V, kWinNone, 64, 1, true, false>, V>(grid, fixed + dyn, st, P, x, y);
   }
   if (Ly == 1 && Lx <= 32) return launch_win_t<V, kWinChain, 32, 1>(P, unit, transpose, x, y, st);
   if (Ly == 1 && Lx <= 48) return launch_win_t<V, kWinChain, 48, 1>(P, unit, transpose, x, y, st);

@@ -209,6 +209,8 @@ hipError_t launch_reduce_win(const ReduceSource& src, uint64_t chunk, uint64_t n
   const dim3 grid((unsigned)((n_threads + kBlock - 1) / kBlock));
   const uint32_t w = (uint32_t)((src.n_bits + 1) * (src.n_bits + 1) * 8);
 #define EDHIP_REDUCE(K, X, Y)                                                                                        \
+  const hipError_t e = lds_from_zero<k_reduce_win<K, X, Y, WRITE>>();                                                \
+  if (e != hipSuccess) return e;                                                                                     \
   hipLaunchKernelGGL((k_reduce_win<K, X, Y, WRITE>), grid, dim3(kBlock), (Win<K, X, Y>::kTabBytes + 64 + w), st, src, \
                      chunk, n_threads, g, counts, offsets, reps, orbits);                                            \
   return hipGetLastError();
