@@ -121,6 +121,7 @@ SIGNATURES = {
     "edhip_set_stream": (_i32, [_vp, _vp]),
     "edhip_get_stream": (_i32, [_vp, _P(_vp)]),
     "edhip_debug_fail_allocs": (_i32, [_i32, _i32]),
+    "edhip_debug_paths": (_i32, [_vp, _P(_i32), _P(_i32)]),
     "edhip_debug_asm_shape": (_i32, [_i32, _i32]),
     "edhip_debug_block_order": (_i32, [_i32]),
     "edhip_synchronize": (_i32, [_vp]),

@@ -1189,6 +1189,7 @@ struct edhip_op {
   int strat_kernel = 0;  // 0 auto, 1 term list, 2 pair groups, 3 assembled rows
   int strat_lookup = 0;  // 0 auto, 1 sorted search (or rank), 2 hash table
   int used_kernel = 0, used_lookup = 0;
+  int product_path = 0, term_path = 0;  // edhip_debug_paths
   double kt_ms = 0.0;  // summed durations of the timed matvec and term-pass kernel launches
   int64_t kt_n = 0;
   // assembled rows of the row form (strategy 3), built on first use
@@ -1781,6 +1782,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
     d.diag_im = op->diag_im.as<double>();
   }
   op->used_kernel = 1;
+  op->product_path = EDHIP_PATH_GENERAL;
   const bool point = idx_lookup == 0 && point_product(op, d, prec, x);
   if (!point) d.ix = sp->index_dev(idx_lookup == 4 ? 0 : idx_lookup);
   // two lanes to a row at least: with half the rows in flight more of the two
@@ -1795,6 +1797,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   if (idx_lookup == 4 && !d.xm.values) fail(EDHIP_ERR_ARGUMENT, "x cannot be spread over the words of this space");
   if (op->ctx->kernel_timing) HIP_OR_THROW(hipEventRecord(op->ctx->ev[14], st));
   if (point) {
+    op->product_path = EDHIP_PATH_POINT;
     const GroupDev& g = d.g;
     const XMapDev& X = sp->pos_dev;
     const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.point_tab, g.point_elem, g.ph_re,
@@ -1805,6 +1808,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
                   (uint32_t)sp->dim, g.point_swap, g.G};
     HIP_OR_THROW(launch_window_product(P, g.Lx, g.Ly, g.unit_phases, prec, transpose ? 1 : 0, x, y, st));
   } else if (ranked || window_product(op, d)) {
+    op->product_path = ranked ? EDHIP_PATH_RANK : EDHIP_PATH_SHAPE;
     const GroupDev& g = d.g;
     const WinOp P{d.rows,      d.orbit,   d.diag_re,   d.diag_im,  g.win_tab, g.win_elem, g.ph_re,
                   g.ph_im,     d.xm.topcode, d.xm.colex, d.xm.values, d.lin_tab, d.ent,      d.rest,
@@ -3377,6 +3381,7 @@ int edhip_term_expect(edhip_op* op, int prec, const void* phi, const void* psi, 
     OpDev d = op->dev_row;
     ExpectRank E{};
     const bool ranked = expect_by_rank(op, E);
+    op->term_path = ranked ? EDHIP_PATH_RANK : EDHIP_PATH_GENERAL;
     if (ranked) {
       const size_t x = (size_t)E.n_upper * (1 + 2 * E.low_bits) * 2, q = ((size_t)kExpectSplits << E.low_bits) * 2;
       op->ex_sums.ensure((x + q) * 8);
@@ -3591,6 +3596,13 @@ int edhip_debug_fail_allocs(int kinds, int count) {
   g_fail_count.store(0);
   g_fail_kinds.store(kinds);
   g_fail_count.store(count);
+  return EDHIP_OK;
+}
+
+int edhip_debug_paths(const edhip_op* op, int* product, int* term_pass) {
+  if (!op || !product || !term_pass) return EDHIP_ERR_ARGUMENT;
+  *product = op->product_path;
+  *term_pass = op->term_path;
   return EDHIP_OK;
 }
 

@@ -423,6 +423,16 @@ int edhip_event_elapsed(edhip_ctx* ctx, int slot0, int slot1, double* ms);
 #define EDHIP_ALLOC_WORKSPACE 2
 #define EDHIP_ALLOC_ASSEMBLED 4
 int edhip_debug_fail_allocs(int kinds, int count);
+/* Testing (no counterpart in the reference): which kernels ran in the operator's
+ * last term-list product and its last term pass (0: none so far): the general
+ * ones, those of a torus's or chain's shape or of a sector without a group
+ * through the spread, those of a square torus's point operations, or those of
+ * a sector without a group by rank. */
+#define EDHIP_PATH_GENERAL 1
+#define EDHIP_PATH_SHAPE 2
+#define EDHIP_PATH_POINT 3
+#define EDHIP_PATH_RANK 4
+int edhip_debug_paths(const edhip_op* op, int* product, int* term_pass);
 /* Tuning (no counterpart in the reference): lanes per row of the
  * assembled-row product, 4, 8, 16 or 32, and entries each lane loads
  * together, 4, 8 or 16 (0: the defaults, lanes chosen from the mean entries

@@ -40,7 +40,7 @@ def _bonds(ed, n, shape):
 
 # rank tables of both sizes, the spread without a group, translations in 32- and
 # 64-bit words, chains, point operations
-CASES = [(16, 8, None, None), (24, 4, None, None), (25, 3, None, None), (26, 3, None, None), (28, 3, None, None),
+CASES = [(16, 8, None, None), (24, 4, None, None), (25, 3, None, None), (26, 3, None, None), (28, 3, None, None), (27, 7, None, None),
          (16, 8, (4, 4), (1, 2)), (24, 5, (4, 6), (0, 0)), (25, 4, (5, 5), (1, 0)), (36, 3, (6, 6), (2, 0)),
          (13, 6, (13, 1), 3), (33, 3, (33, 1), 0), (25, 4, (5, 5), "A1"), (36, 4, (6, 6), "B1")]
 
@@ -80,7 +80,7 @@ def _forms(oracle, ospace, terms, phi, psi):
                      for t in range(len(mask))])
 
 
-@pytest.mark.parametrize("n,up,shape,k", [CASES[i] for i in (0, 1, 3, 4, 5, 9)])
+@pytest.mark.parametrize("n,up,shape,k", [CASES[i] for i in (0, 1, 3, 4, 6, 10)])
 def test_term_pass(ed, oracle, n, up, shape, k):
     import torch
 
