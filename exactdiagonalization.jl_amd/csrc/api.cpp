@@ -3097,6 +3097,7 @@ int edhip_sparse_export_csc(edhip_op* op, int index_bytes, void* colptr, void* r
     if (op->sp_nnz < 0) fail(EDHIP_ERR_ARGUMENT, "call edhip_sparse_build first");
     const int64_t d = op->space->dim, nnz = op->sp_nnz;
     if (index_bytes != 4 && index_bytes != 8) fail(EDHIP_ERR_ARGUMENT, "indices take 4 or 8 bytes");
+    if (!colptr || (nnz > 0 && (!rowval || !values))) fail(EDHIP_ERR_ARGUMENT, "null output");
     if (index_bytes == 4 && (nnz > 0x7fffffffll || d > 0x7fffffffll))
       fail(EDHIP_ERR_ARGUMENT, "the matrix needs 8-byte indices");
     hipStream_t st = op->ctx->stream;
