@@ -111,9 +111,9 @@ struct DevBuf {
 // memory of their own as always.
 //
 // The device memory is a part of a slab that the objects made one after the other
-// share (an operator on 8 sites: 21 kB of its own instead of a 256 kB block); a slab
-// is freed with the last of them.  Parts are never used again before that, so no
-// kernel still reading one needs to be waited for when its object ends.
+// share (operators and reductions on 8 sites: 10 and 21 kB each); a slab is freed
+// with the last of them.  Parts are never used again before that, so no kernel still
+// reading one needs to be waited for when its object ends.
 constexpr size_t kSlabBytes = 256 * 1024;
 struct Slab {
   DevBuf dev;

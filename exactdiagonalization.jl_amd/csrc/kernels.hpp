@@ -29,8 +29,8 @@ hipError_t launch_mark_tops(const uint64_t* d_keys, int64_t dim, int shift, uint
 // x sqrt(G / orbit) (the orbit factor of the images, X.scaled).
 hipError_t launch_xmap_fill(int prec, const XMapDev& X, const uint64_t* d_keys, int64_t dim, const void* x,
                             const uint16_t* d_orbit, int G, hipStream_t st);
-// Ranks of the words' positions in the spread X, which ascend with the words:
-// n_blocks cleared blocks in.
+// Ranks of the words' positions in the spread X, which ascend with the words, in
+// n_blocks blocks, which it clears first.
 hipError_t launch_position_ranks(const XMapDev& X, const uint64_t* d_keys, int64_t dim, uint64_t n_blocks,
                                  RankBits* d_bits, hipStream_t st);
 // prefix[j] = lower_bound(keys, j << shift), j <= n_buckets

@@ -28,8 +28,10 @@ namespace edhip {
 
 enum WinKind : int { kWinNone = 0, kWinPairs = 1, kWinRows = 2, kWinChain = 3, kWinPoint = 4 };
 
-// Shapes compiled as their own kernels (lattices of up to 36 sites on which
-// products take long enough to matter; others run the general kernels).
+// Shapes compiled as their own kernels: tori of 16 to 36 sites with 3 to 8 rows of
+// 3 to 8 bits, the most that a candidate mask holds (a byte per row, a bit per
+// rotation) and the fewest that the windows pay for.  Longer and narrower ones (4x9,
+// 2xN ladders) run the general kernels, as do smaller ones.
 #define EDHIP_WIN_SHAPES(X)                                                                                       \
   X(kWinPairs, 3, 6) X(kWinPairs, 3, 7) X(kWinPairs, 3, 8) X(kWinPairs, 4, 4) X(kWinPairs, 4, 5) X(kWinPairs, 4, 6) \
   X(kWinPairs, 4, 7) X(kWinPairs, 4, 8) X(kWinPairs, 5, 4) X(kWinPairs, 5, 5) X(kWinPairs, 5, 6) X(kWinPairs, 5, 7) \

@@ -441,7 +441,9 @@ int edhip_debug_asm_shape(int lanes, int batch);
 /* Tuning (no counterpart in the reference): block order of the products
  * (term-list and assembled-row kernels).  Workgroups go to the 8 XCDs in
  * turn; with chunk C > 1 each XCD takes C consecutive blocks of every window
- * of 8 C blocks (0 or 1: plain order; at most 64; default 32).
+ * of 8 C blocks (0 or 1: plain order).  chunk is the C of small grids (at most
+ * 64; default 32): C doubles up to four times while the grid still holds 8
+ * whole windows.
  * Process-wide; every order gives the same results. */
 int edhip_debug_block_order(int chunk);
 
