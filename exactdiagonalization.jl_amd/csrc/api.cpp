@@ -1721,10 +1721,16 @@ void asm_matvec(edhip_op* op, int prec, int accumulate, const void* x, void* y) 
 // with 8; 5x6, 5.2M rows: 2072 us with 1, 2360 with 2.  The rule looks at the
 // whole space, not at the rows computed, so that a share of the rows is bitwise
 // the same as in the whole product.
-constexpr int64_t kMvLanes = 1 << 18;
-int mv_row_lanes(int64_t dim, int entries) {
+// Entries matched by mask are tested by each lane of the row, so that more lanes
+// add work: there the rows are split up to 2^16 lanes (kernel, us, with 1, 2, 4, 8
+// lanes: t-J chain of 14 sites, 60,060 rows and 84 such entries 24.3, 21.8, 22.8,
+// 30.7; spin-1 chain of 12, 73,789 rows and 96 entries 16.3, 17.3, 18.8, 24.5; of
+// 10, 8,953 rows 14.2, 12.7, 11.4, 11.6).
+constexpr int64_t kMvLanes = 1 << 18, kMvLanesMasks = 1 << 16;
+int mv_row_lanes(int64_t dim, int n_lin, int n_rest) {
+  const int64_t enough = n_rest > n_lin ? kMvLanesMasks : kMvLanes;
   int lg = 0;
-  while (lg < 4 && (dim << lg) < kMvLanes && (4 << lg) <= entries) ++lg;
+  while (lg < 4 && (dim << lg) < enough && (4 << lg) <= n_lin + n_rest) ++lg;
   return lg;
 }
 
@@ -1776,7 +1782,7 @@ void term_list_matvec(edhip_op* op, int prec, int transpose, int accumulate, con
   OpDev d = transpose ? op->dev_col : op->dev_row;
   d.row_begin = row_begin;
   d.dim = row_end;
-  d.row_lanes = mv_row_lanes(sp->dim, d.n_lin + d.n_rest);
+  d.row_lanes = mv_row_lanes(sp->dim, d.n_lin, d.n_rest);
   if (ensure_diag(op)) {
     d.diag_re = op->diag_re.as<double>();
     d.diag_im = op->diag_im.as<double>();
