@@ -1479,7 +1479,8 @@ bool ensure_diag(edhip_op* op) {
         const size_t at[4] = {T.add(tab), T.add(sets), T.add(D.first), T.add(rest)};
         T.send(st);
         const DiagParity P{T.at<uint64_t>(at[0]), T.at<DiagSet>(at[1]), T.at<int32_t>(at[2]), T.at<DiagTerm>(at[3]),
-                           (int)D.first.size() - 1, mv_chunks(op->space->word_bits()), (int)rest.size()};
+                           (int)D.first.size() - 1, mv_chunks(op->space->word_bits()), (int)rest.size(),
+                           D.carried};
         HIP_OR_THROW(launch_diag_parity(P, d.rows, op->space->dim, op->diag_re.as<double>(), st));
         op->ctx->sync();
         return true;

@@ -247,6 +247,7 @@ struct DiagParity {
   const int32_t* first;  // n_seg + 1 offsets into sets
   const DiagTerm* rest;
   int n_seg, n_chunk, n_rest;
+  bool carried;
 };
 hipError_t launch_diag_parity(const DiagParity& P, const uint64_t* d_rows, int64_t dim, double* d_re, hipStream_t st);
 

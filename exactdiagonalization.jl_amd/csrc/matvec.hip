@@ -23,6 +23,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_values(OpDev op, double* __rest
 // aligned and another where not, so 64 pairs are tested by the XOR of a table
 // entry per 4 bits of the word (mv_match) and counted by coefficient.  4x7 J1-J2,
 // 1.4M rows and 448 terms: 15 us, 217 us term by term.
+template <bool CARRIED>
 __global__ __launch_bounds__(kBlock) void k_diag_parity(DiagParity P, const uint64_t* __restrict__ rows, int64_t dim,
                                                         double* __restrict__ re) {
   extern __shared__ unsigned char lds[];
@@ -30,7 +31,7 @@ __global__ __launch_bounds__(kBlock) void k_diag_parity(DiagParity P, const uint
   __syncthreads();
   const LdsPtr<uint64_t> tab = lds_at<uint64_t>(0);
   for (int64_t row = (int64_t)blockIdx.x * kBlock + threadIdx.x; row < dim; row += (int64_t)gridDim.x * kBlock) {
-    re[row] = diag_value(tab, P.sets, P.first, P.n_seg, P.n_chunk, P.rest, P.n_rest, rows[row]);
+    re[row] = diag_value<CARRIED>(tab, P.sets, P.first, P.n_seg, P.n_chunk, P.rest, P.n_rest, rows[row]);
   }
 }
 
@@ -1110,11 +1111,14 @@ hipError_t launch_diag_values(const OpDev& op, double* d_re, double* d_im, hipSt
 
 hipError_t launch_diag_parity(const DiagParity& P, const uint64_t* d_rows, int64_t dim, double* d_re, hipStream_t st) {
   if (dim == 0) return hipSuccess;
-  const hipError_t e = lds_from_zero<k_diag_parity>();
+  const hipError_t e = P.carried ? lds_from_zero<k_diag_parity<true>>() : lds_from_zero<k_diag_parity<false>>();
   if (e != hipSuccess) return e;
   const int64_t blocks = (dim + 4 * kBlock - 1) / (4 * kBlock);  // (4 rows a lane, for the staging)
-  hipLaunchKernelGGL(k_diag_parity, dim3((unsigned)blocks), dim3(kBlock), (uint32_t)(P.n_seg * P.n_chunk) * 128u, st, P,
-                     d_rows, dim, d_re);
+  const uint32_t lds = (uint32_t)(P.n_seg * P.n_chunk) * 128u;
+  if (P.carried)
+    hipLaunchKernelGGL(k_diag_parity<true>, dim3((unsigned)blocks), dim3(kBlock), lds, st, P, d_rows, dim, d_re);
+  else
+    hipLaunchKernelGGL(k_diag_parity<false>, dim3((unsigned)blocks), dim3(kBlock), lds, st, P, d_rows, dim, d_re);
   return hipGetLastError();
 }
 
