@@ -421,8 +421,8 @@ hipError_t launch_win_t(const WinOp& P, int unit, int transpose, const void* x, 
       win_entries_bytes(P.n_lin, P.n_chunk, P.n_rest) + (KIND == kWinPoint ? 8u * (uint32_t)(P.n_lin + P.n_rest + 1) : 0u);
   // the column form only conjugates the phase
   constexpr bool kT = VT<V>::cx;
-  if (unit) return launch_win_kernel<k_product_win<V, KIND, LX, LY, true, false>, V>(grid, WinLds<KIND, LX, LY, true>::entries + dyn, st, P, x, y);
-  constexpr uint32_t below = WinLds<KIND, LX, LY, false>::entries;
+  constexpr uint32_t below_unit = WinLds<KIND, LX, LY, true>::entries, below = WinLds<KIND, LX, LY, false>::entries;
+  if (unit) return launch_win_kernel<k_product_win<V, KIND, LX, LY, true, false>, V>(grid, below_unit + dyn, st, P, x, y);
   if (transpose) return launch_win_kernel<k_product_win<V, KIND, LX, LY, false, kT>, V>(grid, below + dyn, st, P, x, y);
   return launch_win_kernel<k_product_win<V, KIND, LX, LY, false, false>, V>(grid, below + dyn, st, P, x, y);
 }
